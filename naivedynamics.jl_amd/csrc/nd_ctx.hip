@@ -40,12 +40,14 @@ int nd_ctx_create(int32_t device, nd_ctx **out) {
         ND_HIP(hipSetDevice(device));
         ND_HIP(hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking));
         (void)nd::static_scratch(device);  // the device's scratch address, once per device
+        ND_HIP(hipHostMalloc(&ctx->host, nd::kHostResultBytes, hipHostMallocDefault));
         ND_HIP(hipEventCreate(&ctx->ev0));
         ND_HIP(hipEventCreate(&ctx->ev1));
         nd::clear_status(ctx);
         ND_HIP(hipStreamSynchronize(ctx->stream));
     } catch (const nd::Error &e) {
         int code = e.code;
+        if (ctx->host) (void)hipHostFree(ctx->host);
         delete ctx;
         return code;
     }
@@ -67,6 +69,7 @@ int nd_ctx_destroy(nd_ctx *ctx) {
                           &ctx->rank_keys,
                           &ctx->force_acc, &ctx->force_part, &ctx->async_ws};
     for (auto *b : bufs) b->release();
+    if (ctx->host) (void)hipHostFree(ctx->host);
     if (ctx->ev0) (void)hipEventDestroy(ctx->ev0);
     if (ctx->ev1) (void)hipEventDestroy(ctx->ev1);
     if (ctx->stream) (void)hipStreamDestroy(ctx->stream);

@@ -78,6 +78,7 @@ struct nd_ctx {
     nd::DevBuf stage_store;  // CAS slots etc. of the stage-level nd_bounding_volume_hierarchy
     nd::DevBuf rank_keys;    // nd_quantized_positions: keys and atom order (2N int32)
     nd::SortBufs sort;
+    void *host = nullptr;  // pinned block that kernels write results into (host_result)
     // last tree built by a one-call neighbour list (for nd_tree_export)
     int32_t tree_n = 0, tree_apl = 0;
     bool has_tree = false;
@@ -227,6 +228,14 @@ __device__ __forceinline__ int32_t cell_coord(const CellGrid &cg, float x, int d
 }
 
 void set_error(nd_ctx *ctx, const std::string &m);
+// The context's pinned result block as T: a call's last kernel stores what the
+// host has to know there, and the host reads it after its synchronisation
+// (a copy of a few bytes to pageable memory costs a staging copy on top).
+constexpr size_t kHostResultBytes = 4096;
+template <class T> T *host_result(nd_ctx *ctx) {
+    static_assert(sizeof(T) <= kHostResultBytes, "result block too small");
+    return static_cast<T *>(ctx->host);
+}
 int32_t read_status(nd_ctx *ctx);  // synchronises; returns and clears the status word
 void clear_status(nd_ctx *ctx);
 
