@@ -7,9 +7,9 @@
 // cells cx-1 .. cx+1 of one (cy, cz) row are one contiguous run of the sorted
 // copy.  Every unordered pair is found once from its earlier atom in cell
 // order through a half shell of five runs: the rest of its own cell plus cell
-// cx+1, the row (cy+1, cz), and the three rows (cy-1 .. cy+1, cz+1).  One lane
-// per sorted atom; a counting pass, an exclusive scan and an emitting pass
-// place each atom's pairs at a fixed offset, so the output order is
+// cx+1, the row (cy+1, cz), and the three rows (cy-1 .. cy+1, cz+1).  A counting
+// pass, an exclusive scan and an emitting pass (nd_pairs.hip) place each atom's
+// pairs at a fixed offset in the order of those runs, so the output order is
 // deterministic.  Distances use the reference's exact fold and both of its
 // predicates, so the pair set and every distance equal the brute-force
 // list's bit for bit.
@@ -105,61 +105,6 @@ k_cell_start(const int32_t *__restrict__ keys, int32_t n, int32_t ncell, int32_t
     cstart[k] = lo;
 }
 
-// Half-shell scan of sorted atom t (see the file comment); pairs are
-// (min, max) of the two original indices and the distance.
-template <bool EMIT>
-__global__ void __launch_bounds__(nd::kBlock)
-k_cell_pairs(const float4 *__restrict__ cpos, const int32_t *__restrict__ keys, int32_t n,
-             nd::CellGrid cg, const int32_t *__restrict__ cstart, float r, float r2, int32_t pred,
-             int64_t *__restrict__ counts, const int64_t *__restrict__ offsets,
-             nd_pair *__restrict__ out) {
-    const int32_t t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= n) return;
-    const int32_t key = keys[t];
-    int64_t c = 0;
-    nd_pair *o = nullptr;
-    int64_t limit = 0;
-    if (EMIT) {
-        o = out + offsets[t];
-        limit = offsets[t + 1] - offsets[t];
-    }
-    if (key < cg.ncell) {
-        const float4 p = cpos[t];
-        const int32_t oi = __float_as_int(p.w);
-        const int32_t g0 = cg.g[0], g1 = cg.g[1], g2 = cg.g[2];
-        const int32_t cx = key % g0, cyz = key / g0, cy = cyz % g1, cz = cyz / g1;
-        auto run = [&](int32_t b, int32_t e) {
-            for (int32_t u = b; u < e; ++u) {
-                const float4 q = cpos[u];
-                float d;
-                if (nd::accept(nd::sqdist(p.x, p.y, p.z, q.x, q.y, q.z), r, r2, pred, d)) {
-                    if (EMIT && c < limit) {
-                        const int32_t oj = __float_as_int(q.w);
-                        nd_pair pr;
-                        pr.i = oi < oj ? oi : oj;
-                        pr.j = oi < oj ? oj : oi;
-                        pr.d = d;
-                        o[c] = pr;
-                    }
-                    ++c;
-                }
-            }
-        };
-        const int32_t x0 = cx > 0 ? cx - 1 : 0, x1 = cx + 1 < g0 ? cx + 1 : g0 - 1;
-        run(t + 1, cstart[key + (cx + 1 < g0 ? 2 : 1)]);
-        if (cy + 1 < g1) {
-            const int32_t b = (cz * g1 + cy + 1) * g0;
-            run(cstart[b + x0], cstart[b + x1 + 1]);
-        }
-        if (cz + 1 < g2)
-            for (int32_t y = cy > 0 ? cy - 1 : 0; y <= cy + 1 && y < g1; ++y) {
-                const int32_t b = ((cz + 1) * g1 + y) * g0;
-                run(cstart[b + x0], cstart[b + x1 + 1]);
-            }
-    }
-    if (!EMIT) counts[t] = c;
-}
-
 }  // namespace
 
 namespace nd {
@@ -246,18 +191,23 @@ int nd_cell_neighborlist(nd_ctx *ctx, const float *d_xyz, int32_t n, float cutof
                                                 ctx->cell_vals.as<int32_t>(), cpos, cstart);
     ctx->counts.reserve(sizeof(int64_t) * ((size_t)n + 1));
     ctx->offsets.reserve(sizeof(int64_t) * ((size_t)n + 1));
-    const float r2 = cutoff * cutoff;
-    k_cell_pairs<false><<<nd::grid_for(n), nd::kBlock, 0, st>>>(
-        cpos, keys, n, cg, cstart, cutoff, r2, predicate, ctx->counts.as<int64_t>(), nullptr, nullptr);
-    ND_HIP(hipGetLastError());
+    nd::PairSearch S{};
+    S.kind = nd::kPairsHalf;
+    S.n = n;
+    S.apl = 1;
+    S.cg = cg;
+    S.cpos = cpos;
+    S.ckey = keys;
+    S.cstart = cstart;
+    S.r = cutoff;
+    S.thr = predicate == ND_PRED_SCALAR ? cutoff * cutoff : nd::root_threshold(cutoff);
+    nd::launch_pair_count(st, S, ctx->counts.as<int64_t>(), nullptr);
     const int64_t total = nd::scan_counts(ctx, n);
     *count = total;
     if (total > cap || (total > 0 && d_out == nullptr))
         throw nd::Error(ND_ERR_CAPACITY, "pair buffer too small; *count = required");
     if (total == 0) return ND_OK;
-    k_cell_pairs<true><<<nd::grid_for(n), nd::kBlock, 0, st>>>(
-        cpos, keys, n, cg, cstart, cutoff, r2, predicate, nullptr, ctx->offsets.as<int64_t>(), d_out);
-    ND_HIP(hipGetLastError());
+    nd::launch_pair_emit(st, S, ctx->offsets.as<int64_t>(), 0, d_out);
     ND_HIP(hipStreamSynchronize(st));
     ND_API_END(ctx)
 }

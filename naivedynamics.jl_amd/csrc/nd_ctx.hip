@@ -66,7 +66,7 @@ int nd_ctx_destroy(nd_ctx *ctx) {
                           &ctx->sort.keys_alt, &ctx->sort.vals_alt, &ctx->sort.hist,
                           &ctx->sort.flags, &ctx->cell_keys, &ctx->cell_vals, &ctx->cell_pos,
                           &ctx->cell_start, &ctx->trav_rec, &ctx->scan_tmp, &ctx->stage_store,
-                          &ctx->rank_keys,
+                          &ctx->rank_keys, &ctx->perm_alt, &ctx->prep,
                           &ctx->force_acc, &ctx->force_part, &ctx->async_ws};
     for (auto *b : bufs) b->release();
     if (ctx->host) (void)hipHostFree(ctx->host);

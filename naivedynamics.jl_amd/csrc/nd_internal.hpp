@@ -71,6 +71,7 @@ struct nd_ctx {
     nd::DevBuf codes, codes_sorted, perm, xyz_sorted, nodes, store, counts, offsets, xyz_in,
         pairs_out, bbox;
     nd::DevBuf cell_keys, cell_vals, cell_pos, cell_start;  // nd_cell_neighborlist
+    nd::DevBuf perm_alt, prep;  // one-call lists: second permutation buffer, small work words
     nd::DevBuf trav_rec;  // four-wide records of the one-call traversal
     nd::DevBuf scan_tmp;  // tile sums of scan_counts
     nd::DevBuf force_acc, force_part;  // pair-list forces: fixed-point sums, energy partials
@@ -103,6 +104,11 @@ void launch_bbox(hipStream_t st, const float *xyz, int32_t n, float *bbox6);
 void launch_fill_i32(hipStream_t s, int32_t *p, int64_t n, int32_t v);
 void launch_iota(hipStream_t s, int32_t *p, int32_t n);
 void radix_sort_pairs_auto(nd_ctx *ctx, int32_t *keys, int32_t *vals, int32_t n);
+// Stable sort by the bits of vary (the bits in which keys differ): passes
+// between (*keys, *vals) and (keys2, vals2); the sorted pairs' buffers are left
+// in *keys and *vals.
+void radix_sort_bits(hipStream_t s, SortBufs &b, uint32_t vary, int32_t n, int32_t **keys, int32_t **vals,
+                     int32_t *keys2, int32_t *vals2);
 void launch_gather_xyz(hipStream_t s, const float *xyz, const int32_t *perm, int32_t n,
                        float *out);
 
@@ -219,6 +225,39 @@ CellGrid make_cell_grid(const double lo[3], const double ext[3], double r, int64
 const int32_t *launch_cell_index(hipStream_t st, SortBufs &sb, const float *xyz, int32_t stride,
                                  int32_t n, const CellGrid &cg, int32_t *keys, int32_t *vals,
                                  float4 *cpos, int32_t *cstart);
+
+// nd_pairs.hip: pair searches over cells.  Kinds: the leaf-pair list, the two
+// point-query lists (own-leaf and root-started), the half-shell cell list.
+enum : int32_t { kPairsLeaf = 0, kPairsPointOwn = 1, kPairsPointRoot = 2, kPairsHalf = 3 };
+// The one-call lists over a tree (nd_traverse.hip's entry points): kind
+// kPairsLeaf / kPairsPointOwn / kPairsPointRoot; builds the tree that stays for
+// nd_tree_export and returns the required pair count (pairs are written if it
+// is <= cap).  Synchronous.
+int64_t tree_list(nd_ctx *ctx, const float *d_xyz, int32_t kind, int32_t n, int32_t apl, float r, int32_t pred,
+                  int32_t morton, nd_pair *d_out, int64_t cap);
+struct PairSearch {
+    int32_t kind, n, apl;
+    CellGrid cg;
+    const float4 *cpos;     // cell-sorted atoms, w = slot (half shell: input index)
+    const int32_t *ckey;    // their cells (ncell: in none)
+    const int32_t *cstart;  // ncell + 1
+    const float *xyz;       // positions by slot (lists over a tree)
+    const nd_node *nodes;   // leaf boxes (lists over a tree)
+    const int32_t *idx;     // input index of each slot (lists over a tree)
+    float r;                // the radius
+    float thr;              // accepted: s < thr
+    float certain;          // s below this implies the walk's box test
+};
+// Smallest float whose correctly rounded square root is >= r (r normal, positive).
+float root_threshold(float r);
+// Counts per slot (half shell: per cell-sorted place) and, by atomic maximum,
+// the largest (maxcnt may be null).
+void launch_pair_count(hipStream_t st, const PairSearch &S, int64_t *counts, int32_t *maxcnt);
+// Whether the emitting pass of a list over a tree can hold an atom's (a leaf's)
+// hits in LDS; the half shell's needs no such room.
+bool pair_emit_fits(int32_t kind, int32_t apl, int32_t maxcnt);
+// Pairs at the exclusive offsets of the counts.
+void launch_pair_emit(hipStream_t st, const PairSearch &S, const int64_t *offsets, int32_t maxcnt, nd_pair *out);
 
 __device__ __forceinline__ int32_t cell_coord(const CellGrid &cg, float x, int d) {
     const double t = ((double)x - cg.lo[d]) * cg.inv[d];
@@ -341,6 +380,22 @@ __device__ __forceinline__ uint32_t cell10(float x, float lo, float s) {
     if (!(t > 0.0f)) return 0u;  // also maps NaN to 0 (NaN input is flagged)
     if (t >= 1023.0f) return 1023u;
     return (uint32_t)floorf(t);
+}
+
+// mortoncodes!' key (BVHTraverse.jl:257-288); ok: inside its domain.
+__device__ __forceinline__ int32_t masked_key(float x, float y, float z, bool &ok) {
+    int32_t qx = 0, qy = 0, qz = 0;
+    ok = floor_i32(x / kBinwidth, qx);
+    ok &= floor_i32(y / kBinwidth, qy);
+    ok &= floor_i32(z / kBinwidth, qz);
+    return (qx & kMagic0) | (qy & kMagic1) | (qz & kMagic2);
+}
+
+// The interleaved key over box = (lo, scale); ok: finite.
+__device__ __forceinline__ int32_t interleaved_key(float x, float y, float z, const float *__restrict__ box, bool &ok) {
+    ok = __builtin_isfinite(x) && __builtin_isfinite(y) && __builtin_isfinite(z);
+    const uint32_t cx = cell10(x, box[0], box[3]), cy = cell10(y, box[1], box[4]), cz = cell10(z, box[2], box[5]);
+    return (int32_t)(spread10(cx) | (spread10(cy) << 1) | (spread10(cz) << 2));
 }
 
 }  // namespace nd

@@ -5,12 +5,6 @@
 namespace {
 
 using nd::cell10;
-using nd::floor_i32;
-using nd::kBinwidth;
-using nd::kMagic0;
-using nd::kMagic1;
-using nd::kMagic2;
-using nd::spread10;
 
 __global__ void __launch_bounds__(nd::kBlock)
 k_morton_masked(const float *__restrict__ xyz, int32_t n, int32_t *__restrict__ codes,
@@ -20,11 +14,8 @@ k_morton_masked(const float *__restrict__ xyz, int32_t n, int32_t *__restrict__ 
     const float x = xyz[3 * (int64_t)i + 0];
     const float y = xyz[3 * (int64_t)i + 1];
     const float z = xyz[3 * (int64_t)i + 2];
-    int32_t qx = 0, qy = 0, qz = 0;
-    bool ok = floor_i32(x / kBinwidth, qx);
-    ok &= floor_i32(y / kBinwidth, qy);
-    ok &= floor_i32(z / kBinwidth, qz);
-    codes[i] = (qx & kMagic0) | (qy & kMagic1) | (qz & kMagic2);
+    bool ok;
+    codes[i] = nd::masked_key(x, y, z, ok);
     if (idx) idx[i] = i;
     if (!ok) atomicOr(status, nd::kStatusDomain);
 }
@@ -39,11 +30,11 @@ k_morton_interleave(const float *__restrict__ xyz, int32_t n, const float *__res
     const float x = xyz[3 * (int64_t)i + 0];
     const float y = xyz[3 * (int64_t)i + 1];
     const float z = xyz[3 * (int64_t)i + 2];
-    bool ok = __builtin_isfinite(x) && __builtin_isfinite(y) && __builtin_isfinite(z);
-    const uint32_t cx = cell10(x, box[0], box[3]), cy = cell10(y, box[1], box[4]),
-                   cz = cell10(z, box[2], box[5]);
-    const uint32_t c = HILBERT ? nd::hilbert30(cx, cy, cz) : (spread10(cx) | (spread10(cy) << 1) | (spread10(cz) << 2));
-    codes[i] = (int32_t)c;
+    bool ok;
+    int32_t c = nd::interleaved_key(x, y, z, box, ok);
+    if (HILBERT)
+        c = (int32_t)nd::hilbert30(cell10(x, box[0], box[3]), cell10(y, box[1], box[4]), cell10(z, box[2], box[5]));
+    codes[i] = c;
     if (idx) idx[i] = i;
     if (!ok) atomicOr(status, nd::kStatusDomain);
 }

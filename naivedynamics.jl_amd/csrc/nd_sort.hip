@@ -266,23 +266,31 @@ size_t radix_scratch_blocks(int32_t n) { return (size_t)((n + kTile - 1) / kTile
 
 namespace {
 
+// One stable pass over the BITS-bit digit at shift (hist: R ntiles + R ints).
+template <int BITS>
+void radix_pass(hipStream_t s, int32_t *hist, const int32_t *ki, const int32_t *vi, int32_t n, int32_t shift,
+                int32_t *ko, int32_t *vo) {
+    constexpr int R = 1 << BITS;
+    const int32_t ntiles = (int32_t)radix_scratch_blocks(n);
+    int32_t *totals = hist + (size_t)R * (size_t)ntiles;
+    k_radix_hist<BITS><<<ntiles, kBlock, 0, s>>>(ki, n, shift, ntiles, hist);
+    k_radix_scan_rows<<<R, kBlock, 0, s>>>(hist, ntiles, totals);
+    k_radix_scatter<BITS><<<ntiles, kBlock, 0, s>>>(ki, vi, n, shift, ntiles, hist, totals, ko, vo);
+}
+
 // One LSD pass per BITS-bit digit from first_bit up to end_bit; returns the
 // number of passes (odd: the result is in the alternate buffers).
 template <int BITS>
 int radix_passes(hipStream_t s, SortBufs &b, int32_t *keys, int32_t *vals, int32_t n,
                  int32_t first_bit, int32_t end_bit) {
     constexpr int R = 1 << BITS;
-    const int32_t ntiles = (int32_t)radix_scratch_blocks(n);
     b.keys_alt.reserve(sizeof(int32_t) * (size_t)n);
     b.vals_alt.reserve(sizeof(int32_t) * (size_t)n);
-    b.hist.reserve(sizeof(int32_t) * ((size_t)R * (size_t)ntiles + R));
-    int32_t *hist = b.hist.as<int32_t>(), *totals = hist + (size_t)R * (size_t)ntiles;
+    b.hist.reserve(sizeof(int32_t) * ((size_t)R * radix_scratch_blocks(n) + R));
     int32_t *ki = keys, *vi = vals, *ko = b.keys_alt.as<int32_t>(), *vo = b.vals_alt.as<int32_t>();
     int passes = 0;
     for (int shift = first_bit; shift < end_bit; shift += BITS) {
-        k_radix_hist<BITS><<<ntiles, kBlock, 0, s>>>(ki, n, shift, ntiles, hist);
-        k_radix_scan_rows<<<R, kBlock, 0, s>>>(hist, ntiles, totals);
-        k_radix_scatter<BITS><<<ntiles, kBlock, 0, s>>>(ki, vi, n, shift, ntiles, hist, totals, ko, vo);
+        radix_pass<BITS>(s, b.hist.as<int32_t>(), ki, vi, n, shift, ko, vo);
         std::swap(ki, ko);
         std::swap(vi, vo);
         ++passes;
@@ -315,8 +323,28 @@ void radix_sort_keys10(hipStream_t s, SortBufs &b, int32_t *keys, int32_t *vals,
     }
 }
 
-// Sorts keys/vals in place over only the 8-bit digit windows whose bits vary
-// (synchronises once to read the varying-bit mask).
+// The varying bits lo .. hi take one 10-bit pass where they fit (22 against 2 x
+// 15 us at 262,144 keys: the masked key of the unit cube has 10), else 8-bit
+// passes from lo up, windows without a varying bit left out.
+void radix_sort_bits(hipStream_t s, SortBufs &b, uint32_t vary, int32_t n, int32_t **keys, int32_t **vals,
+                     int32_t *keys2, int32_t *vals2) {
+    if (n <= 1 || vary == 0u) return;
+    const int lo = __builtin_ctz(vary), span = 32 - __builtin_clz(vary) - lo;
+    const bool ten = span > 8 && span <= 10;
+    const size_t ntiles = radix_scratch_blocks(n), R = ten ? 1024 : 256;
+    b.hist.reserve(sizeof(int32_t) * (R * ntiles + R));
+    for (int shift = lo; shift < lo + span; shift += ten ? 10 : 8) {
+        if (!((vary >> shift) & (uint32_t)(R - 1))) continue;
+        if (ten) radix_pass<10>(s, b.hist.as<int32_t>(), *keys, *vals, n, shift, keys2, vals2);
+        else radix_pass<8>(s, b.hist.as<int32_t>(), *keys, *vals, n, shift, keys2, vals2);
+        std::swap(*keys, keys2);
+        std::swap(*vals, vals2);
+    }
+    ND_HIP(hipGetLastError());
+}
+
+// Sorts keys/vals in place over only the bits that vary (synchronises once to
+// read the varying-bit mask).
 void radix_sort_pairs_auto(nd_ctx *ctx, int32_t *keys, int32_t *vals, int32_t n) {
     if (n <= 1) return;
     ctx->sort.flags.reserve(64);
@@ -327,9 +355,15 @@ void radix_sort_pairs_auto(nd_ctx *ctx, int32_t *keys, int32_t *vals, int32_t n)
     uint32_t h[2];
     ND_HIP(hipMemcpyAsync(h, fl, sizeof(h), hipMemcpyDeviceToHost, ctx->stream));
     ND_HIP(hipStreamSynchronize(ctx->stream));
-    const uint32_t vary = h[0] ^ h[1];
-    for (int shift = 0; shift < 32; shift += 8)
-        if ((vary >> shift) & 0xFFu) radix_sort_pairs(ctx->stream, ctx->sort, keys, vals, n, shift, shift + 8);
+    SortBufs &b = ctx->sort;
+    b.keys_alt.reserve(sizeof(int32_t) * (size_t)n);
+    b.vals_alt.reserve(sizeof(int32_t) * (size_t)n);
+    int32_t *k = keys, *v = vals;
+    radix_sort_bits(ctx->stream, b, h[0] ^ h[1], n, &k, &v, b.keys_alt.as<int32_t>(), b.vals_alt.as<int32_t>());
+    if (k != keys) {
+        ND_HIP(hipMemcpyAsync(keys, k, sizeof(int32_t) * (size_t)n, hipMemcpyDeviceToDevice, ctx->stream));
+        ND_HIP(hipMemcpyAsync(vals, v, sizeof(int32_t) * (size_t)n, hipMemcpyDeviceToDevice, ctx->stream));
+    }
 }
 
 void launch_iota(hipStream_t s, int32_t *p, int32_t n) {

@@ -1007,38 +1007,8 @@ int nd_leafbuild_traverse_bvh(nd_ctx *ctx, const float *d_xyz, const nd_bvh_spec
     ND_REQUIRE(morton_mode == ND_MORTON_MASKED || morton_mode == ND_MORTON_INTERLEAVE,
                "unknown key mode");
     ND_HIP(hipSetDevice(ctx->device));
-    const int32_t n = chk.atom_count, apl = chk.atomsperleaf, nL = chk.leaves_count;
-    ctx->has_tree = false;
-    ctx->codes.reserve(sizeof(int32_t) * (size_t)n);
-    ctx->codes_sorted.reserve(sizeof(int32_t) * (size_t)n);
-    ctx->perm.reserve(sizeof(int32_t) * (size_t)n);
-    ctx->xyz_sorted.reserve(sizeof(float) * 3 * (size_t)n);
-    ctx->nodes.reserve(sizeof(nd_node) * (size_t)(2 * nL - 1));
-    ctx->store.reserve(sizeof(int32_t) * nd::lbvh_scratch_ints(nL));
-    // mortoncodes! -> codes (and perm = 1:N)
-    nd::launch_morton(ctx, d_xyz, n, morton_mode, nullptr, nullptr, ctx->codes_sorted.as<int32_t>(),
-                      ctx->perm.as<int32_t>(), ctx->status.as<int32_t>());
-    if (nd::read_status(ctx) & nd::kStatusDomain)
-        throw nd::Error(ND_ERR_DOMAIN,
-                        "mortoncodes!: coordinate outside the Int32 quantisation domain "
-                        "(reference throws InexactError)");
-    // sortperm + permute!
-    nd::radix_sort_pairs_auto(ctx, ctx->codes_sorted.as<int32_t>(), ctx->perm.as<int32_t>(), n);
-    nd::launch_gather_xyz(ctx->stream, d_xyz, ctx->perm.as<int32_t>(), n, ctx->xyz_sorted.as<float>());
-    // leafcluster_primitives + bounding_volume_hierarchy!
-    nd::launch_lbvh(ctx->stream, ctx->xyz_sorted.as<float>(), 3, ctx->codes_sorted.as<int32_t>(), nL,
-                    apl, chk.neighbor_distance, 1, ctx->nodes.as<nd_node>(), ctx->store.as<int32_t>(),
-                    ctx->status.as<int32_t>());
-    ctx->has_tree = true;
-    ctx->tree_n = n;
-    ctx->tree_apl = apl;
-    ctx->tree_nodes = ctx->nodes.as<nd_node>();
-    ctx->tree_perm = ctx->perm.as<int32_t>();
-    ctx->tree_codes = ctx->codes_sorted.as<int32_t>();
-    ctx->tree_store = ctx->store.as<int32_t>();
-    const int64_t total = nd::leaf_traverse(ctx, ctx->nodes.as<nd_node>(), ctx->xyz_sorted.as<float>(),
-                                            ctx->perm.as<int32_t>(), n, apl, chk.neighbor_distance,
-                                            predicate, d_out, cap, true);
+    const int64_t total = nd::tree_list(ctx, d_xyz, nd::kPairsLeaf, chk.atom_count, chk.atomsperleaf,
+                                        chk.neighbor_distance, predicate, morton_mode, d_out, cap);
     *count = total;
     if (total > cap) throw nd::Error(ND_ERR_CAPACITY, "pair buffer too small; *count = required");
     ND_API_END(ctx)
@@ -1171,38 +1141,9 @@ int nd_build_traverse_bvh(nd_ctx *ctx, const float *d_xyz, const nd_bvh_spec *sp
     // exact in Float32 below this bound, so the leaves get +- r exactly
     ND_REQUIRE(chk.neighbor_distance <= 0.5f * FLT_MAX, "nd_build_traverse_bvh: neighbor_distance too large");
     ND_HIP(hipSetDevice(ctx->device));
-    const int32_t n = chk.atom_count, apl = chk.atomsperleaf, nL = chk.leaves_count;
-    ctx->has_tree = false;
-    ctx->codes_sorted.reserve(sizeof(int32_t) * (size_t)n);
-    ctx->perm.reserve(sizeof(int32_t) * (size_t)n);
-    ctx->xyz_sorted.reserve(sizeof(float) * 3 * (size_t)n);
-    ctx->nodes.reserve(sizeof(nd_node) * (size_t)(2 * nL - 1));
-    ctx->store.reserve(sizeof(int32_t) * nd::lbvh_scratch_ints(nL));
-    // mortoncodes! + sortperm + permute! (BVHTraverse.jl:511-516)
-    nd::launch_morton(ctx, d_xyz, n, morton_mode, nullptr, nullptr, ctx->codes_sorted.as<int32_t>(),
-                      ctx->perm.as<int32_t>(), ctx->status.as<int32_t>());
-    if (nd::read_status(ctx) & nd::kStatusDomain)
-        throw nd::Error(ND_ERR_DOMAIN,
-                        "mortoncodes!: coordinate outside the Int32 quantisation domain "
-                        "(reference throws InexactError)");
-    nd::radix_sort_pairs_auto(ctx, ctx->codes_sorted.as<int32_t>(), ctx->perm.as<int32_t>(), n);
-    nd::launch_gather_xyz(ctx->stream, d_xyz, ctx->perm.as<int32_t>(), n, ctx->xyz_sorted.as<float>());
-    // cluster_primitives (+- r leaves) + bounding_volume_hierarchy!; TreeData
-    // overwrites the root box (BVHTraverse.jl:856-858), the root-started form's
-    // build kernel keeps it (NaiveKA.jl:301-302)
-    nd::launch_lbvh(ctx->stream, ctx->xyz_sorted.as<float>(), 3, ctx->codes_sorted.as<int32_t>(), nL, apl,
-                    2.0f * chk.neighbor_distance, query_mode == ND_QUERY_OWN_LEAF ? 1 : 0,
-                    ctx->nodes.as<nd_node>(), ctx->store.as<int32_t>(), ctx->status.as<int32_t>());
-    ctx->has_tree = true;
-    ctx->tree_n = n;
-    ctx->tree_apl = apl;
-    ctx->tree_nodes = ctx->nodes.as<nd_node>();
-    ctx->tree_perm = ctx->perm.as<int32_t>();
-    ctx->tree_codes = ctx->codes_sorted.as<int32_t>();
-    ctx->tree_store = ctx->store.as<int32_t>();
-    const int64_t total = nd::point_traverse(ctx, ctx->nodes.as<nd_node>(), ctx->xyz_sorted.as<float>(),
-                                             ctx->perm.as<int32_t>(), n, apl, chk.neighbor_distance, query_mode,
-                                             d_out, cap);
+    const int64_t total = nd::tree_list(
+        ctx, d_xyz, query_mode == ND_QUERY_ROOT ? nd::kPairsPointRoot : nd::kPairsPointOwn, chk.atom_count,
+        chk.atomsperleaf, chk.neighbor_distance, ND_PRED_SCALAR, morton_mode, d_out, cap);
     *count = total;
     if (total > cap) throw nd::Error(ND_ERR_CAPACITY, "pair buffer too small; *count = required");
     ND_API_END(ctx)
