@@ -235,6 +235,12 @@ enum : int32_t { kPairsLeaf = 0, kPairsPointOwn = 1, kPairsPointRoot = 2, kPairs
 // is <= cap).  Synchronous.
 int64_t tree_list(nd_ctx *ctx, const float *d_xyz, int32_t kind, int32_t n, int32_t apl, float r, int32_t pred,
                   int32_t morton, nd_pair *d_out, int64_t cap);
+// Bounding box of the atoms with finite coordinates; false if there are none.
+// Synchronous.
+bool atoms_box(nd_ctx *ctx, const float *d_xyz, int32_t n, double lo[3], double hi[3]);
+// Scans ctx->counts (n) into ctx->offsets; returns the total, and (where asked
+// for) the word at maxcnt and the context's status word.  Synchronous.
+int64_t pair_total(nd_ctx *ctx, int64_t n, const int32_t *maxcnt, int32_t *most, int32_t *status);
 struct PairSearch {
     int32_t kind, n, apl;
     CellGrid cg;

@@ -9,7 +9,7 @@
 // a leaf of four atoms that straddles an octree jump overlaps thousands of
 // leaves (1.7-1.9 ms per pass for 262,144 points at liquid density).
 //
-// One wave takes kQueries consecutive cell-sorted atoms, in groups that lie in
+// One wave takes 16 to 64 consecutive cell-sorted atoms, in groups that lie in
 // up to k cells of one row along x (k so that k cells hold about a dozen
 // atoms).  A group's candidates are the rows of cells around it, each row one
 // contiguous run of the cell-sorted atoms; they are loaded once into registers
@@ -48,6 +48,7 @@
 // themselves.
 #include <algorithm>
 #include <cmath>
+#include <cstring>
 
 #include "nd_internal.hpp"
 
@@ -55,11 +56,11 @@ namespace {
 
 using nd::wave_lds_sync;
 
-// candidates in registers, in batches of 64 (at liquid density 27 cells of the
-// list radius hold 475-520 atoms, a half shell's 14 some 270)
-__host__ __device__ constexpr int batches(int kind) { return kind == nd::kPairsHalf ? 6 : 10; }
-constexpr int kQueue = 512;   // hits a wave collects before it writes them
-constexpr int kQueries = 16;  // atoms per wave
+// Candidates in registers, in batches of 64: enough for a group at liquid
+// density (475-520 atoms in 27 cells of the list radius, some 270 in a half
+// shell's 14); more take another round.
+__host__ __device__ constexpr int batches(int kind, bool many) { return !many ? 3 : (kind == nd::kPairsHalf ? 6 : 10); }
+constexpr int kQueue = 512;  // hits a group may hold in LDS
 constexpr int kWaves = nd::kBlock / 64;
 
 struct PairArgs {
@@ -68,7 +69,7 @@ struct PairArgs {
     const int32_t *ckey;    // cell of each cell-sorted atom (ncell: none)
     const int32_t *cstart;  // ncell + 1
     nd::CellGrid cg;
-    int32_t k, n, apl;
+    int32_t k, per_wave, many, n, apl;
     float thr, certain, r;
     const nd_node *nodes;   // leaf boxes (lists over a tree)
     const int32_t *idx;     // input index of each slot (lists over a tree)
@@ -76,7 +77,7 @@ struct PairArgs {
     const int64_t *offsets;
     int32_t *maxcnt;
     nd_pair *out;
-    int32_t cap, most;      // hits a wave holds in LDS; most hits of an atom
+    int32_t cap;            // hits a wave holds in LDS
 };
 
 __device__ __forceinline__ float lane_f(float v, int l) {
@@ -100,26 +101,26 @@ __device__ bool box_test(const PairArgs &A, int32_t sq, float qx, float qy, floa
            (qz < c.max[2]);
 }
 
-template <int KIND, bool EMIT>
+template <int KIND, bool EMIT, bool MANY>
 __global__ void __launch_bounds__(nd::kBlock)
 k_cell_search(PairArgs A) {
     constexpr bool HALF = KIND == nd::kPairsHalf;
-    constexpr int ROWS = HALF ? 5 : 9, kBatches = batches(KIND);
-    // per wave: cap hits' places (later their slots), squared distances, queries
+    constexpr int ROWS = HALF ? 5 : 9, kBatches = batches(KIND, MANY);
+    // per wave: cap hits' places or slots, squared distances, queries
     extern __shared__ __align__(16) int32_t s_hits[];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     int32_t *hkey = s_hits + (size_t)w * 2 * A.cap;
     float *hs = reinterpret_cast<float *>(hkey + A.cap);
     uint8_t *hq = reinterpret_cast<uint8_t *>(s_hits + (size_t)kWaves * 2 * A.cap) + (size_t)w * A.cap;
-    const int32_t t0 = __builtin_amdgcn_readfirstlane(((int32_t)blockIdx.x * kWaves + w) * kQueries);
+    const int32_t t0 = __builtin_amdgcn_readfirstlane(((int32_t)blockIdx.x * kWaves + w) * A.per_wave);
     if (t0 >= A.n) return;
-    const int32_t nt = min(kQueries, A.n - t0);
+    const int32_t nt = min(A.per_wave, A.n - t0);
     const int32_t g0 = A.cg.g[0], g1 = A.cg.g[1], g2 = A.cg.g[2];
     // lane q holds atom t0 + q: cell, position, filter word, place of its count
     float px = 0.0f, py = 0.0f, pz = 0.0f;
-    int32_t pk = A.cg.ncell, pf = 0, pslot = 0, pid = 0, found = 0;
+    int32_t pk = A.cg.ncell, pf = 0, pslot = 0, pid = 0;
     int64_t off = 0;
-    int32_t lim = 0;
+    int32_t lim = 0;  // its hits (emitting)
     if (lane < nt) {
         const float4 p = A.cpos[t0 + lane];
         px = p.x;
@@ -135,14 +136,17 @@ k_cell_search(PairArgs A) {
             if (!HALF) pid = (KIND == nd::kPairsLeaf && A.apl > 1) ? pslot : A.idx[pslot];
         }
     }
+    int32_t found = 0;  // lane q: hits of query q so far
+    // lane q: the LDS room of query q's hits (emitting): consecutive, in whole
+    // fours where they are going to be ranked
+    int32_t room = HALF ? lim : (lim + 3) & ~3, end = room;
+    if (EMIT)
+        for (int o = 1; o < 64; o <<= 1) {
+            const int32_t v = __shfl_up(end, o, 64);
+            if (lane >= o) end += v;
+        }
     const int32_t prow = pk / g0;
-    // hits in LDS, query after query, and (lane q) where query q's begin
-    int32_t held = 0, qbase = 0;
-    // Writes the hits held, all queries' together so that every lane has one.
-    // Called by the whole wave: lanes past the end take part in the shuffles.
-    int64_t outrun = HALF && EMIT ? off : 0;  // half shell: consecutive atoms' pairs are one run
-    outrun = ((int64_t)lane_i((int32_t)(outrun >> 32), 0) << 32) | (uint32_t)lane_i((int32_t)outrun, 0);
-    // position of a hit (place or slot)
+    // position of a candidate (place or slot)
     auto atom = [&](int32_t h) -> float3 {
         if constexpr (HALF) {
             const float4 c = A.cpos[h];
@@ -152,93 +156,23 @@ k_cell_search(PairArgs A) {
             return make_float3(c[0], c[1], c[2]);
         }
     };
-    auto flush = [&]() {
-        constexpr int U = 4;  // gathers in flight per lane
-        wave_lds_sync();
-        for (int32_t e0 = 0; e0 < held; e0 += 64 * U) {
-            int32_t q[U], h[U], other[U];
-            float3 c[U];
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const int32_t e = e0 + 64 * u + lane;
-                q[u] = e < held ? (int32_t)hq[e] : 0xFF;
-                h[u] = q[u] != 0xFF ? hkey[e] : 0;
-            }
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                if constexpr (HALF) {
-                    const float4 v = A.cpos[h[u]];
-                    c[u] = make_float3(v.x, v.y, v.z);
-                    other[u] = __float_as_int(v.w);
-                } else {
-                    c[u] = atom(h[u]);
-                    other[u] = h[u];
-                }
-            }
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const int32_t e = e0 + 64 * u + lane, ql = q[u] & 63;
-                const float qx = __shfl(px, ql, 64), qy = __shfl(py, ql, 64), qz = __shfl(pz, ql, 64);
-                const int32_t qi = __shfl(pid, ql, 64);
-                const float s = nd::sqdist(qx, qy, qz, c[u].x, c[u].y, c[u].z);
-                if (q[u] != 0xFF) {
-                    if (HALF) {
-                        nd_pair p;
-                        p.i = min(qi, other[u]);
-                        p.j = max(qi, other[u]);
-                        p.d = sqrtf(s);
-                        A.out[outrun + e] = p;
-                    } else {
-                        hs[e] = s;
-                    }
-                } else if (!HALF && e < held) {
-                    hkey[e] = INT32_MAX;
-                }
-            }
-        }
-        if constexpr (!HALF) {
-            // each hit at the rank of its slot among its query's; the slots
-            // are read in fours (a query's part is filled up to a multiple)
-            wave_lds_sync();
-            for (int32_t e0 = 0; e0 < held; e0 += 64) {
-                const int32_t e = e0 + lane;
-                const int32_t q = e < held ? (int32_t)hq[e] : 0xFF;
-                const bool ok = q != 0xFF;
-                const int32_t b = __shfl(qbase, q & 63, 64), qi = __shfl(pid, q & 63, 64);
-                const int32_t m = __shfl(lim, q & 63, 64);
-                const int64_t o = ((int64_t)__shfl((int32_t)(off >> 32), q & 63, 64) << 32) |
-                                  (uint32_t)__shfl((int32_t)off, q & 63, 64);
-                if (!ok) continue;
-                const int32_t key = hkey[e];
-                int32_t r = 0;
-                for (int32_t t = b; t < b + m; t += 4) {
-                    const int4 v = *reinterpret_cast<const int4 *>(hkey + t);
-                    r += (v.x < key) + (v.y < key) + (v.z < key) + (v.w < key);
-                }
-                nd_pair p;
-                p.i = qi;
-                // leaves of several atoms: slots, until k_merge_leaf
-                p.j = (KIND == nd::kPairsLeaf && A.apl > 1) ? key : A.idx[key];
-                p.d = sqrtf(hs[e]);
-                if (r < m) A.out[o + r] = p;
-            }
-        }
-        wave_lds_sync();
-        outrun += held;
-        held = 0;
-    };
     int32_t q0 = 0;
     while (q0 < nt) {
-        // the group: atoms from q0 on in the next k cells of the same row
+        // the group: atoms from q0 on in the next k cells of the same row,
+        // and (emitting) as many as have room for their hits
         const int32_t k0 = lane_i(pk, q0), row = lane_i(prow, q0);
         if (k0 >= A.cg.ncell) break;  // atoms in no cell (a non-finite coordinate) pair with none
-        const uint64_t in = __builtin_amdgcn_ballot_w64(lane >= q0 && lane < nt && prow == row && pk < k0 + A.k);
+        const int32_t base = EMIT ? lane_i(end, q0) - lane_i(room, q0) : 0;  // LDS place 0 of the group
+        const uint64_t in = __builtin_amdgcn_ballot_w64(lane >= q0 && lane < nt && prow == row && pk < k0 + A.k &&
+                                                        (!EMIT || lane == q0 || end - base <= A.cap));
         const int32_t q1 = q0 + __builtin_popcountll(in);
+        const int32_t held = EMIT ? lane_i(end, q1 - 1) - base : 0;  // LDS places of the group
+        // more hits than LDS holds (half shell, one atom): straight to memory
+        const bool direct = EMIT && held > A.cap;
         const int32_t c0 = k0 - row * g0, c1 = lane_i(pk, q1 - 1) - row * g0;
         const int32_t cy = row % g1, cz = row / g1;
         // candidate rows: lane j holds row j's run; the runs are read as one
-        // sequence, with pre[j] candidates before row j; a sequence position
-        // past pre[j] is step[j] further into the sorted atoms
+        // sequence
         int32_t start = 0, len = 0;
         if (lane < ROWS) {
             int32_t dy, dz;
@@ -256,38 +190,46 @@ k_cell_search(PairArgs A) {
                 len = A.cstart[b + min(c1 + 1, g0 - 1) + 1] - start;
             }
         }
-        int32_t pre[ROWS], step[ROWS], total = 0, before = 0;
+        // lane j: candidates before row j, and its start less those
+        int32_t pre = len;
 #pragma unroll
-        for (int j = 0; j < ROWS; ++j) {
-            const int32_t d = lane_i(start, j) - total;
-            pre[j] = total;
-            step[j] = d - before;
-            before = d;
-            total += lane_i(len, j);
+        for (int o = 1; o < 16; o <<= 1) {
+            const int32_t v = __shfl_up(pre, o, 64);
+            if (lane >= o) pre += v;
         }
+        const int32_t total = lane_i(pre, ROWS - 1);
+        pre -= len;
+        const int32_t rise = start - pre;
         const int mid = (q0 + q1) >> 1;
         const float ox = lane_f(px, mid), oy = lane_f(py, mid), oz = lane_f(pz, mid);
-        // candidate place of sequence position ci
-        auto place = [&](int32_t ci) -> int32_t {
-            int32_t u = ci + step[0];
-#pragma unroll
-            for (int j = 1; j < ROWS; ++j) u += ci >= pre[j] ? step[j] : 0;
-            return u;
-        };
-        float bx[kBatches], by[kBatches], bz[kBatches], bw[kBatches];
-        // order word of the filter: the place (every row of the half shell
-        // but the own one lies after the group), the slot or the input index;
-        // and what a hit leaves in LDS: the place or the slot
-        int32_t bf[kBatches], bslot[kBatches];
-        // the candidates s0 + 64 b + lane; past the end: a copy that the filter drops
-        auto load = [&](int32_t s0) {
+        // lane q's limits: below lo a candidate is a pair, from hi on it is none
+        const float ax = px - ox, ay = py - oy, az = pz - oz;
+        const float a2 = __builtin_fmaf(az, az, __builtin_fmaf(ay, ay, ax * ax));
+        const float reach = 2.0f * sqrtf(a2) + A.r;
+        const bool bound = A.r >= 1e-15f && A.r <= 1e12f && reach < 1e5f * A.r;
+        const float E = bound ? 1.2e-6f * (reach * reach + A.r * A.r) : INFINITY;
+        const float lo = (A.certain - a2) - E, hi = (A.thr - a2) + E;
+        int32_t row_at = 0;  // row of the next batch's first candidate, or one before it
+        for (int32_t s0 = 0; s0 < total; s0 += 64 * kBatches) {
+            // candidates s0 + 64 b + lane (past the end: a copy that the
+            // filter drops), the order word of the filter -- the place (every
+            // row of the half shell but the own one lies after the group),
+            // the slot or the input index -- and the place or slot
+            float bx[kBatches], by[kBatches], bz[kBatches], bw[kBatches];
+            int32_t bf[kBatches], bslot[kBatches];
 #pragma unroll
             for (int b = 0; b < kBatches; ++b) {
-                if (s0 + 64 * b >= total) break;
                 const int32_t ci = s0 + 64 * b + lane;
                 const bool ok = ci < total;
-                const int32_t u = ok ? place(ci) : t0;
-                const float4 c = A.cpos[u];
+                // the rows that begin before the batch's last candidate
+                int32_t u = ci + lane_i(rise, row_at);
+                while (row_at + 1 < ROWS) {
+                    const int32_t p = lane_i(pre, row_at + 1);
+                    if (p > s0 + 64 * b + 63) break;
+                    ++row_at;
+                    u = ci >= p ? ci + lane_i(rise, row_at) : u;
+                }
+                const float4 c = A.cpos[ok ? u : t0];
                 const float x = c.x - ox, y = c.y - oy, z = c.z - oz;
                 bx[b] = -2.0f * x;
                 by[b] = -2.0f * y;
@@ -297,80 +239,147 @@ k_cell_search(PairArgs A) {
                 bf[b] = KIND == nd::kPairsPointRoot ? A.idx[bslot[b]] : bslot[b];
                 if (!ok) bf[b] = INT32_MIN;
             }
-        };
-        const bool once = total <= 64 * kBatches;
-        if (once) load(0);
-        // lane q's limits: below lo a candidate is a pair, from hi on it is none
-        const float ax = px - ox, ay = py - oy, az = pz - oz;
-        const float a2 = __builtin_fmaf(az, az, __builtin_fmaf(ay, ay, ax * ax));
-        const float reach = 2.0f * sqrtf(a2) + A.r;
-        const bool bound = A.r >= 1e-15f && A.r <= 1e12f && reach < 1e5f * A.r;
-        const float E = bound ? 1.2e-6f * (reach * reach + A.r * A.r) : INFINITY;
-        const float lo = (A.certain - a2) - E, hi = (A.thr - a2) + E;
-        for (int32_t q = q0; q < q1; ++q) {
-            const float sx = lane_f(ax, q), sy = lane_f(ay, q), sz = lane_f(az, q);
-            const float slo = lane_f(lo, q), shi = lane_f(hi, q);
-            const float qx = lane_f(px, q), qy = lane_f(py, q), qz = lane_f(pz, q);
-            const int32_t qf = lane_i(pf, q), qslot = lane_i(pslot, q);
-            int32_t H = 0;  // hits so far
-            if (EMIT && !HALF) {
-                // room for this query's hits (at most maxcnt, from the counting pass)
-                if (held + A.most > A.cap) flush();
-                qbase = lane == q ? held : qbase;
-            }
-            for (int32_t s0 = 0; s0 < total; s0 += 64 * kBatches) {
-                if (!once) load(s0);
+            for (int32_t q = q0; q < q1; ++q) {
+                const float sx = lane_f(ax, q), sy = lane_f(ay, q), sz = lane_f(az, q);
+                const float slo = lane_f(lo, q), shi = lane_f(hi, q);
+                const int32_t qf = lane_i(pf, q);
+                // the next hit's LDS place (or, direct, its number)
+                int32_t H = lane_i(found, q);
+                const int32_t H0 = H, shift = EMIT && !direct ? lane_i(end, q) - lane_i(room, q) - base : 0;
 #pragma unroll
                 for (int b = 0; b < kBatches; ++b) {
-                    if (s0 + 64 * b >= total) break;
+                    if (s0 + 64 * b >= total) continue;
                     const float t = __builtin_fmaf(bx[b], sx, __builtin_fmaf(by[b], sy, __builtin_fmaf(bz[b], sz, bw[b])));
                     const uint64_t after = __builtin_amdgcn_ballot_w64(bf[b] > qf);
                     uint64_t m = __builtin_amdgcn_ballot_w64(t < slo) & after;
                     const uint64_t open = __builtin_amdgcn_ballot_w64(!(t >= shi)) & after & ~m;
                     if (open) {
-                        bool hit = (m >> lane) & 1u;
-                        if ((open >> lane) & 1u) {
-                            const float3 c = atom(bslot[b]);
+                        const float qx = lane_f(px, q), qy = lane_f(py, q), qz = lane_f(pz, q);
+                        const int32_t qslot = lane_i(pslot, q);
+                        bool in = false;
+                        if (__builtin_amdgcn_inverse_ballot_w64(open)) {
+                            // opaque to the compiler, which would hoist this
+                            // rare branch's addresses and divisions out of
+                            // the loop and keep them in registers
+                            int32_t sl = bslot[b];
+                            asm volatile("" : "+v"(sl));
+                            const float3 c = atom(sl);
                             const float s = nd::sqdist(qx, qy, qz, c.x, c.y, c.z);
-                            hit = s < A.thr;
+                            in = s < A.thr;
                             if (!HALF) {
-                                if (hit && !(s < A.certain)) hit = box_test<KIND>(A, qslot, qx, qy, qz, bslot[b]);
+                                if (in && !(s < A.certain)) in = box_test<KIND>(A, qslot, qx, qy, qz, sl);
                             }
                         }
-                        m = __builtin_amdgcn_ballot_w64(hit);
+                        m |= __builtin_amdgcn_ballot_w64(in);
                     }
                     if (EMIT) {
-                        if ((m >> lane) & 1u) {
-                            const int32_t at = held + H + (int32_t)__builtin_amdgcn_mbcnt_hi(
-                                                   (uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
-                            if (at < A.cap) {
-                                hkey[at] = bslot[b];
-                                hq[at] = (uint8_t)q;
+                        if (__builtin_amdgcn_inverse_ballot_w64(m)) {
+                            const int32_t at = (int32_t)__builtin_amdgcn_mbcnt_hi(
+                                (uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, (uint32_t)(shift + H)));
+                            if (!HALF || !direct) {
+                                if (at < A.cap) {
+                                    hkey[at] = bslot[b];
+                                    hq[at] = (uint8_t)q;
+                                }
+                            } else if (at < held) {
+                                int32_t sl = bslot[b];
+                                asm volatile("" : "+v"(sl));
+                                const float4 c = A.cpos[sl];
+                                const int32_t id = __float_as_int(c.w), qi = lane_i(pid, q0);
+                                const int64_t o = ((int64_t)lane_i((int32_t)(off >> 32), q0) << 32) |
+                                                  (uint32_t)lane_i((int32_t)off, q0);
+                                nd_pair p;
+                                p.i = min(qi, id);
+                                p.j = max(qi, id);
+                                p.d = sqrtf(nd::sqdist(lane_f(px, q0), lane_f(py, q0), lane_f(pz, q0), c.x, c.y, c.z));
+                                A.out[o + at] = p;
                             }
                         }
                     }
                     H += __builtin_popcountll(m);
-                    if (EMIT && HALF && held + H > A.cap - 64) {
-                        held += H;
-                        H = 0;
-                        flush();
+                }
+                if (H != H0) found = lane == q ? H : found;
+            }
+        }
+        if (EMIT && !direct && held > 0) {
+            if (!HALF && lane >= q0 && lane < q1)
+                for (int32_t e = lim; e < room; ++e) hq[end - room - base + e] = 0xFF;  // fill of the last four
+            wave_lds_sync();
+            const int64_t orun = ((int64_t)lane_i((int32_t)(off >> 32), q0) << 32) | (uint32_t)lane_i((int32_t)off, q0);
+            constexpr int U = 4;  // gathers in flight per lane
+            for (int32_t e0 = 0; e0 < held; e0 += 64 * U) {
+                int32_t q[U], h[U];
+                float3 c[U];
+                int32_t other[U];
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    const int32_t e = e0 + 64 * u + lane;
+                    q[u] = e < held ? (int32_t)hq[e] : 0xFF;
+                    h[u] = q[u] != 0xFF ? hkey[e] : 0;
+                }
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    if constexpr (HALF) {
+                        const float4 v = A.cpos[h[u]];
+                        c[u] = make_float3(v.x, v.y, v.z);
+                        other[u] = __float_as_int(v.w);
+                    } else {
+                        c[u] = atom(h[u]);
+                        other[u] = h[u];
+                    }
+                }
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    // all lanes take part in the shuffles
+                    const int32_t e = e0 + 64 * u + lane, ql = q[u] & 63;
+                    const float s = nd::sqdist(__shfl(px, ql, 64), __shfl(py, ql, 64), __shfl(pz, ql, 64), c[u].x,
+                                               c[u].y, c[u].z);
+                    if constexpr (HALF) {
+                        // consecutive atoms' pairs are one run of the output
+                        const int32_t qi = __shfl(pid, ql, 64);
+                        if (q[u] != 0xFF) {
+                            nd_pair p;
+                            p.i = min(qi, other[u]);
+                            p.j = max(qi, other[u]);
+                            p.d = sqrtf(s);
+                            A.out[orun + e] = p;
+                        }
+                    } else {
+                        if (q[u] != 0xFF) hs[e] = s;
+                        else if (e < held) hkey[e] = INT32_MAX;
                     }
                 }
             }
-            if (!EMIT) {
-                found = lane == q ? H : found;
-            } else {
-                held = min(held + H, A.cap);
-                if (!HALF) {
-                    const int32_t fill = -held & 3;
-                    if (lane < fill) hq[held + lane] = 0xFF;
-                    held += fill;
+            if constexpr (!HALF) {
+                // each hit at the rank of its slot among its query's
+                wave_lds_sync();
+                const int32_t qbase = end - room - base;
+                for (int32_t e0 = 0; e0 < held; e0 += 64) {
+                    const int32_t e = e0 + lane;
+                    const int32_t q = e < held ? (int32_t)hq[e] : 0xFF;
+                    const int32_t b = __shfl(qbase, q & 63, 64), qi = __shfl(pid, q & 63, 64);
+                    const int32_t m = __shfl(lim, q & 63, 64);
+                    const int64_t o = ((int64_t)__shfl((int32_t)(off >> 32), q & 63, 64) << 32) |
+                                      (uint32_t)__shfl((int32_t)off, q & 63, 64);
+                    if (q == 0xFF) continue;
+                    const int32_t key = hkey[e];
+                    int32_t r = 0;
+                    for (int32_t t = b; t < b + m; t += 4) {
+                        const int4 v = *reinterpret_cast<const int4 *>(hkey + t);
+                        r += (v.x < key) + (v.y < key) + (v.z < key) + (v.w < key);
+                    }
+                    nd_pair p;
+                    p.i = qi;
+                    // leaves of several atoms: slots, until k_merge_leaf
+                    p.j = (KIND == nd::kPairsLeaf && A.apl > 1) ? key : A.idx[key];
+                    p.d = sqrtf(hs[e]);
+                    if (r < m) A.out[o + r] = p;
                 }
             }
+            wave_lds_sync();
         }
         q0 = q1;
     }
-    if (EMIT && held > 0) flush();
     if (!EMIT) {
         if (lane < nt) A.counts[pslot] = found;
         if (A.maxcnt) {
@@ -466,9 +475,11 @@ __device__ __forceinline__ int32_t f2ord(float f) {
 }
 __device__ __forceinline__ float ord2f(int32_t i) { return __int_as_float(i >= 0 ? i : i ^ 0x7FFFFFFF); }
 
-// Per-workgroup bounding boxes of the finite coordinates (no atomics: 64
-// workgroups' on six words took 21 us, the launch that joins these 256 takes
-// 4); also clears the cell counts and the status word.
+// Per-workgroup bounding boxes of the finite coordinates (ATOMS: of the atoms
+// whose three coordinates are finite).  No atomics: 64 workgroups' on six words
+// took 21-29 us, these and the launch that joins them take 6 + 4.  Also clears
+// the cell counts and two words.
+template <bool ATOMS>
 __global__ void __launch_bounds__(nd::kBlock)
 k_prep_boxes(const float *__restrict__ xyz, int32_t n, int32_t *__restrict__ part, int32_t *__restrict__ cells,
              int32_t ncells, int32_t *__restrict__ status, int32_t *__restrict__ maxcnt) {
@@ -480,14 +491,16 @@ k_prep_boxes(const float *__restrict__ xyz, int32_t n, int32_t *__restrict__ par
         *maxcnt = 0;
     }
     int32_t mn[3] = {INT32_MAX, INT32_MAX, INT32_MAX}, mx[3] = {INT32_MIN, INT32_MIN, INT32_MIN};
-    for (int32_t i = t; i < n; i += stride)
+    for (int32_t i = t; i < n; i += stride) {
+        const float v[3] = {xyz[3 * (int64_t)i], xyz[3 * (int64_t)i + 1], xyz[3 * (int64_t)i + 2]};
+        const bool all = __builtin_isfinite(v[0]) & __builtin_isfinite(v[1]) & __builtin_isfinite(v[2]);
 #pragma unroll
         for (int d = 0; d < 3; ++d) {
-            const float v = xyz[3 * (int64_t)i + d];
-            if (!__builtin_isfinite(v)) continue;
-            mn[d] = min(mn[d], f2ord(v));
-            mx[d] = max(mx[d], f2ord(v));
+            if (!(ATOMS ? all : __builtin_isfinite(v[d]))) continue;
+            mn[d] = min(mn[d], f2ord(v[d]));
+            mx[d] = max(mx[d], f2ord(v[d]));
         }
+    }
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
         mn[d] = wave_min(mn[d]);
@@ -505,6 +518,18 @@ k_prep_boxes(const float *__restrict__ xyz, int32_t n, int32_t *__restrict__ par
         int32_t v = s[0][threadIdx.x];
         for (int k = 1; k < kWaves; ++k) v = threadIdx.x < 3 ? min(v, s[k][threadIdx.x]) : max(v, s[k][threadIdx.x]);
         part[6 * blockIdx.x + threadIdx.x] = v;
+    }
+}
+
+// The joined box, for the host (thread d < 6: word d).
+__global__ void __launch_bounds__(64)
+k_box_result(const int32_t *__restrict__ part, int32_t nparts, int32_t *__restrict__ host) {
+    for (int d = 0; d < 6; ++d) {
+        int32_t v = d < 3 ? INT32_MAX : INT32_MIN;
+        for (int32_t t = threadIdx.x; t < nparts; t += 64)
+            v = d < 3 ? min(v, part[6 * t + d]) : max(v, part[6 * t + d]);
+        v = d < 3 ? wave_min(v) : wave_max(v);
+        if (threadIdx.x == 0) host[d] = v;
     }
 }
 
@@ -596,7 +621,23 @@ k_prep_keys(const float *__restrict__ xyz, int32_t n, const float *__restrict__ 
         const nd::CellGrid &cg = prep->cg;
         const int32_t c = (nd::cell_coord(cg, z, 2) * cg.g[1] + nd::cell_coord(cg, y, 1)) * cg.g[0] +
                           nd::cell_coord(cg, x, 0);
-        cell_of[i] = make_int2(c, atomicAdd(&cells[c], 1));
+        // a wave's atoms of one cell are counted together while the cells are
+        // crowded (131,072 atoms of eight cells took 1 ms of atomics on their
+        // words); the first cell that few lanes share ends that
+        const int lane = threadIdx.x & 63;
+        int32_t place = -1;
+        while (place < 0) {
+            const uint64_t same = __builtin_amdgcn_ballot_w64(c == __builtin_amdgcn_readfirstlane(c));
+            if (__builtin_popcountll(same) < 4) break;
+            if ((same >> lane) & 1ull) {
+                const int first = __builtin_ctzll(same);
+                int32_t b = 0;
+                if (lane == first) b = atomicAdd(&cells[c], __builtin_popcountll(same));
+                place = __builtin_amdgcn_readlane(b, first) + __builtin_popcountll(same & ((1ull << lane) - 1ull));
+            }
+        }
+        if (place < 0) place = atomicAdd(&cells[c], 1);
+        cell_of[i] = make_int2(c, place);
         const uint32_t k = (uint32_t)code ^ 0x80000000u;
         atomicOr(&so, k);
         atomicAnd(&sa, k);
@@ -744,7 +785,7 @@ __global__ void k_count_result(const int64_t *__restrict__ total, const int32_t 
                                const int32_t *__restrict__ status, CountResult *__restrict__ host) {
     if (threadIdx.x == 0) {
         host->total = *total;
-        host->most = *most;
+        host->most = most ? *most : 0;
         host->status = *status;
     }
 }
@@ -763,7 +804,7 @@ float root_threshold(float r) {
 
 namespace {
 
-// Cells per group: about a dozen atoms.  At liquid density a cell of the list
+// Cells per group: about two dozen atoms.  At liquid density a cell of the list
 // radius holds 18, and groups of one cell test the fewest candidates; where
 // cells hold one or two (65,536 points, 8 neighbours each), groups of one cell
 // would spend their time on the row lookups.
@@ -774,9 +815,13 @@ PairArgs pair_args(const PairSearch &S) {
     A.cstart = S.cstart;
     A.cg = S.cg;
     const double mean = (double)S.n / S.cg.ncell;
+    // longer runs share more of a group's set-up, shorter ones leave enough
+    // waves (8,000 atoms at radius 2.8: cell list 153 us with 16, 186 with 32)
+    A.per_wave = S.n >= 262144 ? 32 : 16;
     // where squared distances underflow, atoms more than a cell apart could
     // pass the test: groups of one cell look at its 27 neighbours only
-    A.k = S.thr < 1e-30f ? 1 : (int32_t)std::min(16.0, std::max(1.0, std::floor(12.0 / mean)));
+    A.k = S.thr < 1e-30f ? 1 : (int32_t)std::min(64.0, std::max(1.0, std::floor(24.0 / mean)));
+    A.many = (S.kind == kPairsHalf ? 4.5 : 9.0) * (A.k + 2) * mean > 160.0;
     A.n = S.n;
     A.apl = S.apl;
     A.thr = S.thr;
@@ -788,12 +833,22 @@ PairArgs pair_args(const PairSearch &S) {
     return A;
 }
 
-unsigned search_grid(int32_t n) { return (unsigned)(((int64_t)n + kQueries * kWaves - 1) / (kQueries * kWaves)); }
+unsigned search_grid(const PairArgs &A) {
+    const int64_t per = (int64_t)A.per_wave * kWaves;
+    return (unsigned)((A.n + per - 1) / per);
+}
+
+template <int KIND>
+void count_kind(hipStream_t st, const PairArgs &A) {
+    if (A.many) k_cell_search<KIND, false, true><<<search_grid(A), kBlock, 0, st>>>(A);
+    else k_cell_search<KIND, false, false><<<search_grid(A), kBlock, 0, st>>>(A);
+}
 
 template <int KIND>
 void emit_kind(hipStream_t st, const PairArgs &A) {
     const size_t lds = 9 * (size_t)A.cap * kWaves;
-    k_cell_search<KIND, true><<<search_grid(A.n), kBlock, lds, st>>>(A);
+    if (A.many) k_cell_search<KIND, true, true><<<search_grid(A), kBlock, lds, st>>>(A);
+    else k_cell_search<KIND, true, false><<<search_grid(A), kBlock, lds, st>>>(A);
 }
 
 }  // namespace
@@ -802,12 +857,11 @@ void launch_pair_count(hipStream_t st, const PairSearch &S, int64_t *counts, int
     PairArgs A = pair_args(S);
     A.counts = counts;
     A.maxcnt = maxcnt;
-    const unsigned g = search_grid(S.n);
     switch (S.kind) {
-        case kPairsLeaf: k_cell_search<kPairsLeaf, false><<<g, kBlock, 0, st>>>(A); break;
-        case kPairsPointOwn: k_cell_search<kPairsPointOwn, false><<<g, kBlock, 0, st>>>(A); break;
-        case kPairsPointRoot: k_cell_search<kPairsPointRoot, false><<<g, kBlock, 0, st>>>(A); break;
-        default: k_cell_search<kPairsHalf, false><<<g, kBlock, 0, st>>>(A); break;
+        case kPairsLeaf: count_kind<kPairsLeaf>(st, A); break;
+        case kPairsPointOwn: count_kind<kPairsPointOwn>(st, A); break;
+        case kPairsPointRoot: count_kind<kPairsPointRoot>(st, A); break;
+        default: count_kind<kPairsHalf>(st, A); break;
     }
     ND_HIP(hipGetLastError());
 }
@@ -828,7 +882,6 @@ void launch_pair_emit(hipStream_t st, const PairSearch &S, const int64_t *offset
     PairArgs A = pair_args(S);
     A.offsets = offsets;
     A.out = out;
-    A.most = (maxcnt + 3) & ~3;
     A.cap = S.kind == kPairsHalf ? kQueue : hits_cap(maxcnt);
     switch (S.kind) {
         case kPairsLeaf: emit_kind<kPairsLeaf>(st, A); break;
@@ -846,6 +899,41 @@ void launch_pair_emit(hipStream_t st, const PairSearch &S, const int64_t *offset
             k_merge_leaf<kBlock><<<(unsigned)nL, kBlock, one, st>>>(offsets, S.idx, nL, S.apl, cap, out);
     }
     ND_HIP(hipGetLastError());
+}
+
+bool atoms_box(nd_ctx *ctx, const float *d_xyz, int32_t n, double lo[3], double hi[3]) {
+    hipStream_t st = ctx->stream;
+    ctx->prep.reserve(sizeof(int32_t) * 6 * kBoxBlocks);
+    int32_t *part = ctx->prep.as<int32_t>(), *status = ctx->status.as<int32_t>();
+    struct Box { int32_t v[6]; };
+    int32_t *hb = host_result<Box>(ctx)->v;
+    const unsigned nb = std::min<unsigned>(grid_for(n), kBoxBlocks);
+    k_prep_boxes<true><<<nb, kBlock, 0, st>>>(d_xyz, n, part, nullptr, 0, status + 9, status + 10);
+    k_box_result<<<1, 64, 0, st>>>(part, (int32_t)nb, hb);
+    ND_HIP(hipGetLastError());
+    ND_HIP(hipStreamSynchronize(st));
+    for (int d = 0; d < 3; ++d) {
+        if (hb[d] > hb[3 + d]) return false;
+        for (int e = 0; e < 2; ++e) {
+            const int32_t o = hb[3 * e + d], b = o >= 0 ? o : o ^ 0x7FFFFFFF;
+            float f;
+            std::memcpy(&f, &b, sizeof f);
+            (e ? hi : lo)[d] = (double)f;
+        }
+    }
+    return true;
+}
+
+int64_t pair_total(nd_ctx *ctx, int64_t n, const int32_t *maxcnt, int32_t *most, int32_t *status) {
+    CountResult *hc = host_result<CountResult>(ctx);
+    int32_t *word = ctx->status.as<int32_t>();
+    launch_scan(ctx, n);
+    k_count_result<<<1, 64, 0, ctx->stream>>>(ctx->offsets.as<int64_t>() + n, maxcnt, word, hc);
+    ND_HIP(hipGetLastError());
+    ND_HIP(hipStreamSynchronize(ctx->stream));
+    if (most) *most = hc->most;
+    if (status) *status = hc->status;
+    return hc->total;
 }
 
 // The one-call lists over a tree: keys, sort, tree, pairs.  Counting and
@@ -892,7 +980,7 @@ int64_t tree_list(nd_ctx *ctx, const float *d_xyz, int32_t kind, int32_t n, int3
     const float thr = pred == ND_PRED_SCALAR ? r * r : root_threshold(r);
     const unsigned nb = std::min<unsigned>(g, kBoxBlocks);
     Prep *hp = host_result<Prep>(ctx);
-    k_prep_boxes<<<nb, kBlock, 0, st>>>(d_xyz, n, part, cells, max_cells + 1, status, maxcnt);
+    k_prep_boxes<false><<<nb, kBlock, 0, st>>>(d_xyz, n, part, cells, max_cells + 1, status, maxcnt);
     k_prep_grid<<<1, kBlock, 0, st>>>(part, (int32_t)nb, r, thr, max_cells, box, prep);
     if (morton == ND_MORTON_MASKED)
         k_prep_keys<true><<<g, kBlock, 0, st>>>(d_xyz, n, box, prep, codes, perm, cells, cell_of, kb, status);
@@ -934,11 +1022,13 @@ int64_t tree_list(nd_ctx *ctx, const float *d_xyz, int32_t kind, int32_t n, int3
                                      d_out, cap);
     };
     // Cells serve radii whose squares are normal numbers, and atoms that are
-    // not crowded into few of the cells (one far outlier stretches the grid
-    // until all others share a cell): a test costs ~1/64 of what a walk's
-    // does, and a walk makes several hundred per atom at liquid density, so
-    // the line lies at 4,096 candidates per atom (27 sum_sq bounds them all).
-    const bool by_cells = r >= 1e-15f && r <= 1e18f && (double)p.sum_sq * 27.0 <= 4096.0 * n && apl <= 64;
+    // not crowded into few of the cells (27 sum_sq bounds the candidates: one
+    // far outlier stretches the grid until all others share a cell).  The line
+    // lies where a walk draws level: 131,072 points at density 0.8, 4 per leaf,
+    // radius 6 (4,800 candidates and 318 pairs an atom): 3.63 ms by cells, 3.99
+    // walking, point queries 3.04 and 4.80; 65,536 points, radius 8 (14,200):
+    // 4.14 and 3.78, point queries 10.3 and 7.3.
+    const bool by_cells = r >= 1e-15f && r <= 1e18f && (double)p.sum_sq * 27.0 <= 5500.0 * n && apl <= 64;
     if (!by_cells) return walk();
     PairSearch S{};
     S.kind = kind;
@@ -958,12 +1048,8 @@ int64_t tree_list(nd_ctx *ctx, const float *d_xyz, int32_t kind, int32_t n, int3
     ctx->offsets.reserve(sizeof(int64_t) * ((size_t)n + 1));
     const int64_t *off = ctx->offsets.as<int64_t>();
     launch_pair_count(st, S, ctx->counts.as<int64_t>(), maxcnt);
-    launch_scan(ctx, n);
-    CountResult *hc = host_result<CountResult>(ctx);
-    k_count_result<<<1, 64, 0, st>>>(off + n, maxcnt, status, hc);
-    ND_HIP(hipGetLastError());
-    ND_HIP(hipStreamSynchronize(st));
-    const CountResult c = *hc;
+    CountResult c{};
+    c.total = pair_total(ctx, n, maxcnt, &c.most, &c.status);
     if (c.status) clear_status(ctx);
     if (c.status & kStatusTree)
         throw Error(ND_ERR_STATE, "neighbour list: malformed tree (rope cycle or bad index)");
