@@ -17,17 +17,29 @@
 // x_k (from v_{k+1} = v_h + c F(x_{k+1}) of step k-1 and v_h = v_k + c F(x_k)
 // of step k) merge into one Hessian-vector product per step.  Per pair,
 //   M_ij = s I + (s'(r)/r) r_ij r_ij^T,  (J a)_i = sum_j M_ij (a_i - a_j).
-// The forward pass keeps (x, v) every checkpoint_every steps; the sweep
-// recomputes each segment forward from its checkpoint, storing its positions,
-// then walks it backwards.  Pair lists (radius max(cutoffs, rdf range) +
-// skin) come from the library's LBVH pair-list path and are rebuilt at the
-// same steps (multiples of rebuild_every) in the forward and the recompute.
+// The forward pass keeps (x, v) every checkpoint_every steps, and of its last
+// segment every position, list and order; the sweep walks that segment
+// backwards at once and recomputes the earlier ones forward from their
+// checkpoints first.  Pair lists (radius max(cutoffs, rdf range) + skin) are
+// rebuilt at the same steps (multiples of rebuild_every) in the forward and
+// the recompute.
 //
-// Kernels run one lane per atom over the atom's row of the pair list (every
-// j paired with i; rows are rebuilt with the list), so nothing is added with
-// atomics.  Forces are summed in 2^-40 fixed point: the sum does not depend
-// on the order within a row, which the list build leaves unspecified, so the
-// recompute reproduces the forward trajectory bit for bit in both
+// Atoms are kept in the order of the last list build, which is the order of
+// the cells (side >= list radius) it searches: a neighbour gather then reads
+// aligned records (position, and in FP64 the charge) that lie near each other,
+// and the build needs no tree.  kRowLanes lanes share an atom's row of the list:
+// at N = 32,768 one lane per atom leaves two waves per CU, and a row is a chain
+// of dependent loads.  One launch makes a step: the pair sums of x_k, the half
+// kick that ends step k - 1 and the half kick and drift of step k; in the
+// reverse sweep the Hessian-vector product and the next step's lambda_h and a.
+// Per step of the forward pass (FP64, 32,768 atoms) the launches of a force
+// (21.8 us), kick (4.1) and kick-drift (3.0) kernel with four lanes per row
+// became one; per list build a key, sort, tree and walk of 21 launches and a
+// host synchronisation became seven launches and none.
+//
+// Forces are summed in 2^-40 fixed point: the sum does not depend on the
+// order within a row or of the atoms, which the build leaves unspecified, so
+// the recompute reproduces the forward trajectory bit for bit in both
 // precisions.  The reverse sweep sums in FP64.
 //
 // No reference counterpart: NaiveDynamics.jl has no gradients.  This is the
@@ -46,6 +58,7 @@ constexpr double kInvFix = 1.0 / 1099511627776.0;
 struct AdjP {
     int32_t n, nbins;
     double eps, sigma, rc, rc2, kc, rcc, rcc2, dt, c;
+    double sig2, inv_eps, inv_sigma, inv_rcc2;
     double flj_rc;   // F_LJ(rc)
     double glj_rc;   // dF_LJ/dsigma at rc
     double rmax, h, dr;
@@ -62,19 +75,31 @@ __host__ __device__ inline double lj_G(double r, double eps, double sigma) {
     return 24.0 * eps * (24.0 * sr6 * sr6 - 6.0 * sr6) / (r * sigma);
 }
 
-// s(r) of the forward force in precision T (LJ + Coulomb, both shifted).
+// s(r) of the forward force in precision T (LJ + Coulomb, both shifted).  FP64
+// takes one division and one square root per pair; FP32 keeps a division for
+// each quotient (its trajectories are held to their last bit).
 template <class T>
 __device__ __forceinline__ T pair_s(T r2, T qq, const AdjP &P) {
     T s = (T)0;
-    const T r = sqrt(r2), ir = (T)1 / r;
-    if (r2 < (T)P.rc2) {
-        const T sr2 = (T)(P.sigma * P.sigma) / r2, sr6 = sr2 * sr2 * sr2;
-        const T F = (T)(24.0 * P.eps) * (sr6 * sr6 + sr6 * sr6 - sr6) * ir;
-        s += (F - (T)P.flj_rc) * ir;
-    }
-    if (r2 < (T)P.rcc2) {
-        const T F = (T)P.kc * qq * ((T)1 / r2 - (T)(1.0 / P.rcc2));
-        s += F * ir;
+    if constexpr (sizeof(T) == 8) {
+        const T ir2 = 1.0 / r2, ir = sqrt(ir2);
+        if (r2 < P.rc2) {
+            const T sr2 = P.sig2 * ir2, sr6 = sr2 * sr2 * sr2;
+            const T F = (24.0 * P.eps) * (sr6 * sr6 + sr6 * sr6 - sr6) * ir;
+            s += (F - P.flj_rc) * ir;
+        }
+        if (r2 < P.rcc2) s += P.kc * qq * (ir2 - P.inv_rcc2) * ir;
+    } else {
+        const T r = sqrt(r2), ir = (T)1 / r;
+        if (r2 < (T)P.rc2) {
+            const T sr2 = (T)(P.sigma * P.sigma) / r2, sr6 = sr2 * sr2 * sr2;
+            const T F = (T)(24.0 * P.eps) * (sr6 * sr6 + sr6 * sr6 - sr6) * ir;
+            s += (F - (T)P.flj_rc) * ir;
+        }
+        if (r2 < (T)P.rcc2) {
+            const T F = (T)P.kc * qq * ((T)1 / r2 - (T)(1.0 / P.rcc2));
+            s += F * ir;
+        }
     }
     return s;
 }
@@ -86,21 +111,21 @@ struct PairD {
 };
 __device__ __forceinline__ PairD pair_d(double r2, double qi, double qj, const AdjP &P) {
     PairD o{0.0, 0.0, 0.0, 0.0, 0.0};
-    const double r = sqrt(r2), ir = 1.0 / r, ir3 = ir * ir * ir;
+    const double ir2 = 1.0 / r2, ir = sqrt(ir2), r = r2 * ir, ir3 = ir * ir2;
     if (r2 < P.rc2) {
-        const double sr2 = P.sigma * P.sigma / r2, sr6 = sr2 * sr2 * sr2, sr12 = sr6 * sr6;
+        const double sr2 = P.sig2 * ir2, sr6 = sr2 * sr2 * sr2, sr12 = sr6 * sr6;
         const double F = 24.0 * P.eps * (2.0 * sr12 - sr6) * ir;
-        const double Fp = 24.0 * P.eps * (-26.0 * sr12 + 7.0 * sr6) * ir * ir;
+        const double Fp = 24.0 * P.eps * (-26.0 * sr12 + 7.0 * sr6) * ir2;
         const double s = (F - P.flj_rc) * ir;
         o.s += s;
         o.ds += (Fp * r - (F - P.flj_rc)) * ir3;
-        o.s_eps = s / P.eps;
-        const double G = 24.0 * P.eps * (24.0 * sr12 - 6.0 * sr6) * ir / P.sigma;
+        o.s_eps = s * P.inv_eps;
+        const double G = 24.0 * P.eps * (24.0 * sr12 - 6.0 * sr6) * ir * P.inv_sigma;
         o.s_sig = (G - P.glj_rc) * ir;
     }
     if (r2 < P.rcc2) {
         const double qq = qi * qj;
-        const double Hf = ir * ir - 1.0 / P.rcc2;  // F_c = kc qq Hf
+        const double Hf = ir2 - P.inv_rcc2;  // F_c = kc qq Hf
         const double F = P.kc * qq * Hf;
         const double Fp = -2.0 * P.kc * qq * ir3;
         o.s += F * ir;
@@ -110,70 +135,174 @@ __device__ __forceinline__ PairD pair_d(double r2, double qi, double qj, const A
     return o;
 }
 
-// Sorted FP32 positions (w = 0) for the list walk.
-__global__ void __launch_bounds__(nd::kBlock)
-k_adj_pos4(const float *__restrict__ xf, const int32_t *__restrict__ perm, int32_t n,
-           float4 *__restrict__ out) {
-    const int32_t s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= n) return;
-    const int64_t o = 3 * (int64_t)perm[s];
-    out[s] = make_float4(xf[o], xf[o + 1], xf[o + 2], 0.0f);
-}
+// Position records: (x, y, z) and, in FP64, the charge (FP32 keeps the charges
+// apart in FP64, as their product is taken).
+template <class T> struct V4;
+template <> struct V4<float> { using R = float4; };
+template <> struct V4<double> { using R = double4; };
 
-// Neighbour rows in the list walk's layout: sorted slot s (atom perm[s])
-// keeps its entries in column s & 63 of the block of its 64 slots (stride
-// 64), as original atom ids once k_adj_map_ids has run; lcnt[s] entries.
+// Rows of the pair list: atom s (in the order of its build) keeps cap entries
+// from lists[s cap], cnt[s] of them used, all of the same order.
 struct Rows {
-    const int32_t *lists, *lcnt, *perm;
+    const int32_t *lists, *cnt;
     int32_t cap;
-    __device__ __forceinline__ const int32_t *col(int32_t s) const {
-        return lists + ((int64_t)(s >> 6) * cap) * 64 + (s & 63);
-    }
-    __device__ __forceinline__ int32_t count(int32_t s) const { return lcnt[s] < cap ? lcnt[s] : cap; }
+    __device__ __forceinline__ const int32_t *row(int32_t s) const { return lists + (int64_t)s * cap; }
+    __device__ __forceinline__ int32_t count(int32_t s) const { return cnt[s] < cap ? cnt[s] : cap; }
 };
 
-// The walk writes sorted indices; the adjoint's kernels want original ids.
-// One lane per slot and list row (blockIdx.y = row): no per-lane loop.
-__global__ void __launch_bounds__(nd::kBlock)
-k_adj_map_ids(const int32_t *__restrict__ perm, int32_t n, int32_t cap, int32_t *__restrict__ lists,
-              const int32_t *__restrict__ lcnt) {
-    const int32_t s = blockIdx.x * blockDim.x + threadIdx.x;
-    const int32_t k = blockIdx.y;
-    if (s >= n || k >= (lcnt[s] < cap ? lcnt[s] : cap)) return;
-    int32_t *e = lists + ((int64_t)(s >> 6) * cap + k) * 64 + (s & 63);
-    *e = perm[*e];
-}
+// Lanes per row: lane t of an atom takes entries t, t + kRowLanes, ...
+constexpr int kRowLanes = 16;
 
-// Rows are split over kRowLanes consecutive lanes of a wave (lane s of an
-// atom takes entries s, s + kRowLanes, ...): at N = 32,768 one lane per atom
-// leaves 2 waves per CU and every row a long chain of dependent loads.
-constexpr int kRowLanes = 4;
-
-// F_i = sum_j s(r_ij) r_ij over row i, summed in 2^-40 fixed point: the sum
-// is the same whatever the order of the row (and however it is split).
+// x, v of the caller's order and precision as records, and the FP32 positions
+// the list build bins.
 template <class T>
 __global__ void __launch_bounds__(nd::kBlock)
-k_adj_force(Rows R, const T *__restrict__ x, const double *__restrict__ q, AdjP P,
-            unsigned long long *__restrict__ F) {
-    const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    const int32_t sl = (int32_t)(t / kRowLanes), sub = (int32_t)(t % kRowLanes);
-    const int32_t i = sl < P.n ? R.perm[sl] : 0;
-    long long fx = 0, fy = 0, fz = 0;
-    if (sl < P.n) {
-    const int32_t *col = R.col(sl);
-    const int32_t c = R.count(sl);
-    const T xi = x[3 * (int64_t)i], yi = x[3 * (int64_t)i + 1], zi = x[3 * (int64_t)i + 2];
-    const double qi = q[i];
-    for (int32_t k = sub; k < c; k += kRowLanes) {
-        const int32_t j = col[(int64_t)k * 64];
-        const T dx = xi - x[3 * (int64_t)j], dy = yi - x[3 * (int64_t)j + 1], dz = zi - x[3 * (int64_t)j + 2];
-        const T r2 = dx * dx + dy * dy + dz * dz;
-        if (!(r2 < (T)P.rc2 || r2 < (T)P.rcc2)) continue;
-        const T s = pair_s<T>(r2, (T)(qi * q[j]), P);
-        fx += llrint((double)(s * dx) * kFix);
-        fy += llrint((double)(s * dy) * kFix);
-        fz += llrint((double)(s * dz) * kFix);
+k_adj_init(const double *__restrict__ x, const double *__restrict__ v, const double *__restrict__ q, int32_t n,
+           typename V4<T>::R *__restrict__ xo, typename V4<T>::R *__restrict__ vo, float4 *__restrict__ x32,
+           int32_t *__restrict__ orig) {
+    const int32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    typename V4<T>::R a, b;
+    a.x = (T)x[3 * (int64_t)i]; a.y = (T)x[3 * (int64_t)i + 1]; a.z = (T)x[3 * (int64_t)i + 2];
+    a.w = sizeof(T) == 8 ? (T)q[i] : (T)0;
+    b.x = (T)v[3 * (int64_t)i]; b.y = (T)v[3 * (int64_t)i + 1]; b.z = (T)v[3 * (int64_t)i + 2];
+    b.w = 0;
+    xo[i] = a;
+    vo[i] = b;
+    x32[i] = make_float4((float)a.x, (float)a.y, (float)a.z, 0.0f);
+    orig[i] = i;
+}
+
+template <class R>
+__global__ void __launch_bounds__(nd::kBlock)
+k_adj_to_f32(const R *__restrict__ x, int32_t n, float4 *__restrict__ out) {
+    const int32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) out[i] = make_float4((float)x[i].x, (float)x[i].y, (float)x[i].z, 0.0f);
+}
+
+// Atom i goes to its place in the cells: the cell-sorted FP32 copy with its
+// number in the state's order, and (xo != null) the state into that order.
+template <class R>
+__global__ void __launch_bounds__(nd::kBlock)
+k_adj_place(const float4 *__restrict__ x32, const int2 *__restrict__ cell_of, const int32_t *__restrict__ cells,
+            int32_t n, float4 *__restrict__ cpos, int32_t *__restrict__ ckey, const R *__restrict__ x,
+            const R *__restrict__ v, const int32_t *__restrict__ orig, const double *__restrict__ q,
+            R *__restrict__ xo, R *__restrict__ vo, int32_t *__restrict__ origo, double *__restrict__ qs) {
+    const int32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    const int2 c = cell_of[i];
+    const int32_t u = cells[c.x] + c.y;
+    const float4 p = x32[i];
+    cpos[u] = make_float4(p.x, p.y, p.z, __int_as_float(xo ? u : i));
+    ckey[u] = c.x;
+    if (!xo) return;
+    xo[u] = x[i];
+    vo[u] = v[i];
+    const int32_t o = orig[i];
+    origo[u] = o;
+    qs[u] = q[o];
+}
+
+// Rows of the list: the pairs of cell-sorted atoms closer than the list radius,
+// each in both rows.  A wave takes kListAtoms consecutive atoms in groups of
+// one cell row (k cells of about two dozen atoms): a batch of 64 candidates
+// from the nine rows of cells around the group is tested against its atoms one
+// after another, and a ballot places the hits.
+constexpr int kListAtoms = 8;
+
+__global__ void __launch_bounds__(nd::kBlock)
+k_adj_rows(const float4 *__restrict__ cpos, const int32_t *__restrict__ ckey, const int32_t *__restrict__ cells,
+           const nd::CellGrid *__restrict__ grid, int32_t n, float rl2, int32_t cap, int32_t *__restrict__ lists,
+           int32_t *__restrict__ cnt, int32_t *__restrict__ most) {
+    const int lane = threadIdx.x & 63;
+    const int32_t t0 = __builtin_amdgcn_readfirstlane((int32_t)((blockIdx.x * blockDim.x + threadIdx.x) >> 6) * kListAtoms);
+    if (t0 >= n) return;
+    const int32_t nt = min(kListAtoms, n - t0);
+    const int32_t g0 = grid->g[0], g1 = grid->g[1], g2 = grid->g[2];
+    const int32_t k = max(1, (int32_t)(24.0f * (float)grid->ncell / (float)n));
+    float px = 0.0f, py = 0.0f, pz = 0.0f;
+    int32_t pk = -1, pid = 0, found = 0;
+    if (lane < nt) {
+        const float4 p = cpos[t0 + lane];
+        px = p.x;
+        py = p.y;
+        pz = p.z;
+        pid = __float_as_int(p.w);
+        pk = ckey[t0 + lane];
     }
+    const int32_t prow = pk / g0;
+    auto lf = [](float v, int l) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l)); };
+    int32_t q0 = 0;
+    while (q0 < nt) {
+        const int32_t k0 = __builtin_amdgcn_readlane(pk, q0), row = __builtin_amdgcn_readlane(prow, q0);
+        const uint64_t in = __builtin_amdgcn_ballot_w64(lane >= q0 && lane < nt && prow == row && pk < k0 + k);
+        const int32_t q1 = q0 + __builtin_popcountll(in);
+        const int32_t c0 = k0 - row * g0, c1 = __builtin_amdgcn_readlane(pk, q1 - 1) - row * g0;
+        const int32_t cy = row % g1, cz = row / g1;
+        for (int32_t z = max(cz - 1, 0); z <= min(cz + 1, g2 - 1); ++z)
+            for (int32_t y = max(cy - 1, 0); y <= min(cy + 1, g1 - 1); ++y) {
+                const int32_t b = (z * g1 + y) * g0;
+                const int32_t u1 = cells[b + min(c1 + 1, g0 - 1) + 1];
+                for (int32_t u0 = cells[b + max(c0 - 1, 0)]; u0 < u1; u0 += 64) {
+                    const int32_t u = u0 + lane;
+                    const float4 c = cpos[min(u, u1 - 1)];
+                    for (int32_t q = q0; q < q1; ++q) {
+                        const float dx = c.x - lf(px, q), dy = c.y - lf(py, q), dz = c.z - lf(pz, q);
+                        const bool hit = (dx * dx + dy * dy + dz * dz < rl2) & (u < u1) & (u != t0 + q);
+                        const uint64_t m = __builtin_amdgcn_ballot_w64(hit);
+                        const int32_t have = __builtin_amdgcn_readlane(found, q);
+                        if (hit) {
+                            const int32_t at = (int32_t)__builtin_amdgcn_mbcnt_hi(
+                                (uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, (uint32_t)have));
+                            if (at < cap)
+                                lists[(int64_t)__builtin_amdgcn_readlane(pid, q) * cap + at] = __float_as_int(c.w);
+                        }
+                        found = lane == q ? have + __builtin_popcountll(m) : found;
+                    }
+                }
+            }
+        q0 = q1;
+    }
+    if (lane < nt) cnt[pid] = found;
+    int32_t mx = found;
+    for (int o = 32; o > 0; o >>= 1) mx = max(mx, __shfl_xor(mx, o, 64));
+    if (lane == 0 && mx > __hip_atomic_load(most, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(most, mx);
+}
+
+__device__ __forceinline__ double fix_val(unsigned long long v) { return (double)(long long)v * kInvFix; }
+
+// One launch of the forward model at x_k: F_i = sum_j s(r_ij) r_ij over row i,
+// summed in 2^-40 fixed point (the same whatever the order of the row and
+// however it is split); FINISH: the half kick that ends step k - 1; vck: the
+// velocity at k kept; DRIFT: the half kick and drift that begin step k.
+template <class T, bool FINISH, bool DRIFT>
+__global__ void __launch_bounds__(nd::kBlock)
+k_adj_step(Rows R, const typename V4<T>::R *__restrict__ x, const double *__restrict__ qs, AdjP P,
+           typename V4<T>::R *__restrict__ v, typename V4<T>::R *__restrict__ vck,
+           typename V4<T>::R *__restrict__ xo, float4 *__restrict__ x32) {
+    using V = typename V4<T>::R;
+    const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+    const int32_t s = (int32_t)(t / kRowLanes), sub = (int32_t)(t % kRowLanes);
+    long long fx = 0, fy = 0, fz = 0;
+    V xi{};
+    if (s < P.n) {
+        const int32_t *row = R.row(s);
+        const int32_t c = R.count(s);
+        xi = x[s];
+        const double qi = sizeof(T) == 8 ? (double)xi.w : qs[s];
+        int32_t j = sub < c ? row[sub] : 0;
+        for (int32_t k = sub; k < c; k += kRowLanes) {
+            const V xj = x[j];
+            const double qj = sizeof(T) == 8 ? (double)xj.w : qs[j];
+            j = k + kRowLanes < c ? row[k + kRowLanes] : 0;
+            const T dx = xi.x - xj.x, dy = xi.y - xj.y, dz = xi.z - xj.z;
+            const T r2 = dx * dx + dy * dy + dz * dz;
+            if (!(r2 < (T)P.rc2 || r2 < (T)P.rcc2)) continue;
+            const T f = pair_s<T>(r2, (T)(qi * qj), P);
+            fx += llrint((double)(f * dx) * kFix);
+            fy += llrint((double)(f * dy) * kFix);
+            fz += llrint((double)(f * dz) * kFix);
+        }
     }
     // exact integer sums over the atom's lanes (all lanes take part)
 #pragma unroll
@@ -182,41 +311,27 @@ k_adj_force(Rows R, const T *__restrict__ x, const double *__restrict__ q, AdjP 
         fy += __shfl_xor(fy, off, 64);
         fz += __shfl_xor(fz, off, 64);
     }
-    if (sl < P.n && sub == 0) {
-        F[3 * (int64_t)i] = (unsigned long long)fx;
-        F[3 * (int64_t)i + 1] = (unsigned long long)fy;
-        F[3 * (int64_t)i + 2] = (unsigned long long)fz;
+    if (s >= P.n || sub != 0) return;
+    const T f[3] = {(T)fix_val((unsigned long long)fx), (T)fix_val((unsigned long long)fy),
+                    (T)fix_val((unsigned long long)fz)};
+    V w = v[s];
+    if (FINISH) {
+        w.x = w.x + (T)P.c * f[0];
+        w.y = w.y + (T)P.c * f[1];
+        w.z = w.z + (T)P.c * f[2];
     }
-}
-
-__device__ __forceinline__ double fix_val(unsigned long long v) { return (double)(long long)v * kInvFix; }
-
-// v += c F; x += dt v
-template <class T>
-__global__ void __launch_bounds__(nd::kBlock)
-k_adj_kick_drift(T *__restrict__ x, T *__restrict__ v, const unsigned long long *__restrict__ F,
-                 AdjP P) {
-    const int64_t k = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (k >= 3 * (int64_t)P.n) return;
-    T vv = v[k] + (T)P.c * (T)fix_val(F[k]);
-    v[k] = vv;
-    x[k] = x[k] + (T)P.dt * vv;
-}
-
-// v += c F
-template <class T>
-__global__ void __launch_bounds__(nd::kBlock)
-k_adj_kick(T *__restrict__ v, const unsigned long long *__restrict__ F, AdjP P) {
-    const int64_t k = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (k >= 3 * (int64_t)P.n) return;
-    v[k] = v[k] + (T)P.c * (T)fix_val(F[k]);
-}
-
-template <class T>
-__global__ void __launch_bounds__(nd::kBlock)
-k_adj_to_f32(const T *__restrict__ x, int64_t m, float *__restrict__ out) {
-    const int64_t k = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (k < m) out[k] = (float)x[k];
+    if (vck) vck[s] = w;
+    if (DRIFT) {
+        w.x = w.x + (T)P.c * f[0];
+        w.y = w.y + (T)P.c * f[1];
+        w.z = w.z + (T)P.c * f[2];
+        xi.x = xi.x + (T)P.dt * w.x;
+        xi.y = xi.y + (T)P.dt * w.y;
+        xi.z = xi.z + (T)P.dt * w.z;
+        xo[s] = xi;
+        if (x32) x32[s] = make_float4((float)xi.x, (float)xi.y, (float)xi.z, 0.0f);
+    }
+    v[s] = w;
 }
 
 // RDF kernel weight of pair distance r for bin b
@@ -229,28 +344,29 @@ __device__ __forceinline__ double rdf_dK(double d, double h) {
     return fabs(u) < 1.0 ? -6.0 * u * t * t / h : 0.0;
 }
 
-// raw histogram sum_{i<j} K(r_ij - r_b) (normalisation on the host); bins
-// are summed per workgroup in LDS, then added once per workgroup
+// raw histogram sum_{i<j} K(r_ij - r_b) (normalisation on the host); bins are
+// summed per workgroup in LDS, the workgroups' in index order by k_rdf_sum
 constexpr int kMaxBins = 1024;
+constexpr int kHistBlocks = 512;
 
 template <class T>
 __global__ void __launch_bounds__(nd::kBlock)
-k_rdf_hist(Rows R, const T *__restrict__ x, AdjP P, double *__restrict__ hist) {
+k_rdf_hist(Rows R, const typename V4<T>::R *__restrict__ x, AdjP P, double *__restrict__ part) {
     __shared__ double hb[kMaxBins];
     for (int b = threadIdx.x; b < P.nbins; b += blockDim.x) hb[b] = 0.0;
     __syncthreads();
-    const int32_t sl = blockIdx.x * blockDim.x + threadIdx.x;
-    if (sl < P.n) {
-        const int32_t i = R.perm[sl];
-        const double xi = (double)x[3 * (int64_t)i], yi = (double)x[3 * (int64_t)i + 1],
-                     zi = (double)x[3 * (int64_t)i + 2];
-        const int32_t *col = R.col(sl);
-        const int32_t c = R.count(sl);
-        for (int32_t k = 0; k < c; ++k) {
-            const int32_t j = col[(int64_t)k * 64];
-            if (j < i) continue;  // each unordered pair once
-            const double dx = xi - (double)x[3 * (int64_t)j], dy = yi - (double)x[3 * (int64_t)j + 1],
-                         dz = zi - (double)x[3 * (int64_t)j + 2];
+    const int32_t sub = threadIdx.x % kRowLanes;
+    for (int32_t s = (int32_t)((blockIdx.x * blockDim.x + threadIdx.x) / kRowLanes); s < P.n;
+         s += (int32_t)(gridDim.x * blockDim.x / kRowLanes)) {
+        const auto xi = x[s];
+        const int32_t *row = R.row(s);
+        const int32_t c = R.count(s);
+        for (int32_t k = sub; k < c; k += kRowLanes) {
+            const int32_t j = row[k];
+            if (j < s) continue;  // each unordered pair once
+            const auto xj = x[j];
+            const double dx = (double)xi.x - (double)xj.x, dy = (double)xi.y - (double)xj.y,
+                         dz = (double)xi.z - (double)xj.z;
             const double r = sqrt(dx * dx + dy * dy + dz * dz);
             if (!(r < P.rmax + P.h)) continue;
             const int32_t b0 = max(0, (int32_t)floor((r - P.h) / P.dr - 0.5));
@@ -262,89 +378,119 @@ k_rdf_hist(Rows R, const T *__restrict__ x, AdjP P, double *__restrict__ hist) {
         }
     }
     __syncthreads();
-    for (int b = threadIdx.x; b < P.nbins; b += blockDim.x)
-        if (hb[b] != 0.0) unsafeAtomicAdd(&hist[b], hb[b]);
+    for (int b = threadIdx.x; b < P.nbins; b += blockDim.x) part[(int64_t)blockIdx.x * P.nbins + b] = hb[b];
 }
 
-// lambda_x += dL/dx with L = sum_b (g_b - t_b)^2: wb[b] = 2 (g_b - t_b) norm_b
-template <class T>
+// hist[b] = sum over the workgroups' parts, one workgroup per bin
 __global__ void __launch_bounds__(nd::kBlock)
-k_rdf_grad(Rows R, const T *__restrict__ x, AdjP P, const double *__restrict__ wb,
-           double *__restrict__ lam) {
-    const int32_t sl = blockIdx.x * blockDim.x + threadIdx.x;
-    if (sl >= P.n) return;
-    const int32_t i = R.perm[sl];
-    const int32_t *col = R.col(sl);
-    const int32_t c = R.count(sl);
-    const double xi = (double)x[3 * (int64_t)i], yi = (double)x[3 * (int64_t)i + 1],
-                 zi = (double)x[3 * (int64_t)i + 2];
-    double gx = 0.0, gy = 0.0, gz = 0.0;
-    for (int32_t k = 0; k < c; ++k) {
-        const int32_t j = col[(int64_t)k * 64];
-        const double dx = xi - (double)x[3 * (int64_t)j], dy = yi - (double)x[3 * (int64_t)j + 1],
-                     dz = zi - (double)x[3 * (int64_t)j + 2];
-        const double r = sqrt(dx * dx + dy * dy + dz * dz);
-        if (!(r < P.rmax + P.h)) continue;
-        const int32_t b0 = max(0, (int32_t)floor((r - P.h) / P.dr - 0.5));
-        const int32_t b1 = min(P.nbins - 1, (int32_t)ceil((r + P.h) / P.dr - 0.5));
-        double g = 0.0;
-        for (int32_t b = b0; b <= b1; ++b) g += wb[b] * rdf_dK(r - (b + 0.5) * P.dr, P.h);
-        const double s = g / r;
-        gx += s * dx;
-        gy += s * dy;
-        gz += s * dz;
+k_rdf_sum(const double *__restrict__ part, int32_t nparts, int32_t nbins, double *__restrict__ hist) {
+    __shared__ double sh[nd::kBlock / 64];
+    double v = 0.0;
+    for (int32_t k = threadIdx.x; k < nparts; k += nd::kBlock) v += part[(int64_t)k * nbins + blockIdx.x];
+    for (int o = 32; o > 0; o >>= 1) v += __shfl_down(v, o, 64);
+    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int k = 1; k < nd::kBlock / 64; ++k) v += sh[k];
+        hist[blockIdx.x] = v;
     }
-    lam[3 * (int64_t)i] += gx;
-    lam[3 * (int64_t)i + 1] += gy;
-    lam[3 * (int64_t)i + 2] += gz;
 }
+
+// Adjoint records of an atom, FP64.
+struct Lam {
+    double4 *x, *v, *a;  // lambda_x, lambda_v, a = w lambda_h
+};
 
 // lambda_h = lambda_v + dt lambda_x; lambda_v = lambda_h; a = w lambda_h
-__global__ void __launch_bounds__(nd::kBlock)
-k_adj_vec(const double *__restrict__ lx, double *__restrict__ lv, double *__restrict__ a, int64_t m,
-          double dt, double w) {
-    const int64_t k = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (k >= m) return;
-    const double h = lv[k] + dt * lx[k];
-    lv[k] = h;
-    a[k] = w * h;
+__device__ __forceinline__ void next_vec(const Lam &L, int32_t s, const double4 &lx, double dt, double w) {
+    double4 h = L.v[s];
+    h.x += dt * lx.x;
+    h.y += dt * lx.y;
+    h.z += dt * lx.z;
+    L.v[s] = h;
+    L.a[s] = make_double4(w * h.x, w * h.y, w * h.z, 0.0);
 }
 
-// lambda_x += J(x) a; dq, (eps, sigma) += (dF/dtheta)^T a.  Row i gives atom
-// i's own terms; each unordered pair sits in two rows, so its eps / sigma
-// term is taken with weight 1/2 from each.
+// Start of the reverse sweep: lambda_x = dL/dx_T with L = sum_b (g_b - t_b)^2,
+// wb[b] = 2 (g_b - t_b) norm_b; lambda_v = 0; then the last step's vectors.
 template <class T>
 __global__ void __launch_bounds__(nd::kBlock)
-k_adj_hvp(Rows R, const T *__restrict__ x, const double *__restrict__ q, AdjP P,
-          const double *__restrict__ a, double *__restrict__ lam, double *__restrict__ dq,
-          double *__restrict__ dpar) {
+k_rdf_grad(Rows R, const typename V4<T>::R *__restrict__ x, AdjP P, const double *__restrict__ wb, Lam L,
+           double wvec) {
+    const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+    const int32_t s = (int32_t)(t / kRowLanes), sub = (int32_t)(t % kRowLanes);
+    double gx = 0.0, gy = 0.0, gz = 0.0;
+    if (s < P.n) {
+        const int32_t *row = R.row(s);
+        const int32_t c = R.count(s);
+        const auto xi = x[s];
+        for (int32_t k = sub; k < c; k += kRowLanes) {
+            const auto xj = x[row[k]];
+            const double dx = (double)xi.x - (double)xj.x, dy = (double)xi.y - (double)xj.y,
+                         dz = (double)xi.z - (double)xj.z;
+            const double r = sqrt(dx * dx + dy * dy + dz * dz);
+            if (!(r < P.rmax + P.h)) continue;
+            const int32_t b0 = max(0, (int32_t)floor((r - P.h) / P.dr - 0.5));
+            const int32_t b1 = min(P.nbins - 1, (int32_t)ceil((r + P.h) / P.dr - 0.5));
+            double g = 0.0;
+            for (int32_t b = b0; b <= b1; ++b) g += wb[b] * rdf_dK(r - (b + 0.5) * P.dr, P.h);
+            const double f = g / r;
+            gx += f * dx;
+            gy += f * dy;
+            gz += f * dz;
+        }
+    }
+#pragma unroll
+    for (int off = 1; off < kRowLanes; off <<= 1) {
+        gx += __shfl_xor(gx, off, 64);
+        gy += __shfl_xor(gy, off, 64);
+        gz += __shfl_xor(gz, off, 64);
+    }
+    if (s >= P.n || sub != 0) return;
+    const double4 lx = make_double4(gx, gy, gz, 0.0);
+    L.x[s] = lx;
+    L.v[s] = make_double4(0.0, 0.0, 0.0, 0.0);
+    next_vec(L, s, lx, P.dt, wvec);
+}
+
+// One launch of the reverse sweep at x_k: lambda_x += J(x_k) a; dq, (eps,
+// sigma) += (dF/dtheta)^T a; and, for k > 0, the vectors of step k - 1 (the new
+// a goes to anext, since others still read this one).  Row i gives atom i's own
+// terms; each unordered pair sits in two rows, so its eps / sigma term is taken
+// with weight 1/2 from each.
+template <class T>
+__global__ void __launch_bounds__(nd::kBlock)
+k_adj_hvp(Rows R, const typename V4<T>::R *__restrict__ x, const double *__restrict__ qs,
+          const int32_t *__restrict__ orig, AdjP P, Lam L, double4 *__restrict__ anext, double wnext,
+          double *__restrict__ dq, double *__restrict__ dpar) {
     __shared__ double sh[2][nd::kBlock / 64];
     const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    const int32_t sl = (int32_t)(t / kRowLanes), sub = (int32_t)(t % kRowLanes);
-    const int32_t i = sl < P.n ? R.perm[sl] : 0;
+    const int32_t s = (int32_t)(t / kRowLanes), sub = (int32_t)(t % kRowLanes);
     double ge = 0.0, gs = 0.0;
     double mx = 0.0, my = 0.0, mz = 0.0, gq = 0.0;
-    if (sl < P.n) {
-        const double xi = (double)x[3 * (int64_t)i], yi = (double)x[3 * (int64_t)i + 1],
-                     zi = (double)x[3 * (int64_t)i + 2];
-        const double ai = a[3 * (int64_t)i], bi = a[3 * (int64_t)i + 1], ci = a[3 * (int64_t)i + 2];
-        const double qi = q[i];
-        const int32_t *col = R.col(sl);
-        const int32_t c = R.count(sl);
+    if (s < P.n) {
+        const auto xi = x[s];
+        const double4 ai = L.a[s];
+        const double qi = sizeof(T) == 8 ? (double)xi.w : qs[s];
+        const int32_t *row = R.row(s);
+        const int32_t c = R.count(s);
+        int32_t j = sub < c ? row[sub] : 0;
         for (int32_t k = sub; k < c; k += kRowLanes) {
-            const int32_t j = col[(int64_t)k * 64];
-            const double dx = xi - (double)x[3 * (int64_t)j], dy = yi - (double)x[3 * (int64_t)j + 1],
-                         dz = zi - (double)x[3 * (int64_t)j + 2];
+            const auto xj = x[j];
+            const double4 aj = L.a[j];
+            const double qj = sizeof(T) == 8 ? (double)xj.w : qs[j];
+            j = k + kRowLanes < c ? row[k + kRowLanes] : 0;
+            const double dx = (double)xi.x - (double)xj.x, dy = (double)xi.y - (double)xj.y,
+                         dz = (double)xi.z - (double)xj.z;
             const double r2 = dx * dx + dy * dy + dz * dz;
             if (!(r2 < P.rc2 || r2 < P.rcc2)) continue;
-            const PairD d = pair_d(r2, qi, q[j], P);
-            const double ax = ai - a[3 * (int64_t)j], ay = bi - a[3 * (int64_t)j + 1],
-                         az = ci - a[3 * (int64_t)j + 2];
+            const PairD d = pair_d(r2, qi, qj, P);
+            const double ax = ai.x - aj.x, ay = ai.y - aj.y, az = ai.z - aj.z;
             const double rda = dx * ax + dy * ay + dz * az;
             mx += d.s * ax + d.ds * rda * dx;
             my += d.s * ay + d.ds * rda * dy;
             mz += d.s * az + d.ds * rda * dz;
-            gq += P.kc * q[j] * d.H * rda;
+            gq += P.kc * qj * d.H * rda;
             ge += 0.5 * d.s_eps * rda;
             gs += 0.5 * d.s_sig * rda;
         }
@@ -357,11 +503,18 @@ k_adj_hvp(Rows R, const T *__restrict__ x, const double *__restrict__ q, AdjP P,
         mz += __shfl_xor(mz, off, 64);
         gq += __shfl_xor(gq, off, 64);
     }
-    if (sl < P.n && sub == 0) {
-        lam[3 * (int64_t)i] += mx;
-        lam[3 * (int64_t)i + 1] += my;
-        lam[3 * (int64_t)i + 2] += mz;
-        dq[i] += gq;
+    if (s < P.n && sub == 0) {
+        double4 lx = L.x[s];
+        lx.x += mx;
+        lx.y += my;
+        lx.z += mz;
+        L.x[s] = lx;
+        dq[orig[s]] += gq;
+        if (anext) {
+            Lam N = L;
+            N.a = anext;
+            next_vec(N, s, lx, P.dt, wnext);
+        }
     }
     for (int o = 32; o > 0; o >>= 1) {
         ge += __shfl_down(ge, o, 64);
@@ -371,10 +524,67 @@ k_adj_hvp(Rows R, const T *__restrict__ x, const double *__restrict__ q, AdjP P,
     if (lane == 0) { sh[0][w] = ge; sh[1][w] = gs; }
     __syncthreads();
     if (threadIdx.x == 0) {
-        double e = 0.0, s = 0.0;
-        for (int t = 0; t < (int)(blockDim.x >> 6); ++t) { e += sh[0][t]; s += sh[1][t]; }
-        unsafeAtomicAdd(&dpar[0], e);
-        unsafeAtomicAdd(&dpar[1], s);
+        double e = 0.0, g = 0.0;
+        for (int k = 0; k < (int)(blockDim.x >> 6); ++k) { e += sh[0][k]; g += sh[1][k]; }
+        // this workgroup's own words, summed over the sweep
+        dpar[2 * (int64_t)blockIdx.x] += e;
+        dpar[2 * (int64_t)blockIdx.x + 1] += g;
+    }
+}
+
+// The adjoint records from one order to another, by way of the caller's.
+__global__ void __launch_bounds__(nd::kBlock)
+k_adj_to_caller(const int32_t *__restrict__ orig, int32_t n, Lam L, Lam O) {
+    const int32_t s = blockIdx.x * blockDim.x + threadIdx.x;
+    if (s >= n) return;
+    const int32_t o = orig[s];
+    O.x[o] = L.x[s];
+    O.v[o] = L.v[s];
+    O.a[o] = L.a[s];
+}
+__global__ void __launch_bounds__(nd::kBlock)
+k_adj_from_caller(const int32_t *__restrict__ orig, int32_t n, Lam O, Lam L, const double *__restrict__ q,
+                  double *__restrict__ qs) {
+    const int32_t s = blockIdx.x * blockDim.x + threadIdx.x;
+    if (s >= n) return;
+    const int32_t o = orig[s];
+    L.x[s] = O.x[o];
+    L.v[s] = O.v[o];
+    L.a[s] = O.a[o];
+    qs[s] = q[o];
+}
+
+// (x, y, z) records in build order to n x 3 of the caller's order, in FP64.
+template <class R>
+__global__ void __launch_bounds__(nd::kBlock)
+k_adj_export(const R *__restrict__ a, const int32_t *__restrict__ orig, int32_t n, double *__restrict__ out) {
+    const int32_t s = blockIdx.x * blockDim.x + threadIdx.x;
+    if (s >= n) return;
+    const int64_t o = 3 * (int64_t)orig[s];
+    out[o] = (double)a[s].x;
+    out[o + 1] = (double)a[s].y;
+    out[o + 2] = (double)a[s].z;
+}
+
+// The workgroups' eps / sigma sums in index order (one workgroup).
+__global__ void __launch_bounds__(nd::kBlock)
+k_adj_sum_par(const double *__restrict__ part, int32_t m, double *__restrict__ out) {
+    __shared__ double sh[2][nd::kBlock / 64];
+    double e = 0.0, g = 0.0;
+    for (int32_t k = threadIdx.x; k < m; k += nd::kBlock) {
+        e += part[2 * (int64_t)k];
+        g += part[2 * (int64_t)k + 1];
+    }
+    for (int o = 32; o > 0; o >>= 1) {
+        e += __shfl_down(e, o, 64);
+        g += __shfl_down(g, o, 64);
+    }
+    if ((threadIdx.x & 63) == 0) { sh[0][threadIdx.x >> 6] = e; sh[1][threadIdx.x >> 6] = g; }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int k = 1; k < nd::kBlock / 64; ++k) { e += sh[0][k]; g += sh[1][k]; }
+        out[0] = e;
+        out[1] = g;
     }
 }
 
@@ -390,129 +600,197 @@ struct nd_adj {
     nd_adj_params p{};
     AdjP P{};
     bool dbl = true;
-    size_t esz = 8;  // bytes per state scalar
-    int32_t apl = 1;
     float rlist = 0.0f;
-    // state and scratch
-    nd::DevBuf x, v, F, xf, xs, codes, perm, nodes, store, flags, q, ckx, ckv, seg, lx, lv, a, dq,
-        dpar, hist, wb, rec, lists, lcnt;
-    nd::SortBufs sort;
+    // input of the call (FP64, caller's order) and charges
+    nd::DevBuf x0, v0, q;
+    // state: positions of the current segment (x_k for its every step) and of
+    // x_T, the drifted positions before a build, velocities (two: a build
+    // moves them), charges in build order (FP32)
+    nd::DevBuf seg, xT, tmp, x32, vel[2], qs;
+    int vcur = 0;
+    nd::DevBuf ckx, ckv, ck_orig;  // checkpoints of all segments but the last
+    // lists of the current segment's windows (slot w) and of x_T; a slot past
+    // the memory kept for them is shared, tagged with the window it holds
+    nd::DevBuf lists, lcnt, orig;
+    int32_t nwin = 0;              // orders kept: windows of a segment, x_T, and one spare
+    int32_t nslots = 0;            // rows kept
+    std::vector<int32_t> holds;    // window of each slot's rows
+    std::vector<int32_t> order;    // index of each window's order in orig
+    int32_t spare = 0;             // index of the unused order
+    nd::DevBuf bins, cell_of, cells, cpos, ckey;  // list build
+    nd::DevBuf lam, lam_caller, dq, dpar, out, hist, part, wb;
     int32_t cap = 0;  // row capacity
-    int32_t nck = 0;
     bool have_forward = false;
-    std::vector<double> target, rdf, norm;
+    std::vector<double> target, rdf, norm, weights;
     double loss = 0.0;
 };
 
 namespace {
 
-size_t state_bytes(const nd_adj *s) { return s->esz * 3 * (size_t)s->p.n; }
+// Bytes of rows kept for the reverse sweep; windows past them are listed again.
+constexpr size_t kListBytes = (size_t)4 << 30;
 
-template <class T> T *at(nd::DevBuf &b, size_t off_elems = 0) { return b.as<T>() + off_elems; }
-
-// neighbour rows (radius rlist, Hilbert key LBVH) at positions xp (device, T)
-// the walk's blocks of [cap][64] slots per 64 sorted atoms
 void reserve_rows(nd_adj *s) {
-    const size_t n64 = ((size_t)s->p.n + 63) & ~(size_t)63;
-    s->lists.reserve(sizeof(int32_t) * (size_t)s->cap * n64);
+    const size_t one = sizeof(int32_t) * (size_t)s->cap * (size_t)s->p.n;
+    s->nslots = (int32_t)std::max<size_t>(2, std::min<size_t>((size_t)s->nwin - 1, kListBytes / one));
+    s->lists.reserve(one * (size_t)s->nslots);
+    s->lcnt.reserve(sizeof(int32_t) * (size_t)s->p.n * (size_t)s->nslots);
+    s->holds.assign(s->nslots, -1);
 }
 
-Rows rows_of(nd_adj *s) {
-    return Rows{s->lists.as<int32_t>(), s->lcnt.as<int32_t>(), s->perm.as<int32_t>(), s->cap};
+int32_t slot_of(const nd_adj *s, int32_t w) { return std::min(w, s->nslots - 1); }
+
+Rows rows_of(nd_adj *s, int32_t w) {
+    const int64_t o = (int64_t)slot_of(s, w) * s->p.n;
+    return Rows{s->lists.as<int32_t>() + o * s->cap, s->lcnt.as<int32_t>() + o, s->cap};
 }
 
-template <class T>
-void build_list(nd_adj *s, const T *xp) {
-    nd_ctx *ctx = s->ctx;
-    hipStream_t st = ctx->stream;
-    const int32_t n = s->p.n, nL = n / s->apl;
-    const int64_t m = 3 * (int64_t)n;
-    int32_t *codes = s->codes.as<int32_t>(), *perm = s->perm.as<int32_t>(), *flags = s->flags.as<int32_t>();
-    k_adj_to_f32<T><<<nd::grid_for(m), nd::kBlock, 0, st>>>(xp, m, s->xf.as<float>());
-    nd::launch_fill_i32(st, flags, 8, 0);
-    nd::launch_morton(ctx, s->xf.as<float>(), n, ND_MORTON_HILBERT, nullptr, nullptr, codes, perm, flags + 2);
-    nd::radix_sort_pairs(st, s->sort, codes, perm, n, 0, 30);  // Hilbert keys are < 2^30
-    k_adj_pos4<<<nd::grid_for(n), nd::kBlock, 0, st>>>(s->xf.as<float>(), perm, n, s->xs.as<float4>());
-    nd::launch_lbvh(st, s->xs.as<float>(), 4, codes, nL, s->apl, s->rlist, 0, s->nodes.as<nd_node>(),
-                    s->store.as<int32_t>(), flags + 1);
-    for (int attempt = 0; attempt < 4; ++attempt) {
-        // the simulation's list walk over the sorted atoms, then original ids
-        nd::launch_list_walk(st, s->nodes.as<nd_node>(), s->rec.as<float4>(), s->xs.as<float4>(), n, nL,
-                             s->apl, s->rlist, s->cap, s->lists.as<int32_t>(), s->lcnt.as<int32_t>(), flags + 4);
-        k_adj_map_ids<<<dim3(nd::grid_for(n), (unsigned)s->cap), nd::kBlock, 0, st>>>(
-            perm, n, s->cap, s->lists.as<int32_t>(), s->lcnt.as<int32_t>());
-        ND_HIP(hipGetLastError());
-        int32_t h[8];
-        ND_HIP(hipMemcpyAsync(h, flags, sizeof(h), hipMemcpyDeviceToHost, st));
-        ND_HIP(hipStreamSynchronize(st));
-        if (h[2]) throw nd::Error(ND_ERR_DOMAIN, "adjoint: non-finite coordinate");
-        if (h[1] || h[6]) throw nd::Error(ND_ERR_STATE, "adjoint: malformed neighbour tree");
-        if (h[4] <= s->cap) return;
-        s->cap = h[4] + h[4] / 4 + 8;
-        // k_adj_map_ids takes one grid row per list row
-        if (s->cap > 65535) throw nd::Error(ND_ERR_CAPACITY, "adjoint: more than 65,535 neighbours per atom");
-        reserve_rows(s);
-        nd::launch_fill_i32(st, flags + 4, 3, 0);
-    }
-    throw nd::Error(ND_ERR_CAPACITY, "adjoint: neighbour rows kept overflowing");
-}
+int32_t *order_of(nd_adj *s, int32_t w) { return s->orig.as<int32_t>() + (size_t)s->order[w] * s->p.n; }
 
-template <class T>
-void compute_force(nd_adj *s, const T *xs) {
+// flags: [0] largest row, [1] status bits of the list builds since the last clear
+int32_t *flags_of(nd_adj *s) { return s->hist.as<int32_t>(); }
+double *hist_of(nd_adj *s) { return s->hist.as<double>() + 2; }
+
+// Rows (and, move, the new order) of window w at the positions in s->x32.
+template <class V>
+void build_rows(nd_adj *s, int32_t w, const V *x, const V *v, const int32_t *orig, V *xo, V *vo, int32_t *origo) {
     hipStream_t st = s->ctx->stream;
-    const int64_t m = 3 * (int64_t)s->p.n;
-    (void)m;
-    k_adj_force<T><<<nd::grid_for((int64_t)s->p.n * kRowLanes), nd::kBlock, 0, st>>>(rows_of(s),
-                                                                 xs, s->q.as<double>(), s->P,
-                                                                 s->F.as<unsigned long long>());
+    const int32_t n = s->p.n;
+    const int32_t max_cells = std::max(27, n / 2);
+    const float4 *x32 = s->x32.as<float4>();
+    const nd::CellGrid *cg = nd::launch_cell_bins(st, s->bins.p, x32, n, s->rlist, max_cells, s->cell_of.as<int2>(),
+                                                  s->cells.as<int32_t>(), flags_of(s) + 1);
+    k_adj_place<V><<<nd::grid_for(n), nd::kBlock, 0, st>>>(
+        x32, s->cell_of.as<int2>(), s->cells.as<int32_t>(), n, s->cpos.as<float4>(), s->ckey.as<int32_t>(), x, v, orig,
+        s->q.as<double>(), xo, vo, origo, s->qs.as<double>());
+    const Rows R = rows_of(s, w);
+    k_adj_rows<<<nd::grid_for(((int64_t)n + kListAtoms - 1) / kListAtoms * 64), nd::kBlock, 0, st>>>(
+        s->cpos.as<float4>(), s->ckey.as<int32_t>(), s->cells.as<int32_t>(), cg, n, s->rlist * s->rlist, s->cap,
+        const_cast<int32_t *>(R.lists), const_cast<int32_t *>(R.cnt), flags_of(s));
+    ND_HIP(hipGetLastError());
+    s->holds[slot_of(s, w)] = w;
+}
+
+// The list of window w for the positions in s->tmp (order from): moves the
+// state into its order, the positions to xo.
+template <class T>
+void build_list(nd_adj *s, int32_t w, int32_t from, typename V4<T>::R *xo) {
+    using V = typename V4<T>::R;
+    int32_t *orig = s->orig.as<int32_t>();
+    const size_t n = (size_t)s->p.n;
+    const int32_t src = from, dst = s->spare;
+    build_rows<V>(s, w, s->tmp.as<V>(), s->vel[s->vcur].as<V>(), orig + (size_t)src * n, xo,
+                  s->vel[s->vcur ^ 1].as<V>(), orig + (size_t)dst * n);
+    s->vcur ^= 1;
+    // the order window w had before is free now
+    s->spare = s->order[w];
+    s->order[w] = dst;
+}
+
+template <class T>
+typename V4<T>::R *seg_at(nd_adj *s, int32_t k) {
+    return s->seg.as<typename V4<T>::R>() + (size_t)k * s->p.n;
+}
+
+// The launch at step k (positions x, rows of window w).
+template <class T>
+void launch_step(nd_adj *s, int32_t w, const typename V4<T>::R *x, bool finish, typename V4<T>::R *vck,
+                 typename V4<T>::R *xo, bool to_bins) {
+    using V = typename V4<T>::R;
+    hipStream_t st = s->ctx->stream;
+    const unsigned g = nd::grid_for((int64_t)s->p.n * kRowLanes);
+    V *v = s->vel[s->vcur].as<V>();
+    float4 *x32 = to_bins ? s->x32.as<float4>() : nullptr;
+    const Rows R = rows_of(s, w);
+    const double *qs = s->qs.as<double>();
+    if (finish && xo) k_adj_step<T, true, true><<<g, nd::kBlock, 0, st>>>(R, x, qs, s->P, v, vck, xo, x32);
+    else if (xo) k_adj_step<T, false, true><<<g, nd::kBlock, 0, st>>>(R, x, qs, s->P, v, vck, xo, x32);
+    else k_adj_step<T, true, false><<<g, nd::kBlock, 0, st>>>(R, x, qs, s->P, v, vck, nullptr, nullptr);
     ND_HIP(hipGetLastError());
 }
 
-// Advance steps [k0, k1) from (x, v) with F = F(x_k0) already in s->F and the
-// list valid for x_k0.  If seg != null, x_k (k0 <= k < k1) is stored there.
+// Steps k0 .. of a segment, whose first list (window 0, x_k0 in seg[0]) is
+// there.  forward: to k1, with the list at k1 (the next segment's first, or
+// x_T's); else (recompute) to x_{k1-1}.
 template <class T>
-void advance(nd_adj *s, int32_t k0, int32_t k1, T *seg) {
-    hipStream_t st = s->ctx->stream;
-    const int64_t m = 3 * (int64_t)s->p.n;
-    T *x = s->x.as<T>(), *v = s->v.as<T>();
-    for (int32_t k = k0; k < k1; ++k) {
-        if (seg)
-            ND_HIP(hipMemcpyAsync(seg + (size_t)(k - k0) * m, x, state_bytes(s), hipMemcpyDeviceToDevice, st));
-        k_adj_kick_drift<T><<<nd::grid_for(m), nd::kBlock, 0, st>>>(x, v, s->F.as<unsigned long long>(), s->P);
-        if ((k + 1) % s->p.rebuild_every == 0) build_list<T>(s, x);
-        compute_force<T>(s, x);
-        k_adj_kick<T><<<nd::grid_for(m), nd::kBlock, 0, st>>>(v, s->F.as<unsigned long long>(), s->P);
-        ND_HIP(hipGetLastError());
+void advance(nd_adj *s, int32_t k0, int32_t k1, bool forward, bool finish_first, typename V4<T>::R *vck) {
+    using V = typename V4<T>::R;
+    const int32_t W = s->p.rebuild_every, T_ = s->p.nsteps;
+    const int32_t last = forward ? k1 : k1 - 1;  // positions wanted up to here
+    for (int32_t k = k0; k < last; ++k) {
+        const int32_t w = (k - k0) / W;
+        const bool end = k + 1 == k1, build = (k + 1) % W == 0 || k + 1 == T_;
+        V *xo = build ? s->tmp.as<V>() : seg_at<T>(s, k + 1 - k0);
+        launch_step<T>(s, w, seg_at<T>(s, k - k0), k > k0 || finish_first, k == k0 ? vck : nullptr, xo, build);
+        if (!build) continue;
+        if (k + 1 == T_) build_list<T>(s, s->nwin - 2, s->order[w], s->xT.as<V>());
+        else build_list<T>(s, end ? 0 : w + 1, s->order[w], seg_at<T>(s, end ? 0 : k + 1 - k0));
     }
+}
+
+// Reads the flags; throws what the list builds found.  Returns the largest row.
+int32_t check_flags(const int32_t *h) {
+    if (h[1] & nd::kStatusDomain) throw nd::Error(ND_ERR_DOMAIN, "adjoint: non-finite coordinate");
+    // (the list build took one grid row per list row)
+    if (h[0] > 65535) throw nd::Error(ND_ERR_CAPACITY, "adjoint: more than 65,535 neighbours per atom");
+    return h[0];
 }
 
 template <class T>
 void forward_impl(nd_adj *s) {
+    using V = typename V4<T>::R;
     hipStream_t st = s->ctx->stream;
-    const int32_t K = s->p.checkpoint_every, T_ = s->p.nsteps;
-    T *x = s->x.as<T>(), *v = s->v.as<T>();
-    build_list<T>(s, x);
-    compute_force<T>(s, x);
-    for (int32_t c = 0; c * K < T_; ++c) {
-        ND_HIP(hipMemcpyAsync(s->ckx.as<T>() + (size_t)c * 3 * s->p.n, x, state_bytes(s), hipMemcpyDeviceToDevice, st));
-        ND_HIP(hipMemcpyAsync(s->ckv.as<T>() + (size_t)c * 3 * s->p.n, v, state_bytes(s), hipMemcpyDeviceToDevice, st));
-        const int32_t k1 = (c + 1) * K < T_ ? (c + 1) * K : T_;
-        advance<T>(s, c * K, k1, (T *)nullptr);
+    const int32_t K = s->p.checkpoint_every, T_ = s->p.nsteps, n = s->p.n, nb = s->p.nbins;
+    const size_t vb = sizeof(V) * (size_t)n, ib = sizeof(int32_t) * (size_t)n;
+    std::vector<double> h(2 + nb);
+    const int32_t *hf = reinterpret_cast<const int32_t *>(h.data());
+    for (int attempt = 0;; ++attempt) {
+        if (attempt == 8) throw nd::Error(ND_ERR_CAPACITY, "adjoint: neighbour rows kept overflowing");
+        auto grow = [&](int32_t most) {
+            s->cap = most + most / 4 + 8;
+            reserve_rows(s);
+        };
+        nd::launch_fill_i32(st, flags_of(s), 4, 0);
+        s->vcur = 0;
+        k_adj_init<T><<<nd::grid_for(n), nd::kBlock, 0, st>>>(
+            s->x0.as<double>(), s->v0.as<double>(), s->q.as<double>(), n, s->tmp.as<V>(), s->vel[0].as<V>(),
+            s->x32.as<float4>(), order_of(s, s->nwin - 2));
+        build_list<T>(s, 0, s->order[s->nwin - 2], seg_at<T>(s, 0));
+        // room for the first list is made before the steps run on it
+        ND_HIP(hipMemcpyAsync(h.data(), s->hist.p, 8, hipMemcpyDeviceToHost, st));
+        ND_HIP(hipStreamSynchronize(st));
+        if (const int32_t most = check_flags(hf); most > s->cap) {
+            grow(most);
+            continue;
+        }
+        for (int32_t c = 0; c * K < T_; ++c) {
+            const int32_t k0 = c * K, k1 = std::min((c + 1) * K, T_);
+            V *vck = nullptr;
+            if (k1 < T_) {  // the last segment needs no checkpoint: its positions stay
+                ND_HIP(hipMemcpyAsync(s->ckx.as<V>() + (size_t)c * n, seg_at<T>(s, 0), vb, hipMemcpyDeviceToDevice, st));
+                ND_HIP(hipMemcpyAsync(s->ck_orig.as<int32_t>() + (size_t)c * n, order_of(s, 0), ib,
+                                      hipMemcpyDeviceToDevice, st));
+                vck = s->ckv.as<V>() + (size_t)c * n;
+            }
+            advance<T>(s, k0, k1, true, c > 0, vck);
+        }
+        // the last half kick, and the final frame's radial distribution
+        launch_step<T>(s, s->nwin - 2, s->xT.as<V>(), true, nullptr, nullptr, false);
+        const Rows R = rows_of(s, s->nwin - 2);
+        const unsigned hb = std::min<unsigned>(nd::grid_for((int64_t)n * kRowLanes), kHistBlocks);
+        k_rdf_hist<T><<<hb, nd::kBlock, 0, st>>>(R, s->xT.as<V>(), s->P, s->part.as<double>());
+        k_rdf_sum<<<nb, nd::kBlock, 0, st>>>(s->part.as<double>(), (int32_t)hb, nb, hist_of(s));
+        ND_HIP(hipGetLastError());
+        ND_HIP(hipMemcpyAsync(h.data(), s->hist.p, sizeof(double) * h.size(), hipMemcpyDeviceToHost, st));
+        ND_HIP(hipStreamSynchronize(st));
+        const int32_t most = check_flags(hf);
+        if (most <= s->cap) break;
+        grow(most);  // a later list overflowed: its forces were short
     }
-    // final frame: radial distribution (pairs of the list valid at x_T)
-    if (T_ % s->p.rebuild_every != 0) build_list<T>(s, x);
-    const int32_t nb = s->p.nbins;
-    k_zero_f64<<<nd::grid_for(nb), nd::kBlock, 0, st>>>(s->hist.as<double>(), nb);
-    k_rdf_hist<T><<<nd::grid_for(s->p.n), nd::kBlock, 0, st>>>(rows_of(s),
-                                                                x, s->P, s->hist.as<double>());
-    ND_HIP(hipGetLastError());
-    std::vector<double> h(nb);
-    ND_HIP(hipMemcpyAsync(h.data(), s->hist.p, sizeof(double) * nb, hipMemcpyDeviceToHost, st));
-    ND_HIP(hipStreamSynchronize(st));
     s->rdf.resize(nb);
     s->loss = 0.0;
     for (int32_t b = 0; b < nb; ++b) {
-        s->rdf[b] = s->norm[b] * h[b];
+        s->rdf[b] = s->norm[b] * h[2 + b];
         if (!s->target.empty()) s->loss += (s->rdf[b] - s->target[b]) * (s->rdf[b] - s->target[b]);
     }
     s->have_forward = true;
@@ -520,46 +798,67 @@ void forward_impl(nd_adj *s) {
 
 template <class T>
 void backward_impl(nd_adj *s) {
+    using V = typename V4<T>::R;
     hipStream_t st = s->ctx->stream;
     const int32_t K = s->p.checkpoint_every, T_ = s->p.nsteps, W = s->p.rebuild_every, n = s->p.n;
-    const int64_t m = 3 * (int64_t)n;
-    double *lx = s->lx.as<double>(), *lv = s->lv.as<double>(), *a = s->a.as<double>();
-    k_zero_f64<<<nd::grid_for(m), nd::kBlock, 0, st>>>(lx, m);
-    k_zero_f64<<<nd::grid_for(m), nd::kBlock, 0, st>>>(lv, m);
-    k_zero_f64<<<nd::grid_for(n), nd::kBlock, 0, st>>>(s->dq.as<double>(), n);
-    k_zero_f64<<<1, 64, 0, st>>>(s->dpar.as<double>(), 2);
-    // dL/dx_T: x still holds x_T and the list is valid there
-    std::vector<double> wb(s->p.nbins);
+    const size_t vb = sizeof(V) * (size_t)n, ib = sizeof(int32_t) * (size_t)n;
+    const unsigned g = nd::grid_for(n), gr = nd::grid_for((int64_t)n * kRowLanes);
+    double4 *lam = s->lam.as<double4>(), *lc = s->lam_caller.as<double4>();
+    Lam L{lam, lam + n, lam + 2 * (size_t)n}, C{lc, lc + n, lc + 2 * (size_t)n};
+    double4 *a2 = lam + 3 * (size_t)n;
+    k_zero_f64<<<g, nd::kBlock, 0, st>>>(s->dq.as<double>(), n);
+    k_zero_f64<<<nd::grid_for(2 * (int64_t)gr), nd::kBlock, 0, st>>>(s->dpar.as<double>(), 2 * (int64_t)gr);
+    std::vector<double> &wb = s->weights;  // outlives the copy
+    wb.resize(s->p.nbins);
     for (int32_t b = 0; b < s->p.nbins; ++b) wb[b] = 2.0 * (s->rdf[b] - s->target[b]) * s->norm[b];
     ND_HIP(hipMemcpyAsync(s->wb.p, wb.data(), sizeof(double) * wb.size(), hipMemcpyHostToDevice, st));
-    k_rdf_grad<T><<<nd::grid_for(n), nd::kBlock, 0, st>>>(rows_of(s),
-                                                           s->x.as<T>(), s->P, s->wb.as<double>(), lx);
-    ND_HIP(hipGetLastError());
-    T *seg = s->seg.as<T>();
+    auto weight = [&](int32_t k) { return k == 0 ? s->P.c : 2.0 * s->P.c; };
+    const int32_t fin = s->nwin - 2;
+    if (s->holds[slot_of(s, fin)] != fin) throw nd::Error(ND_ERR_STATE, "adjoint: the final list is gone");
+    k_rdf_grad<T><<<gr, nd::kBlock, 0, st>>>(rows_of(s, fin), s->xT.as<V>(), s->P, s->wb.as<double>(), L,
+                                             weight(T_ - 1));
+    const int32_t *at = order_of(s, fin);  // the adjoint records' order
     for (int32_t c = (T_ - 1) / K; c >= 0; --c) {
-        const int32_t k0 = c * K, k1 = (c + 1) * K < T_ ? (c + 1) * K : T_;
-        // recompute the segment from its checkpoint, storing x_k0 .. x_{k1-1}
-        ND_HIP(hipMemcpyAsync(s->x.p, s->ckx.as<T>() + (size_t)c * m, state_bytes(s), hipMemcpyDeviceToDevice, st));
-        ND_HIP(hipMemcpyAsync(s->v.p, s->ckv.as<T>() + (size_t)c * m, state_bytes(s), hipMemcpyDeviceToDevice, st));
-        build_list<T>(s, s->x.as<T>());  // k0 is a multiple of W
-        compute_force<T>(s, s->x.as<T>());
-        advance<T>(s, k0, k1, seg);
-        int32_t list_at = -1;
+        const int32_t k0 = c * K, k1 = std::min((c + 1) * K, T_);
+        if (k1 < T_) {
+            // the records wait in the caller's order while the segment is
+            // recomputed from its checkpoint
+            k_adj_to_caller<<<g, nd::kBlock, 0, st>>>(at, n, L, C);
+            at = nullptr;
+            ND_HIP(hipMemcpyAsync(s->tmp.p, s->ckx.as<V>() + (size_t)c * n, vb, hipMemcpyDeviceToDevice, st));
+            ND_HIP(hipMemcpyAsync(s->vel[s->vcur].p, s->ckv.as<V>() + (size_t)c * n, vb, hipMemcpyDeviceToDevice, st));
+            ND_HIP(hipMemcpyAsync(order_of(s, fin), s->ck_orig.as<int32_t>() + (size_t)c * n, ib,
+                                  hipMemcpyDeviceToDevice, st));
+            k_adj_to_f32<V><<<g, nd::kBlock, 0, st>>>(s->tmp.as<V>(), n, s->x32.as<float4>());
+            build_list<T>(s, 0, s->order[fin], seg_at<T>(s, 0));
+            advance<T>(s, k0, k1, false, false, nullptr);
+        }
+        int32_t win = -1;
         for (int32_t k = k1 - 1; k >= k0; --k) {
-            const int32_t w0 = (k / W) * W;
-            const T *xk = seg + (size_t)(k - k0) * m;
-            if (list_at != w0) {
-                build_list<T>(s, seg + (size_t)(w0 - k0) * m);
-                list_at = w0;
+            const int32_t w = (k - k0) / W;
+            if (w != win) {
+                if (at) k_adj_to_caller<<<g, nd::kBlock, 0, st>>>(at, n, L, C);
+                at = order_of(s, w);
+                k_adj_from_caller<<<g, nd::kBlock, 0, st>>>(at, n, C, L, s->q.as<double>(), s->qs.as<double>());
+                if (s->holds[slot_of(s, w)] != w) {
+                    // rows not kept: listed again for the window's first positions, in its order
+                    k_adj_to_f32<V><<<g, nd::kBlock, 0, st>>>(seg_at<T>(s, w * W), n, s->x32.as<float4>());
+                    build_rows<V>(s, w, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr);
+                }
+                win = w;
             }
-            k_adj_vec<<<nd::grid_for(m), nd::kBlock, 0, st>>>(lx, lv, a, m, s->P.dt,
-                                                                k == 0 ? s->P.c : 2.0 * s->P.c);
-            k_adj_hvp<T><<<nd::grid_for((int64_t)n * kRowLanes), nd::kBlock, 0, st>>>(rows_of(s),
-                                                                  xk, s->q.as<double>(), s->P, a, lx,
-                                                                  s->dq.as<double>(), s->dpar.as<double>());
+            k_adj_hvp<T><<<gr, nd::kBlock, 0, st>>>(rows_of(s, w), seg_at<T>(s, k - k0), s->qs.as<double>(), at, s->P,
+                                                    L, k > 0 ? a2 : nullptr, k > 0 ? weight(k - 1) : 0.0,
+                                                    s->dq.as<double>(), s->dpar.as<double>());
             ND_HIP(hipGetLastError());
+            std::swap(L.a, a2);
         }
     }
+    double *out = s->out.as<double>();
+    k_adj_export<double4><<<g, nd::kBlock, 0, st>>>(L.x, at, n, out);
+    k_adj_export<double4><<<g, nd::kBlock, 0, st>>>(L.v, at, n, out + 3 * (size_t)n);
+    k_adj_sum_par<<<1, nd::kBlock, 0, st>>>(s->dpar.as<double>(), (int32_t)gr, out + 6 * (size_t)n);
+    ND_HIP(hipGetLastError());
 }
 
 }  // namespace
@@ -572,8 +871,7 @@ int nd_adj_create(nd_ctx *ctx, const nd_adj_params *p, nd_adj **out) {
     *out = nullptr;
     ND_REQUIRE(p->n >= 8 && p->n % 4 == 0 && p->nsteps >= 1 && p->checkpoint_every >= 1 &&
                    p->rebuild_every >= 1,
-               "nd_adj_create: n >= 8 and a multiple of 4 (list leaves of 4, 8 or 16 atoms); nsteps, "
-               "checkpoint_every, rebuild_every >= 1");
+               "nd_adj_create: n >= 8 and a multiple of 4; nsteps, checkpoint_every, rebuild_every >= 1");
     ND_REQUIRE(p->checkpoint_every % p->rebuild_every == 0,
                "nd_adj_create: checkpoint_every must be a multiple of rebuild_every");
     ND_REQUIRE(p->precision == ND_PREC_FP32 || p->precision == ND_PREC_FP64,
@@ -589,38 +887,37 @@ int nd_adj_create(nd_ctx *ctx, const nd_adj_params *p, nd_adj **out) {
         s->ctx = ctx;
         s->p = *p;
         s->dbl = p->precision == ND_PREC_FP64;
-        s->esz = s->dbl ? 8 : 4;
-        s->apl = 4;
-        for (int32_t a : {16, 8, 4})
-            if (p->n % a == 0 && p->n / a >= 2) { s->apl = a; break; }
         const double reach = std::max(std::max(p->rc, p->rc_coul), p->rdf_rmax + p->rdf_h);
         // FP32 copies of the coordinates feed the list: pad by their rounding
         s->rlist = (float)((reach + p->skin) * (1.0 + 2.0e-6) + 1e-6);
-        const size_t n = (size_t)p->n, m = 3 * n;
-        const int32_t nck = (p->nsteps + p->checkpoint_every - 1) / p->checkpoint_every;
-        s->nck = nck;
-        s->x.reserve(s->esz * m);
-        s->v.reserve(s->esz * m);
-        s->F.reserve(8 * m);
-        s->xf.reserve(4 * m);
-        s->q.reserve(8 * n);
-        s->ckx.reserve(s->esz * m * (size_t)nck);
-        s->ckv.reserve(s->esz * m * (size_t)nck);
-        s->seg.reserve(s->esz * m * (size_t)p->checkpoint_every);
-        s->lx.reserve(8 * m);
-        s->lv.reserve(8 * m);
-        s->a.reserve(8 * m);
-        s->dq.reserve(8 * n);
-        s->dpar.reserve(16);
-        s->hist.reserve(8 * (size_t)p->nbins);
-        s->xs.reserve(sizeof(float4) * n);
-        s->lcnt.reserve(4 * n);
-        s->rec.reserve(8 * sizeof(float4) * (size_t)(p->n / s->apl - 1));
-        s->codes.reserve(4 * n);
-        s->perm.reserve(4 * n);
-        s->nodes.reserve(sizeof(nd_node) * (size_t)(2 * (p->n / s->apl) - 1));
-        s->store.reserve(sizeof(int32_t) * nd::lbvh_scratch_ints(p->n / s->apl));
-        s->flags.reserve(64);  // [0..3] tree build status words, [4..6] the walk's counters
+        const size_t n = (size_t)p->n, vb = (s->dbl ? sizeof(double4) : sizeof(float4)) * n;
+        const int32_t K = std::min(p->checkpoint_every, p->nsteps);
+        const size_t nck = (size_t)((p->nsteps - 1) / p->checkpoint_every);  // all segments but the last
+        // windows of a segment, then x_T's, then the spare order
+        s->nwin = (K + p->rebuild_every - 1) / p->rebuild_every + 2;
+        s->order.resize(s->nwin - 1);
+        for (int32_t w = 0; w < s->nwin - 1; ++w) s->order[w] = w;
+        s->spare = s->nwin - 1;
+        for (nd::DevBuf *b : {&s->x0, &s->v0}) b->reserve(24 * n);
+        for (nd::DevBuf *b : {&s->q, &s->qs, &s->dq}) b->reserve(8 * n);
+        for (nd::DevBuf *b : {&s->xT, &s->tmp, &s->vel[0], &s->vel[1]}) b->reserve(vb);
+        s->seg.reserve(vb * (size_t)K);
+        s->ckx.reserve(vb * nck);
+        s->ckv.reserve(vb * nck);
+        s->ck_orig.reserve(4 * n * nck);
+        s->orig.reserve(4 * n * (size_t)s->nwin);
+        s->x32.reserve(sizeof(float4) * n);
+        s->cpos.reserve(sizeof(float4) * n);
+        s->ckey.reserve(4 * n);
+        s->cell_of.reserve(sizeof(int2) * n);
+        s->cells.reserve(4 * (size_t)(std::max(27, p->n / 2) + 1));
+        s->bins.reserve(nd::cell_bins_bytes());
+        s->lam.reserve(4 * sizeof(double4) * n);
+        s->lam_caller.reserve(3 * sizeof(double4) * n);
+        s->dpar.reserve(16 * (size_t)nd::grid_for((int64_t)n * kRowLanes));
+        s->out.reserve(8 * (6 * n + 2));
+        s->hist.reserve(8 * (2 + (size_t)p->nbins));  // flags, then the bins
+        s->part.reserve(8 * (size_t)kHistBlocks * (size_t)p->nbins);
         s->wb.reserve(8 * (size_t)p->nbins);
         s->cap = 96;
         reserve_rows(s);
@@ -646,10 +943,10 @@ int nd_adj_destroy(nd_adj *s) {
         (void)hipSetDevice(s->ctx->device);
         (void)hipStreamSynchronize(s->ctx->stream);
     }
-    nd::DevBuf *bufs[] = {&s->rec, &s->lists, &s->lcnt, &s->x, &s->v, &s->F, &s->xf, &s->xs, &s->codes, &s->perm, &s->nodes,
-                          &s->store, &s->flags, &s->q, &s->ckx, &s->ckv, &s->seg, &s->lx, &s->lv,
-                          &s->a, &s->dq, &s->dpar, &s->hist, &s->wb,
-                          &s->sort.keys_alt, &s->sort.vals_alt, &s->sort.hist, &s->sort.flags};
+    nd::DevBuf *bufs[] = {&s->x0, &s->v0, &s->q, &s->seg, &s->xT, &s->tmp, &s->x32, &s->vel[0], &s->vel[1], &s->qs,
+                          &s->ckx, &s->ckv, &s->ck_orig, &s->lists, &s->lcnt, &s->orig, &s->bins, &s->cell_of,
+                          &s->cells, &s->cpos, &s->ckey, &s->lam, &s->lam_caller, &s->dq, &s->dpar, &s->out,
+                          &s->hist, &s->part, &s->wb};
     for (auto *b : bufs) b->release();
     delete s;
     return ND_OK;
@@ -670,6 +967,10 @@ int nd_adj_set_potential(nd_adj *s, double eps, double sigma) {
     P.kc = p.k_coul;
     P.rcc = p.rc_coul;
     P.rcc2 = p.rc_coul > 0.0 ? p.rc_coul * p.rc_coul : 0.0;
+    P.sig2 = sigma * sigma;
+    P.inv_eps = 1.0 / eps;
+    P.inv_sigma = 1.0 / sigma;
+    P.inv_rcc2 = p.rc_coul > 0.0 ? 1.0 / P.rcc2 : 0.0;
     P.dt = p.dt;
     P.c = 0.5 * p.dt;
     P.flj_rc = lj_F(p.rc, eps, sigma);
@@ -692,15 +993,9 @@ int nd_adj_forward(nd_adj *s, const double *h_x0, const double *h_v0, const doub
     std::vector<double> q(n, 0.0);
     if (h_q) q.assign(h_q, h_q + n);
     ND_HIP(hipMemcpyAsync(s->q.p, q.data(), 8 * n, hipMemcpyHostToDevice, st));
-    if (s->dbl) {
-        ND_HIP(hipMemcpyAsync(s->x.p, h_x0, 8 * m, hipMemcpyHostToDevice, st));
-        ND_HIP(hipMemcpyAsync(s->v.p, h_v0, 8 * m, hipMemcpyHostToDevice, st));
-    } else {
-        std::vector<float> xf(h_x0, h_x0 + m), vf(h_v0, h_v0 + m);
-        ND_HIP(hipMemcpyAsync(s->x.p, xf.data(), 4 * m, hipMemcpyHostToDevice, st));
-        ND_HIP(hipMemcpyAsync(s->v.p, vf.data(), 4 * m, hipMemcpyHostToDevice, st));
-        ND_HIP(hipStreamSynchronize(st));
-    }
+    ND_HIP(hipMemcpyAsync(s->x0.p, h_x0, 8 * m, hipMemcpyHostToDevice, st));
+    ND_HIP(hipMemcpyAsync(s->v0.p, h_v0, 8 * m, hipMemcpyHostToDevice, st));
+    s->have_forward = false;
     s->target.clear();
     if (h_target) s->target.assign(h_target, h_target + s->p.nbins);
     if (s->dbl) forward_impl<double>(s);
@@ -717,20 +1012,20 @@ int nd_adj_final_state(nd_adj *s, double *h_x, double *h_v) {
     ND_HIP(hipSetDevice(ctx->device));
     const size_t m = 3 * (size_t)s->p.n;
     hipStream_t st = ctx->stream;
+    const unsigned g = nd::grid_for(s->p.n);
+    const int32_t *at = order_of(s, s->nwin - 2);
+    double *out = s->out.as<double>();
     if (s->dbl) {
-        if (h_x) ND_HIP(hipMemcpyAsync(h_x, s->x.p, 8 * m, hipMemcpyDeviceToHost, st));
-        if (h_v) ND_HIP(hipMemcpyAsync(h_v, s->v.p, 8 * m, hipMemcpyDeviceToHost, st));
-        ND_HIP(hipStreamSynchronize(st));
+        k_adj_export<double4><<<g, nd::kBlock, 0, st>>>(s->xT.as<double4>(), at, s->p.n, out);
+        k_adj_export<double4><<<g, nd::kBlock, 0, st>>>(s->vel[s->vcur].as<double4>(), at, s->p.n, out + m);
     } else {
-        std::vector<float> xf(m), vf(m);
-        ND_HIP(hipMemcpyAsync(xf.data(), s->x.p, 4 * m, hipMemcpyDeviceToHost, st));
-        ND_HIP(hipMemcpyAsync(vf.data(), s->v.p, 4 * m, hipMemcpyDeviceToHost, st));
-        ND_HIP(hipStreamSynchronize(st));
-        for (size_t k = 0; k < m; ++k) {
-            if (h_x) h_x[k] = xf[k];
-            if (h_v) h_v[k] = vf[k];
-        }
+        k_adj_export<float4><<<g, nd::kBlock, 0, st>>>(s->xT.as<float4>(), at, s->p.n, out);
+        k_adj_export<float4><<<g, nd::kBlock, 0, st>>>(s->vel[s->vcur].as<float4>(), at, s->p.n, out + m);
     }
+    ND_HIP(hipGetLastError());
+    if (h_x) ND_HIP(hipMemcpyAsync(h_x, out, 8 * m, hipMemcpyDeviceToHost, st));
+    if (h_v) ND_HIP(hipMemcpyAsync(h_v, out + m, 8 * m, hipMemcpyDeviceToHost, st));
+    ND_HIP(hipStreamSynchronize(st));
     ND_API_END(ctx)
 }
 
@@ -744,10 +1039,11 @@ int nd_adj_backward(nd_adj *s, double *h_dx0, double *h_dv0, double *h_dq, doubl
     else backward_impl<float>(s);
     hipStream_t st = ctx->stream;
     const size_t n = (size_t)s->p.n;
-    if (h_dx0) ND_HIP(hipMemcpyAsync(h_dx0, s->lx.p, 8 * 3 * n, hipMemcpyDeviceToHost, st));
-    if (h_dv0) ND_HIP(hipMemcpyAsync(h_dv0, s->lv.p, 8 * 3 * n, hipMemcpyDeviceToHost, st));
+    const double *out = s->out.as<double>();
+    if (h_dx0) ND_HIP(hipMemcpyAsync(h_dx0, out, 24 * n, hipMemcpyDeviceToHost, st));
+    if (h_dv0) ND_HIP(hipMemcpyAsync(h_dv0, out + 3 * n, 24 * n, hipMemcpyDeviceToHost, st));
     if (h_dq) ND_HIP(hipMemcpyAsync(h_dq, s->dq.p, 8 * n, hipMemcpyDeviceToHost, st));
-    if (h_dparams) ND_HIP(hipMemcpyAsync(h_dparams, s->dpar.p, 16, hipMemcpyDeviceToHost, st));
+    if (h_dparams) ND_HIP(hipMemcpyAsync(h_dparams, out + 6 * n, 16, hipMemcpyDeviceToHost, st));
     ND_HIP(hipStreamSynchronize(st));
     // the recompute overwrote the final state: the forward must be rerun before another backward
     s->have_forward = false;

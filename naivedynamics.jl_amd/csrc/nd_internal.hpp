@@ -154,17 +154,6 @@ void launch_lbvh(hipStream_t s, const float *xyz_sorted, int32_t xyz_stride,
 // addressed through a buffer resource whose byte range (cap * 256) is int32.
 constexpr int32_t kMaxListRows = (1 << 23) - 1;
 
-// nd_sim.hip: the two-phase list walk over an LBVH of float4 positions
-// (sorted; leaf boxes +- rlist/2) with 4, 8, 16 or 32 atoms per leaf.  It
-// writes the four-wide records into rec (8 float4 per internal node), one
-// block of [cap][64] int32 neighbour slots per 64 sorted atoms into nbr (the
-// neighbours' sorted indices), each atom's count into ncount, and into ctr:
-// [0] the largest count (atomic max), [1] 1 if any count exceeds cap,
-// [2] kStatusTree if the tree was malformed.
-void launch_list_walk(hipStream_t st, const nd_node *nodes, float4 *rec, const float4 *pos, int32_t n,
-                      int32_t nL, int32_t apl, float rlist, int32_t cap, int32_t *nbr, int32_t *ncount,
-                      int32_t *ctr);
-
 // nd_traverse.hip
 // own_tree: the tree was built by launch_lbvh (well formed: left pointers and
 // ropes describe one depth-first order), which allows the wave-cooperative walk.
@@ -235,6 +224,14 @@ enum : int32_t { kPairsLeaf = 0, kPairsPointOwn = 1, kPairsPointRoot = 2, kPairs
 // is <= cap).  Synchronous.
 int64_t tree_list(nd_ctx *ctx, const float *d_xyz, int32_t kind, int32_t n, int32_t apl, float r, int32_t pred,
                   int32_t morton, nd_pair *d_out, int64_t cap);
+// Atoms into cells of side >= r (at most max_cells), kernels only: cell and
+// place of each in cell_of, first place of each cell in cells (max_cells + 1
+// ints; cells[ncell] = n), kStatusDomain into *status for a non-finite
+// coordinate.  work: cell_bins_bytes() of device memory.  Returns the grid's
+// device address.
+size_t cell_bins_bytes();
+const CellGrid *launch_cell_bins(hipStream_t st, void *work, const float4 *x, int32_t n, float r, int32_t max_cells,
+                                 int2 *cell_of, int32_t *cells, int32_t *status);
 // Bounding box of the atoms with finite coordinates; false if there are none.
 // Synchronous.
 bool atoms_box(nd_ctx *ctx, const float *d_xyz, int32_t n, double lo[3], double hi[3]);

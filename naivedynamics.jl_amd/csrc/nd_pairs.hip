@@ -475,15 +475,36 @@ __device__ __forceinline__ int32_t f2ord(float f) {
 }
 __device__ __forceinline__ float ord2f(int32_t i) { return __int_as_float(i >= 0 ? i : i ^ 0x7FFFFFFF); }
 
-// Per-workgroup bounding boxes of the finite coordinates (ATOMS: of the atoms
-// whose three coordinates are finite).  No atomics: 64 workgroups' on six words
-// took 21-29 us, these and the launch that joins them take 6 + 4.  Also clears
-// the cell counts and two words.
-template <bool ATOMS>
+// Positions as (x, y, z) triples or as float4.
+struct Xyz3 {
+    const float *p;
+    __device__ __forceinline__ float3 operator()(int32_t i) const {
+        return make_float3(p[3 * (int64_t)i], p[3 * (int64_t)i + 1], p[3 * (int64_t)i + 2]);
+    }
+};
+struct Xyz4 {
+    const float4 *p;
+    __device__ __forceinline__ float3 operator()(int32_t i) const {
+        const float4 v = p[i];
+        return make_float3(v.x, v.y, v.z);
+    }
+};
+
+// One workgroup's part of the bounding box (as ordered ints) and of the sums.
+struct BoxPart {
+    int32_t mn[3], mx[3];
+    double sum[3], sq[3];
+};
+
+// Per-workgroup bounding boxes and sums of the finite coordinates (ATOMS: of
+// the atoms whose three coordinates are finite).  No atomics: 64 workgroups' on
+// six words took 21-29 us, these and the launch that joins them take 6 + 4.
+// Also clears the cell counts and two words.
+template <bool ATOMS, class SRC>
 __global__ void __launch_bounds__(nd::kBlock)
-k_prep_boxes(const float *__restrict__ xyz, int32_t n, int32_t *__restrict__ part, int32_t *__restrict__ cells,
-             int32_t ncells, int32_t *__restrict__ status, int32_t *__restrict__ maxcnt) {
-    __shared__ int32_t s[kWaves][6];
+k_prep_boxes(SRC xyz, int32_t n, BoxPart *__restrict__ part, int32_t *__restrict__ cells, int32_t ncells,
+             int32_t *__restrict__ status, int32_t *__restrict__ maxcnt) {
+    __shared__ BoxPart s[kWaves];
     const int32_t t = blockIdx.x * blockDim.x + threadIdx.x, stride = gridDim.x * blockDim.x;
     for (int32_t c = t; c < ncells; c += stride) cells[c] = 0;
     if (t == 0) {
@@ -491,45 +512,68 @@ k_prep_boxes(const float *__restrict__ xyz, int32_t n, int32_t *__restrict__ par
         *maxcnt = 0;
     }
     int32_t mn[3] = {INT32_MAX, INT32_MAX, INT32_MAX}, mx[3] = {INT32_MIN, INT32_MIN, INT32_MIN};
+    double sum[3] = {0.0, 0.0, 0.0}, sq[3] = {0.0, 0.0, 0.0};
     for (int32_t i = t; i < n; i += stride) {
-        const float v[3] = {xyz[3 * (int64_t)i], xyz[3 * (int64_t)i + 1], xyz[3 * (int64_t)i + 2]};
+        const float3 p = xyz(i);
+        const float v[3] = {p.x, p.y, p.z};
         const bool all = __builtin_isfinite(v[0]) & __builtin_isfinite(v[1]) & __builtin_isfinite(v[2]);
 #pragma unroll
         for (int d = 0; d < 3; ++d) {
             if (!(ATOMS ? all : __builtin_isfinite(v[d]))) continue;
             mn[d] = min(mn[d], f2ord(v[d]));
             mx[d] = max(mx[d], f2ord(v[d]));
+            sum[d] += (double)v[d];
+            sq[d] += (double)v[d] * (double)v[d];
         }
     }
+    const int w = threadIdx.x >> 6;
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
         mn[d] = wave_min(mn[d]);
         mx[d] = wave_max(mx[d]);
-    }
-    const int w = threadIdx.x >> 6;
-    if ((threadIdx.x & 63) == 0)
-#pragma unroll
-        for (int d = 0; d < 3; ++d) {
-            s[w][d] = mn[d];
-            s[w][3 + d] = mx[d];
+        for (int o = 32; o > 0; o >>= 1) {
+            sum[d] += __shfl_xor(sum[d], o, 64);
+            sq[d] += __shfl_xor(sq[d], o, 64);
         }
+        if ((threadIdx.x & 63) == 0) {
+            s[w].mn[d] = mn[d];
+            s[w].mx[d] = mx[d];
+            s[w].sum[d] = sum[d];
+            s[w].sq[d] = sq[d];
+        }
+    }
     __syncthreads();
-    if (threadIdx.x < 6) {
-        int32_t v = s[0][threadIdx.x];
-        for (int k = 1; k < kWaves; ++k) v = threadIdx.x < 3 ? min(v, s[k][threadIdx.x]) : max(v, s[k][threadIdx.x]);
-        part[6 * blockIdx.x + threadIdx.x] = v;
+    if (threadIdx.x < 3) {
+        const int d = threadIdx.x;
+        BoxPart &q = part[blockIdx.x];
+        for (int k = 1; k < kWaves; ++k) {
+            s[0].mn[d] = min(s[0].mn[d], s[k].mn[d]);
+            s[0].mx[d] = max(s[0].mx[d], s[k].mx[d]);
+            s[0].sum[d] += s[k].sum[d];
+            s[0].sq[d] += s[k].sq[d];
+        }
+        q.mn[d] = s[0].mn[d];
+        q.mx[d] = s[0].mx[d];
+        q.sum[d] = s[0].sum[d];
+        q.sq[d] = s[0].sq[d];
     }
 }
 
 // The joined box, for the host (thread d < 6: word d).
 __global__ void __launch_bounds__(64)
-k_box_result(const int32_t *__restrict__ part, int32_t nparts, int32_t *__restrict__ host) {
-    for (int d = 0; d < 6; ++d) {
-        int32_t v = d < 3 ? INT32_MAX : INT32_MIN;
-        for (int32_t t = threadIdx.x; t < nparts; t += 64)
-            v = d < 3 ? min(v, part[6 * t + d]) : max(v, part[6 * t + d]);
-        v = d < 3 ? wave_min(v) : wave_max(v);
-        if (threadIdx.x == 0) host[d] = v;
+k_box_result(const BoxPart *__restrict__ part, int32_t nparts, int32_t *__restrict__ host) {
+    for (int d = 0; d < 3; ++d) {
+        int32_t a = INT32_MAX, b = INT32_MIN;
+        for (int32_t t = threadIdx.x; t < nparts; t += 64) {
+            a = min(a, part[t].mn[d]);
+            b = max(b, part[t].mx[d]);
+        }
+        a = wave_min(a);
+        b = wave_max(b);
+        if (threadIdx.x == 0) {
+            host[d] = a;
+            host[3 + d] = b;
+        }
     }
 }
 
@@ -538,21 +582,39 @@ k_box_result(const int32_t *__restrict__ part, int32_t nparts, int32_t *__restri
 // walk's box test whatever its leaves' boxes are: coordinates within r less
 // two units in the last place of the largest coordinate +- r keep their order
 // after rounding x +- r/2 (or x +- r).
+//
+// The grid spans four standard deviations around the mean where that is less
+// than the bounding box: coordinates outside go to the edge cells, which keeps
+// atoms within a cell's side in neighbouring cells, and a few outliers do not
+// stretch the cells of all others.
 __global__ void __launch_bounds__(nd::kBlock)
-k_prep_grid(const int32_t *__restrict__ part, int32_t nparts, float r, float thr, int32_t max_cells,
+k_prep_grid(const BoxPart *__restrict__ part, int32_t nparts, int32_t n, float r, float thr, int32_t max_cells,
             float *__restrict__ box, Prep *__restrict__ prep) {
-    __shared__ int32_t s[kWaves][6];
-    int32_t v[6];
+    __shared__ BoxPart s[kWaves];
+    const int w = threadIdx.x >> 6;
 #pragma unroll
-    for (int d = 0; d < 6; ++d) {
-        v[d] = d < 3 ? INT32_MAX : INT32_MIN;
-        for (int32_t t = threadIdx.x; t < nparts; t += nd::kBlock)
-            v[d] = d < 3 ? min(v[d], part[6 * t + d]) : max(v[d], part[6 * t + d]);
-        v[d] = d < 3 ? wave_min(v[d]) : wave_max(v[d]);
+    for (int d = 0; d < 3; ++d) {
+        int32_t a = INT32_MAX, b = INT32_MIN;
+        double u = 0.0, v = 0.0;
+        for (int32_t t = threadIdx.x; t < nparts; t += nd::kBlock) {
+            a = min(a, part[t].mn[d]);
+            b = max(b, part[t].mx[d]);
+            u += part[t].sum[d];
+            v += part[t].sq[d];
+        }
+        a = wave_min(a);
+        b = wave_max(b);
+        for (int o = 32; o > 0; o >>= 1) {
+            u += __shfl_xor(u, o, 64);
+            v += __shfl_xor(v, o, 64);
+        }
+        if ((threadIdx.x & 63) == 0) {
+            s[w].mn[d] = a;
+            s[w].mx[d] = b;
+            s[w].sum[d] = u;
+            s[w].sq[d] = v;
+        }
     }
-    if ((threadIdx.x & 63) == 0)
-#pragma unroll
-        for (int d = 0; d < 6; ++d) s[threadIdx.x >> 6][d] = v[d];
     __syncthreads();
     if (threadIdx.x != 0) return;
     nd::CellGrid cg;
@@ -562,16 +624,22 @@ k_prep_grid(const int32_t *__restrict__ part, int32_t nparts, float r, float thr
     const double side = (double)r * (1.0 + 1e-4);
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
-        int32_t a = s[0][d], b = s[0][3 + d];
+        int32_t a = s[0].mn[d], b = s[0].mx[d];
+        double u = s[0].sum[d], v = s[0].sq[d];
         for (int k = 1; k < kWaves; ++k) {
-            a = min(a, s[k][d]);
-            b = max(b, s[k][3 + d]);
+            a = min(a, s[k].mn[d]);
+            b = max(b, s[k].mx[d]);
+            u += s[k].sum[d];
+            v += s[k].sq[d];
         }
         const float l = ord2f(a), h = ord2f(b), e = h - l;
-        box[d] = l;
-        box[3 + d] = e > 0.0f ? 1024.0f / e : 0.0f;
-        lo[d] = (double)l;
-        ext[d] = a <= b ? (double)h - (double)l : 0.0;
+        if (box) {
+            box[d] = l;
+            box[3 + d] = e > 0.0f ? 1024.0f / e : 0.0f;
+        }
+        const double mean = u / n, dev = 4.0 * sqrt(fmax(v / n - mean * mean, 0.0));
+        lo[d] = fmax((double)l, mean - dev);
+        ext[d] = a <= b ? fmin((double)h, mean + dev) - lo[d] : 0.0;
         const double q = ext[d] > 0.0 ? floor(ext[d] / side) : 1.0;
         g[d] = q >= 1.0 ? (q > 1024.0 ? 1024 : (int64_t)q) : 1;
         if (a <= b) most = fmaxf(most, fmaxf(fabsf(l), fabsf(h)));
@@ -596,6 +664,43 @@ k_prep_grid(const int32_t *__restrict__ part, int32_t nparts, float r, float thr
     prep->certain = in > 0.0 ? fminf((float)(in * in * (1.0 - 0x1p-20)), thr) : -1.0f;
 }
 
+// Counts an atom in cell c; returns its place among the cell's atoms.  A wave's
+// atoms of one cell are counted together while the cells are crowded (131,072
+// atoms of eight cells took 1 ms of atomics on their words); the first cell
+// that few lanes share ends that.
+__device__ __forceinline__ int32_t count_in_cell(int32_t *cells, int32_t c) {
+    const int lane = threadIdx.x & 63;
+    int32_t place = -1;
+    while (place < 0) {
+        const uint64_t same = __builtin_amdgcn_ballot_w64(c == __builtin_amdgcn_readfirstlane(c));
+        if (__builtin_popcountll(same) < 4) break;
+        if ((same >> lane) & 1ull) {
+            const int first = __builtin_ctzll(same);
+            int32_t b = 0;
+            if (lane == first) b = atomicAdd(&cells[c], __builtin_popcountll(same));
+            place = __builtin_amdgcn_readlane(b, first) + __builtin_popcountll(same & ((1ull << lane) - 1ull));
+        }
+    }
+    return place < 0 ? atomicAdd(&cells[c], 1) : place;
+}
+
+__device__ __forceinline__ int32_t cell_index(const nd::CellGrid &cg, float x, float y, float z) {
+    return (nd::cell_coord(cg, z, 2) * cg.g[1] + nd::cell_coord(cg, y, 1)) * cg.g[0] + nd::cell_coord(cg, x, 0);
+}
+
+// Cell and place of every atom.
+__global__ void __launch_bounds__(nd::kBlock)
+k_bin_atoms(const float4 *__restrict__ x, int32_t n, const Prep *__restrict__ prep, int32_t *__restrict__ cells,
+            int2 *__restrict__ cell_of, int32_t *__restrict__ status) {
+    const int32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    const float4 p = x[i];
+    if (!(__builtin_isfinite(p.x) && __builtin_isfinite(p.y) && __builtin_isfinite(p.z)))
+        atomicOr(status, nd::kStatusDomain);
+    const int32_t c = cell_index(prep->cg, p.x, p.y, p.z);
+    cell_of[i] = make_int2(c, count_in_cell(cells, c));
+}
+
 // Key and cell of every atom, and the atom's place among its cell's (by an
 // atomic count: in any order, the emitting pass sorts).  kb[2 b], kb[2 b + 1]:
 // or and and of workgroup b's keys.
@@ -618,25 +723,8 @@ k_prep_keys(const float *__restrict__ xyz, int32_t n, const float *__restrict__ 
         codes[i] = code;
         perm[i] = i;
         if (!ok) atomicOr(status, nd::kStatusDomain);
-        const nd::CellGrid &cg = prep->cg;
-        const int32_t c = (nd::cell_coord(cg, z, 2) * cg.g[1] + nd::cell_coord(cg, y, 1)) * cg.g[0] +
-                          nd::cell_coord(cg, x, 0);
-        // a wave's atoms of one cell are counted together while the cells are
-        // crowded (131,072 atoms of eight cells took 1 ms of atomics on their
-        // words); the first cell that few lanes share ends that
-        const int lane = threadIdx.x & 63;
-        int32_t place = -1;
-        while (place < 0) {
-            const uint64_t same = __builtin_amdgcn_ballot_w64(c == __builtin_amdgcn_readfirstlane(c));
-            if (__builtin_popcountll(same) < 4) break;
-            if ((same >> lane) & 1ull) {
-                const int first = __builtin_ctzll(same);
-                int32_t b = 0;
-                if (lane == first) b = atomicAdd(&cells[c], __builtin_popcountll(same));
-                place = __builtin_amdgcn_readlane(b, first) + __builtin_popcountll(same & ((1ull << lane) - 1ull));
-            }
-        }
-        if (place < 0) place = atomicAdd(&cells[c], 1);
+        const int32_t c = cell_index(prep->cg, x, y, z);
+        const int32_t place = count_in_cell(cells, c);
         cell_of[i] = make_int2(c, place);
         const uint32_t k = (uint32_t)code ^ 0x80000000u;
         atomicOr(&so, k);
@@ -728,6 +816,7 @@ k_cell_starts(int32_t *__restrict__ cells, int32_t n, const Prep *__restrict__ p
     }
     if (blockIdx.x != 0) return;
     if (t == 0) cells[ncell] = n;
+    if (host == nullptr) return;
     __shared__ uint32_t so, sa;
     __shared__ unsigned long long sq;
     if (t == 0) {
@@ -901,14 +990,43 @@ void launch_pair_emit(hipStream_t st, const PairSearch &S, const int64_t *offset
     ND_HIP(hipGetLastError());
 }
 
+namespace {
+// work words of launch_cell_bins
+struct BinWork {
+    BoxPart part[kBoxBlocks];
+    Prep prep;
+    uint64_t tsq[kMaxCells / kTileCells];
+    int32_t tsum[kMaxCells / kTileCells];
+    int32_t word;
+};
+}  // namespace
+
+size_t cell_bins_bytes() { return sizeof(BinWork); }
+
+const CellGrid *launch_cell_bins(hipStream_t st, void *work, const float4 *x, int32_t n, float r, int32_t max_cells,
+                                 int2 *cell_of, int32_t *cells, int32_t *status) {
+    BinWork *w = static_cast<BinWork *>(work);
+    if (max_cells > kMaxCells) max_cells = kMaxCells;
+    const int32_t tiles = (max_cells + kTileCells - 1) / kTileCells;
+    const unsigned g = grid_for(n), nb = std::min<unsigned>(g, kBoxBlocks);
+    k_prep_boxes<true><<<nb, kBlock, 0, st>>>(Xyz4{x}, n, w->part, cells, max_cells + 1, &w->word, &w->word);
+    k_prep_grid<<<1, kBlock, 0, st>>>(w->part, (int32_t)nb, n, r, 0.0f, max_cells, nullptr, &w->prep);
+    k_bin_atoms<<<g, kBlock, 0, st>>>(x, n, &w->prep, cells, cell_of, status);
+    k_cell_tiles<<<tiles, kBlock, 0, st>>>(cells, &w->prep, w->tsum, w->tsq);
+    k_cell_starts<<<tiles, kBlock, 0, st>>>(cells, n, &w->prep, w->tsum, w->tsq, nullptr, 0, nullptr, nullptr);
+    ND_HIP(hipGetLastError());
+    return &w->prep.cg;
+}
+
 bool atoms_box(nd_ctx *ctx, const float *d_xyz, int32_t n, double lo[3], double hi[3]) {
     hipStream_t st = ctx->stream;
-    ctx->prep.reserve(sizeof(int32_t) * 6 * kBoxBlocks);
-    int32_t *part = ctx->prep.as<int32_t>(), *status = ctx->status.as<int32_t>();
+    ctx->prep.reserve(sizeof(BoxPart) * kBoxBlocks);
+    BoxPart *part = ctx->prep.as<BoxPart>();
+    int32_t *status = ctx->status.as<int32_t>();
     struct Box { int32_t v[6]; };
     int32_t *hb = host_result<Box>(ctx)->v;
     const unsigned nb = std::min<unsigned>(grid_for(n), kBoxBlocks);
-    k_prep_boxes<true><<<nb, kBlock, 0, st>>>(d_xyz, n, part, nullptr, 0, status + 9, status + 10);
+    k_prep_boxes<true><<<nb, kBlock, 0, st>>>(Xyz3{d_xyz}, n, part, nullptr, 0, status + 9, status + 10);
     k_box_result<<<1, 64, 0, st>>>(part, (int32_t)nb, hb);
     ND_HIP(hipGetLastError());
     ND_HIP(hipStreamSynchronize(st));
@@ -958,11 +1076,11 @@ int64_t tree_list(nd_ctx *ctx, const float *d_xyz, int32_t kind, int32_t n, int3
     ctx->cell_vals.reserve(sizeof(int2) * (size_t)n);
     ctx->bbox.reserve(64);
     // work words: box parts, prep, tile sums, key bits
-    const size_t off_prep = sizeof(int32_t) * 6 * kBoxBlocks, off_sq = off_prep + 256,
+    const size_t off_prep = sizeof(BoxPart) * kBoxBlocks, off_sq = off_prep + 256,
                  off_sum = off_sq + sizeof(uint64_t) * (size_t)tiles, off_kb = off_sum + sizeof(int32_t) * (size_t)tiles;
     ctx->prep.reserve(off_kb + 8 * (size_t)g + 16);
     char *work = ctx->prep.as<char>();
-    int32_t *part = reinterpret_cast<int32_t *>(work);
+    BoxPart *part = reinterpret_cast<BoxPart *>(work);
     Prep *prep = reinterpret_cast<Prep *>(work + off_prep);
     static_assert(sizeof(Prep) <= 256, "prep block");
     uint64_t *tsq = reinterpret_cast<uint64_t *>(work + off_sq);
@@ -980,8 +1098,8 @@ int64_t tree_list(nd_ctx *ctx, const float *d_xyz, int32_t kind, int32_t n, int3
     const float thr = pred == ND_PRED_SCALAR ? r * r : root_threshold(r);
     const unsigned nb = std::min<unsigned>(g, kBoxBlocks);
     Prep *hp = host_result<Prep>(ctx);
-    k_prep_boxes<false><<<nb, kBlock, 0, st>>>(d_xyz, n, part, cells, max_cells + 1, status, maxcnt);
-    k_prep_grid<<<1, kBlock, 0, st>>>(part, (int32_t)nb, r, thr, max_cells, box, prep);
+    k_prep_boxes<false><<<nb, kBlock, 0, st>>>(Xyz3{d_xyz}, n, part, cells, max_cells + 1, status, maxcnt);
+    k_prep_grid<<<1, kBlock, 0, st>>>(part, (int32_t)nb, n, r, thr, max_cells, box, prep);
     if (morton == ND_MORTON_MASKED)
         k_prep_keys<true><<<g, kBlock, 0, st>>>(d_xyz, n, box, prep, codes, perm, cells, cell_of, kb, status);
     else

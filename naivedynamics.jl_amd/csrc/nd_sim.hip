@@ -1927,28 +1927,6 @@ __global__ void k_misc_reset_counters(SimMisc *misc) {
 
 }  // namespace
 
-namespace nd {
-
-void launch_list_walk(hipStream_t st, const nd_node *nodes, float4 *rec, const float4 *pos, int32_t n,
-                      int32_t nL, int32_t apl, float rlist, int32_t cap, int32_t *nbr, int32_t *ncount,
-                      int32_t *ctr) {
-    if (nL >= kMaxLeaves3) throw Error(ND_ERR_ARG, "list walk: too many leaves");
-    if (cap < 1 || cap > kMaxListRows) throw Error(ND_ERR_CAPACITY, "list walk: capacity out of range");
-    launch_lbvh_wide4(st, nodes, nL, rec);
-    const float hl = rlist / 2.0f, rl2 = rlist * rlist;
-    const unsigned g = grid_for(n);
-    switch (apl) {
-        case 4: k_nlist3<4><<<g, kBlock, 0, st>>>(pos, rec, n, nL, hl, rl2, cap, nbr, ncount, ctr); break;
-        case 8: k_nlist3<8><<<g, kBlock, 0, st>>>(pos, rec, n, nL, hl, rl2, cap, nbr, ncount, ctr); break;
-        case 16: k_nlist3<16><<<g, kBlock, 0, st>>>(pos, rec, n, nL, hl, rl2, cap, nbr, ncount, ctr); break;
-        case 32: k_nlist3<32><<<g, kBlock, 0, st>>>(pos, rec, n, nL, hl, rl2, cap, nbr, ncount, ctr); break;
-        default: throw Error(ND_ERR_ARG, "list walk: leaf size must be 4, 8, 16 or 32");
-    }
-    ND_HIP(hipGetLastError());
-}
-
-}  // namespace nd
-
 struct nd_sim {
     nd_ctx *ctx = nullptr;
     nd_sim_params p{};
