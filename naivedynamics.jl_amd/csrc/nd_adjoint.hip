@@ -34,8 +34,10 @@
 // reverse sweep the Hessian-vector product and the next step's lambda_h and a.
 // Per step of the forward pass (FP64, 32,768 atoms) the launches of a force
 // (21.8 us), kick (4.1) and kick-drift (3.0) kernel with four lanes per row
-// became one; per list build a key, sort, tree and walk of 21 launches and a
-// host synchronisation became seven launches and none.
+// became one (11.5), of a vector (4.9) and a Hessian-product (35.7) kernel one
+// (16.7); per list build a key, sort, tree and walk of 21 launches (250 us) and
+// a host synchronisation became seven launches (60 us) and none.  FP64 VALU
+// issue bounds both step kernels.
 //
 // Forces are summed in 2^-40 fixed point: the sum does not depend on the
 // order within a row or of the atoms, which the build leaves unspecified, so
@@ -75,14 +77,23 @@ __host__ __device__ inline double lj_G(double r, double eps, double sigma) {
     return 24.0 * eps * (24.0 * sr6 * sr6 - 6.0 * sr6) / (r * sigma);
 }
 
+// 1 / sqrt(x) in FP64 to its last place or so: the hardware's estimate (2^-23
+// or better) and one cubically converging step (Halley's).  A division and a
+// square root take some 25 instructions, this seven, and its square is 1 / x.
+__device__ __forceinline__ double rsqrt64(double x) {
+    const double y = __builtin_amdgcn_rsq(x);
+    const double e = fma(-(x * y), y, 1.0);
+    return fma(y * e, fma(e, 0.375, 0.5), y);
+}
+
 // s(r) of the forward force in precision T (LJ + Coulomb, both shifted).  FP64
-// takes one division and one square root per pair; FP32 keeps a division for
-// each quotient (its trajectories are held to their last bit).
+// takes one inverse square root per pair; FP32 keeps a division for each
+// quotient, whose rounding its trajectories follow.
 template <class T>
 __device__ __forceinline__ T pair_s(T r2, T qq, const AdjP &P) {
     T s = (T)0;
     if constexpr (sizeof(T) == 8) {
-        const T ir2 = 1.0 / r2, ir = sqrt(ir2);
+        const T ir = rsqrt64(r2), ir2 = ir * ir;
         if (r2 < P.rc2) {
             const T sr2 = P.sig2 * ir2, sr6 = sr2 * sr2 * sr2;
             const T F = (24.0 * P.eps) * (sr6 * sr6 + sr6 * sr6 - sr6) * ir;
@@ -111,7 +122,7 @@ struct PairD {
 };
 __device__ __forceinline__ PairD pair_d(double r2, double qi, double qj, const AdjP &P) {
     PairD o{0.0, 0.0, 0.0, 0.0, 0.0};
-    const double ir2 = 1.0 / r2, ir = sqrt(ir2), r = r2 * ir, ir3 = ir * ir2;
+    const double ir = rsqrt64(r2), ir2 = ir * ir, r = r2 * ir, ir3 = ir * ir2;
     if (r2 < P.rc2) {
         const double sr2 = P.sig2 * ir2, sr6 = sr2 * sr2 * sr2, sr12 = sr6 * sr6;
         const double F = 24.0 * P.eps * (2.0 * sr12 - sr6) * ir;
@@ -150,8 +161,10 @@ struct Rows {
     __device__ __forceinline__ int32_t count(int32_t s) const { return cnt[s] < cap ? cnt[s] : cap; }
 };
 
-// Lanes per row: lane t of an atom takes entries t, t + kRowLanes, ...
-constexpr int kRowLanes = 16;
+// Lanes per row: lane t of an atom takes entries t, t + kRowLanes, ...  (32,768
+// atoms, some 82 entries: 8 / 16 / 32 lanes take 16.7 / 18.2 / 21.9 us in the
+// reverse step and 11.5 / 11.6 / 13.9 in the forward one.)
+constexpr int kRowLanes = 8;
 
 // x, v of the caller's order and precision as records, and the FP32 positions
 // the list build bins.
@@ -239,28 +252,60 @@ k_adj_rows(const float4 *__restrict__ cpos, const int32_t *__restrict__ ckey, co
         const int32_t q1 = q0 + __builtin_popcountll(in);
         const int32_t c0 = k0 - row * g0, c1 = __builtin_amdgcn_readlane(pk, q1 - 1) - row * g0;
         const int32_t cy = row % g1, cz = row / g1;
-        for (int32_t z = max(cz - 1, 0); z <= min(cz + 1, g2 - 1); ++z)
-            for (int32_t y = max(cy - 1, 0); y <= min(cy + 1, g1 - 1); ++y) {
+        // lane j < 9: the run of cell row j around the group
+        int32_t from = 0, to = 0;
+        if (lane < 9) {
+            const int32_t y = cy + lane % 3 - 1, z = cz + lane / 3 - 1;
+            if (y >= 0 && y < g1 && z >= 0 && z < g2) {
                 const int32_t b = (z * g1 + y) * g0;
-                const int32_t u1 = cells[b + min(c1 + 1, g0 - 1) + 1];
-                for (int32_t u0 = cells[b + max(c0 - 1, 0)]; u0 < u1; u0 += 64) {
-                    const int32_t u = u0 + lane;
-                    const float4 c = cpos[min(u, u1 - 1)];
-                    for (int32_t q = q0; q < q1; ++q) {
-                        const float dx = c.x - lf(px, q), dy = c.y - lf(py, q), dz = c.z - lf(pz, q);
-                        const bool hit = (dx * dx + dy * dy + dz * dz < rl2) & (u < u1) & (u != t0 + q);
-                        const uint64_t m = __builtin_amdgcn_ballot_w64(hit);
-                        const int32_t have = __builtin_amdgcn_readlane(found, q);
-                        if (hit) {
-                            const int32_t at = (int32_t)__builtin_amdgcn_mbcnt_hi(
-                                (uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, (uint32_t)have));
-                            if (at < cap)
-                                lists[(int64_t)__builtin_amdgcn_readlane(pid, q) * cap + at] = __float_as_int(c.w);
-                        }
-                        found = lane == q ? have + __builtin_popcountll(m) : found;
-                    }
-                }
+                from = cells[b + max(c0 - 1, 0)];
+                to = cells[b + min(c1 + 1, g0 - 1) + 1];
             }
+        }
+        // the runs as one sequence; lane j: candidates before run j, and its
+        // start less those
+        int32_t pre = to - from;
+#pragma unroll
+        for (int o = 1; o < 16; o <<= 1) {
+            const int32_t v = __shfl_up(pre, o, 64);
+            if (lane >= o) pre += v;
+        }
+        const int32_t total = __builtin_amdgcn_readlane(pre, 8);
+        pre -= to - from;
+        const int32_t rise = from - pre;
+        int32_t at_run = 0;
+        auto fetch = [&](int32_t s0, int32_t &u) {
+            const int32_t ci = s0 + lane;
+            u = ci + __builtin_amdgcn_readlane(rise, at_run);
+            while (at_run < 8) {
+                const int32_t p = __builtin_amdgcn_readlane(pre, at_run + 1);
+                if (p > s0 + 63) break;
+                ++at_run;
+                u = ci >= p ? ci + __builtin_amdgcn_readlane(rise, at_run) : u;
+            }
+            if (ci >= total) u = -1;
+            return cpos[u < 0 ? t0 : u];
+        };
+        int32_t un;
+        float4 c = fetch(0, un);
+        for (int32_t s0 = 0; s0 < total; s0 += 64) {
+            // the next batch is on its way while this one is tested
+            const int32_t u = un;
+            const float4 d = c;
+            if (s0 + 64 < total) c = fetch(s0 + 64, un);
+            for (int32_t q = q0; q < q1; ++q) {
+                const float dx = d.x - lf(px, q), dy = d.y - lf(py, q), dz = d.z - lf(pz, q);
+                const bool hit = (dx * dx + dy * dy + dz * dz < rl2) & (u >= 0) & (u != t0 + q);
+                const uint64_t m = __builtin_amdgcn_ballot_w64(hit);
+                const int32_t have = __builtin_amdgcn_readlane(found, q);
+                if (hit) {
+                    const int32_t at = (int32_t)__builtin_amdgcn_mbcnt_hi(
+                        (uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, (uint32_t)have));
+                    if (at < cap) lists[(int64_t)__builtin_amdgcn_readlane(pid, q) * cap + at] = __float_as_int(d.w);
+                }
+                found = lane == q ? have + __builtin_popcountll(m) : found;
+            }
+        }
         q0 = q1;
     }
     if (lane < nt) cnt[pid] = found;
@@ -273,12 +318,15 @@ __device__ __forceinline__ double fix_val(unsigned long long v) { return (double
 
 // One launch of the forward model at x_k: F_i = sum_j s(r_ij) r_ij over row i,
 // summed in 2^-40 fixed point (the same whatever the order of the row and
-// however it is split); FINISH: the half kick that ends step k - 1; vck: the
-// velocity at k kept; DRIFT: the half kick and drift that begin step k.
-template <class T, bool FINISH, bool DRIFT>
+// however it is split); finish: the half kick that ends step k - 1; vck: the
+// velocity at k kept; xo: the half kick and drift that begin step k.
+// One instance serves every step (finish and a null xo are arguments): another
+// could contract its products differently, and the recompute has to repeat the
+// forward pass to the bit.
+template <class T>
 __global__ void __launch_bounds__(nd::kBlock)
 k_adj_step(Rows R, const typename V4<T>::R *__restrict__ x, const double *__restrict__ qs, AdjP P,
-           typename V4<T>::R *__restrict__ v, typename V4<T>::R *__restrict__ vck,
+           typename V4<T>::R *__restrict__ v, int32_t finish, typename V4<T>::R *__restrict__ vck,
            typename V4<T>::R *__restrict__ xo, float4 *__restrict__ x32) {
     using V = typename V4<T>::R;
     const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
@@ -315,13 +363,13 @@ k_adj_step(Rows R, const typename V4<T>::R *__restrict__ x, const double *__rest
     const T f[3] = {(T)fix_val((unsigned long long)fx), (T)fix_val((unsigned long long)fy),
                     (T)fix_val((unsigned long long)fz)};
     V w = v[s];
-    if (FINISH) {
+    if (finish) {
         w.x = w.x + (T)P.c * f[0];
         w.y = w.y + (T)P.c * f[1];
         w.z = w.z + (T)P.c * f[2];
     }
     if (vck) vck[s] = w;
-    if (DRIFT) {
+    if (xo) {
         w.x = w.x + (T)P.c * f[0];
         w.y = w.y + (T)P.c * f[1];
         w.z = w.z + (T)P.c * f[2];
@@ -703,9 +751,7 @@ void launch_step(nd_adj *s, int32_t w, const typename V4<T>::R *x, bool finish, 
     float4 *x32 = to_bins ? s->x32.as<float4>() : nullptr;
     const Rows R = rows_of(s, w);
     const double *qs = s->qs.as<double>();
-    if (finish && xo) k_adj_step<T, true, true><<<g, nd::kBlock, 0, st>>>(R, x, qs, s->P, v, vck, xo, x32);
-    else if (xo) k_adj_step<T, false, true><<<g, nd::kBlock, 0, st>>>(R, x, qs, s->P, v, vck, xo, x32);
-    else k_adj_step<T, true, false><<<g, nd::kBlock, 0, st>>>(R, x, qs, s->P, v, vck, nullptr, nullptr);
+    k_adj_step<T><<<g, nd::kBlock, 0, st>>>(R, x, qs, s->P, v, finish ? 1 : 0, vck, xo, x32);
     ND_HIP(hipGetLastError());
 }
 

@@ -1145,8 +1145,11 @@ int64_t tree_list(nd_ctx *ctx, const float *d_xyz, int32_t kind, int32_t n, int3
     // lies where a walk draws level: 131,072 points at density 0.8, 4 per leaf,
     // radius 6 (4,800 candidates and 318 pairs an atom): 3.63 ms by cells, 3.99
     // walking, point queries 3.04 and 4.80; 65,536 points, radius 8 (14,200):
-    // 4.14 and 3.78, point queries 10.3 and 7.3.
-    const bool by_cells = r >= 1e-15f && r <= 1e18f && (double)p.sum_sq * 27.0 <= 5500.0 * n && apl <= 64;
+    // 4.14 and 3.78, point queries 10.3 and 7.3.  Leaves of 64 atoms (a hit is
+    // placed in 63 other lists) draw level with a walk over a compact order:
+    // 131,072 points 1.25 ms and 1.23; 32 atoms 0.70 and 1.12.
+    const bool by_cells = r >= 1e-15f && r <= 1e18f && (double)p.sum_sq * 27.0 <= 5500.0 * n &&
+                          apl <= (!leaf || morton == ND_MORTON_MASKED ? 64 : 32);
     if (!by_cells) return walk();
     PairSearch S{};
     S.kind = kind;
