@@ -278,7 +278,7 @@ typedef struct {
                              comparison point; needs hi > lo) */
     int32_t pair_batch;   /* step kernel: neighbours per software-pipeline batch, 2, 4 or
                              8 (FP32; MIXED and FP64 use 4); 0 = 4 */
-    int32_t walk_front;   /* two-phase walk: tree records fetched per round trip, 8 or
+    int32_t walk_front;   /* two-phase walk over a tree (MIXED): records fetched per round trip, 8 or
                              16; 0 = 8 */
     int32_t atom_lanes;   /* step kernel: lanes per atom, 1 or 2 (two lanes split an
                              atom's list and add their sums in a fixed order); 0 = 1 */

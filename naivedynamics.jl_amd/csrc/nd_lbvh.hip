@@ -558,6 +558,21 @@ void launch_lbvh_refit_wide4(hipStream_t s, const float *xyz_sorted, int32_t xyz
     ND_HIP(hipGetLastError());
 }
 
+// Boxes of 64 consecutive boxes each (leaves' into chunks', chunks' likewise).
+void launch_chunk_boxes(hipStream_t s, const nd_node *boxes, int32_t count, float4 *chunks) {
+    const int64_t nchunks = (count + kChunk - 1) / kChunk;
+    k_lbvh_chunks<<<grid_for(nchunks * 64), kBlock, 0, s>>>(boxes, count, chunks);
+    ND_HIP(hipGetLastError());
+}
+
+void launch_leaf_chunk_boxes(hipStream_t s, const float *xyz, int32_t stride, int32_t n, float r, nd_node *leaves,
+                             float4 *chunks, float4 *tq, float4 *lc) {
+    constexpr int32_t kAtoms = 32 * kChunk;
+    k_leaf_chunk_boxes<32><<<(unsigned)((n + kAtoms - 1) / kAtoms), kBlock, 0, s>>>(xyz, stride, n, r / 2.0f, leaves,
+                                                                                 chunks, tq, lc);
+    ND_HIP(hipGetLastError());
+}
+
 void launch_lbvh_wide(hipStream_t s, const nd_node *nodes, int32_t nL, float4 *wide) {
     k_lbvh_wide<<<grid_for(nL - 1), kBlock, 0, s>>>(nodes, nL, wide);
     ND_HIP(hipGetLastError());

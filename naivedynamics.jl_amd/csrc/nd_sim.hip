@@ -1063,24 +1063,45 @@ k_nlist2(const float4 *__restrict__ pos, const float4 *__restrict__ wide, int32_
 
 using nd::wave_lds_sync;
 
-// Two-phase walk over four-wide records for leaves of A atoms (A = 4, 8, 16,
-// 32).  Every internal node has a record holding its grandchildren (a child
+// The list walk of the simulation: a wave of 64 consecutive atoms lists its
+// neighbours from the leaves (runs of A consecutive atoms) around it, in two
+// phases.  Phase 1 finds the leaves and queues each for every group of 8 lanes
+// (8 consecutive atoms) with a lane whose sphere of radius r_list meets the
+// leaf's box, together with the group's 8 overlap bits; it has two forms.
+//
+// Leaf form (TREE false; FP32 and FP64, A = 32 whatever the tree's leaf size
+// is).  The atoms lie along the sort key's curve, so 64 consecutive leaves (a
+// chunk) are a compact region, whose box is kept: the wave tests 64 chunks at a
+// time, a chunk per lane, against the box of its atoms, then the 64 leaves of
+// each chunk it meets, a leaf per lane; the leaves that pass (some 65 at liquid
+// density) are tested one after another, box in scalar registers, against
+// every lane's own sphere.  Two dependent fetches reach the leaves where the
+// tree takes one per two levels (eight round trips for 8,192 leaves, and 140
+// box tests a wave), and no tree is built or refitted.  Beyond kFlatChunks
+// chunks the boxes of 64 chunks each (supers) are tested first.  Leaves of 32
+// against 4, 8, 16 atoms: 32.6 us a step against 40.2, 35.4, 32.7 (262,144
+// atoms), 107 against 136, 113, 107 (4,096 atoms, a list every step).
+// 262,144 liquid atoms: walk and table 127.5 -> 98.6 us a list, and the refit of
+// the tree (7.7) gone; 4,096 atoms with a list every step: 192 -> 111 us a step.
+//
+// Tree form (TREE true; MIXED, A the tree's leaf size 4, 8, 16 or 32).  MIXED
+// sums runs of eight pairs in FP32, so its results follow the order of the
+// lists, which is the order of this walk.  Every internal node has a record holding its grandchildren (a child
 // that is a leaf stands for itself): up to 4 entries with boxes and node
 // numbers.  Phase 1 pops up to kFront records from the wave's LDS stack and
 // fetches them together (lane l loads float4 l & 7 of records (l >> 3) + 8 u),
 // so one memory latency covers up to kFront records (two tree levels each); every lane
-// tests its sphere of radius r_list against each entry's box, overlapped internal entries are pushed,
-// and an overlapped leaf is queued for each group of 8 lanes (8 consecutive
-// atoms) with an overlapping lane, together with the group's 8 overlap bits.
+// tests its sphere against each entry's box, overlapped internal entries are
+// pushed and overlapped leaves queued.
 // Phase 2 drains the 8 group queues side by side: per step each group stages
 // the atoms of its next leaf in its own LDS slot (the following leaf's load
 // already in flight) and each lane whose bit is set tests them, collecting
-// hits in a bit mask that it then appends.  A group of 8 Morton-consecutive
+// hits in a bit mask that it then appends.  A group of 8 curve-consecutive
 // atoms overlaps about as many leaves as its busiest lane, so the wave does
 // far fewer leaf steps than a walk that tests the whole wave against every
 // leaf any lane overlaps.  A lane gets exactly the neighbour set of its own
 // single-atom walk.
-// The stack never overflows for trees of depth <= 63 (any LBVH over 30-bit
+// The tree form's stack never overflows for trees of depth <= 63 (any LBVH over 30-bit
 // keys, i.e. <= 32 record levels): when fewer than kStackDfs free entries
 // remain the frontier shrinks to one record (plain depth-first order), which
 // adds at most 3 entries per record level.  Queue entries pack
@@ -1088,54 +1109,60 @@ using nd::wave_lds_sync;
 // kFront: records per phase-1 round trip (8, or 16 where the autotuner picks it)
 constexpr int kFront = 8, kStack2 = 256, kStackDfs = 128, kGroupQ = 128;
 constexpr int32_t kMaxLeaves3 = 1 << 23;
+constexpr int kWalkLeaf = 32;     // atoms per leaf of the leaf form
+constexpr int kLeafChunk = 64;    // leaves per chunk, chunks per super
+constexpr int kFlatChunks = 512;  // more chunks than this have supers
+
+// What phase 1 reads: the leaves' boxes (padded by h on each side) and the boxes
+// of 64 leaves and of 64 chunks (supers null where the chunks are few), or the
+// tree's four-wide records.
+struct WalkBoxes {
+    const nd_node *leaves;
+    const float4 *chunks, *supers, *wide;
+};
 
 // records per atom in the walk's record buffer: cap rounded up to 8
 __host__ __device__ __forceinline__ int32_t rec_stride(int32_t cap) { return (cap + 7) & ~7; }
 
-// REC: instead of list rows, each atom gets one record per leaf it has
-// neighbours in, (group g, mask): its neighbours there are the sorted indices
-// 32 g + b for the set bits b of the mask (leaves of A <= 32 atoms start at
-// multiples of A, so a leaf lies in one 32-atom group).  Records of an atom
-// are contiguous (recs[i * rec_stride(cap) + k], k < nrecs[i]; blocks of 64 B
-// multiples, so a reader fetches two records per 16-byte load); each holds
-// at least one neighbour, so there are never more records than list entries.
+// Each atom gets one record per 32-atom group it has neighbours in, (group g,
+// mask): its neighbours there are the sorted indices 32 g + b for the set bits
+// b of the mask (leaves of A <= 32 atoms start at multiples of A, so a leaf
+// lies in one group).  Records of an atom are contiguous
+// (recs[i * rec_stride(cap) + k], k < nrecs[i]; blocks of 64 B multiples, so a
+// reader fetches two records per 16-byte load); each holds at least one
+// neighbour, so there are never more records than list entries.
 // LDS of the walk: per wave a staging buffer (8 group slots of A atoms, or
 // F fetched records), a node stack and 8 group queues with dummy slots.
-template <int A, int F> struct Walk3Lds {
+template <int A, int F, bool TREE> struct Walk3Lds {
     static constexpr int kSlot = 4 * A + 4;  // floats per group slot (16 B pad: no bank conflicts)
-    static constexpr int kBufF = 8 * kSlot > 32 * F ? 8 * kSlot : 32 * F;  // records: 8 float4 each
+    static constexpr int kRec = TREE ? 32 * F : 0;  // records: 8 float4 each
+    static constexpr int kBufF = 8 * kSlot > kRec ? 8 * kSlot : kRec;
     static constexpr int kW = nd::kBlock / 64;
     __align__(16) float buf[kW][kBufF];
-    int32_t stk[kW][kStack2];
+    int32_t stk[TREE ? kW : 1][TREE ? kStack2 : 1];
     int32_t q[kW][8 * kGroupQ + 64];
 };
 
-template <int A, bool REC, int F, bool LOCAL = false>
+template <int A, int F, bool TREE, bool LOCAL>
 __device__ __forceinline__ void
-walk3_body(const float4 *__restrict__ pos, const float4 *__restrict__ wide, int32_t n, int32_t nL, float h,
-           float rl2, int32_t cap, int32_t *__restrict__ nbr, int32_t *__restrict__ ncount,
-           int32_t *__restrict__ ctr, uint2 *__restrict__ recs, int32_t *__restrict__ nrecs,
-           Walk3Lds<A, F> &L, int32_t blk, int32_t *__restrict__ work,
+walk3_body(const float4 *__restrict__ pos, const WalkBoxes B, int32_t n, int32_t nL, float h, float rl2, int32_t cap,
+           int32_t *__restrict__ ncount, int32_t *__restrict__ ctr, uint2 *__restrict__ recs,
+           int32_t *__restrict__ nrecs, Walk3Lds<A, F, TREE> &L, int32_t blk, int32_t *__restrict__ work,
            const float4 *__restrict__ tq = nullptr, const float4 *__restrict__ lc = nullptr) {
     static_assert(A == 4 || A == 8 || A == 16 || A == 32, "leaf size");
     constexpr int NV = (A + 7) / 8;      // atoms a lane stages per leaf (1, 2 or 4)
-    constexpr int kSlot = Walk3Lds<A, F>::kSlot;
+    constexpr int kSlot = Walk3Lds<A, F, TREE>::kSlot;
     const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int grp = lane >> 3, gl = lane & 7;
     float *buf = L.buf[w];
     float4 *rec = reinterpret_cast<float4 *>(buf);
-    int32_t *stk = L.stk[w], *gq = L.q[w];
+    int32_t *stk = L.stk[TREE ? w : 0], *gq = L.q[w];  // the stack: tree form
 
     const int32_t i = blk * nd::kBlock + threadIdx.x;
     const bool active = i < n;
-    // this wave's block of the list as a buffer resource: a row at or past cap
-    // lies outside it, and the hardware drops such a store (no branch per hit)
-    const __amdgpu_buffer_rsrc_t lrs = __builtin_amdgcn_make_buffer_rsrc(
-        (void *)(nbr + (int64_t)__builtin_amdgcn_readfirstlane(i >> 6) * cap * 64), 0, cap * 256, kBufWord3);
-    uint32_t voff = (uint32_t)lane * 4u;  // byte offset of row cnt in this lane's column
-    int32_t rcnt = 0, nrec = 0;           // REC: list entries and records so far
-    uint32_t pend_g = ~0u, pend_b = 0u;    // REC: the record being built (leaves of one group merge)
-    uint2 *myrec = recs + (REC ? (int64_t)i * rec_stride(cap) : 0);
+    int32_t rcnt = 0, nrec = 0;           // list entries and records so far
+    uint32_t pend_g = ~0u, pend_b = 0u;    // the record being built (leaves of one group merge)
+    uint2 *myrec = recs + (int64_t)i * rec_stride(cap);
     const float4 p = active ? pos[i] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     // A lane overlaps a node when its sphere of radius r_list meets the
     // node's atoms' box (the stored box less the padding h = r_list / 2 on
@@ -1147,7 +1174,7 @@ walk3_body(const float4 *__restrict__ pos, const float4 *__restrict__ wide, int3
     // lanes without an atom overlap nothing.
     const float slack = (fmaxf(fmaxf(fabsf(p.x), fabsf(p.y)), fabsf(p.z)) + 4.0f * h) * 0x1p-20f;
     const float hc = h - slack, rlb2 = rl2 * (1.0f + 0x1p-20f);
-    bool bad = false;
+    bool bad = false;  // tree form: a malformed tree
 
     int32_t glen = 0;  // lanes 0..7: length of queue `lane`
     int32_t nqu = 0;   // leaves queued since the last drain (bounds every glen)
@@ -1160,190 +1187,281 @@ walk3_body(const float4 *__restrict__ pos, const float4 *__restrict__ wide, int3
         ++nqu;
     };
 
-    int32_t sp = 1, fetched = 0;
-    int32_t rounds = 0, leaf_steps = 0;  // wave-uniform work counters (phase 1, phase 2)
-    stk[0] = nL + 1;  // the root is internal (nL >= 2)
-    wave_lds_sync();
-    while (sp > 0 || nqu > 0) {
-        if (nqu > 0 && (sp == 0 || nqu > kGroupQ - 4 * F)) {
-            // ---- phase 2: drain the group queues ----
-            const int32_t len = __shfl(glen, grp, 64);
-            int32_t steps = len;
-            for (int off = 32; off > 0; off >>= 1) steps = max(steps, __shfl_xor(steps, off, 64));
-            steps = __builtin_amdgcn_readfirstlane(steps);
-            leaf_steps += steps;
-            float *slot = buf + grp * kSlot;
-            // atom gl + 8 r of the group's leaf k; lanes past the leaf size load atom 0
-            // (named registers, not an array: the loads stay in flight across the step)
-            // LOCAL: the leaf-local copies (-2 q', |q'|^2) and the leaf's
-            // (centre, R^2), loaded with the atoms
-            const float4 *src = (LOCAL ? tq : pos) + (gl < A ? gl : 0);
-            const float4 zero = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-            float4 v0 = zero, v1 = zero, v2 = zero, v3 = zero, cn = zero;
-            auto load4 = [&](int32_t e) {
-                const float4 *lp = src + ((e >> 8) - 1) * A;
-                v0 = lp[0];
-                if constexpr (NV > 1) v1 = lp[8];
-                if constexpr (NV > 2) { v2 = lp[16]; v3 = lp[24]; }
-                if constexpr (LOCAL) cn = lc[(e >> 8) - 1];
+    int32_t rounds = 0, tests = 0, leaf_steps = 0;  // wave-uniform work counters (phases 1 and 2)
+
+    auto drain = [&]() {
+        // ---- phase 2: drain the group queues ----
+        const int32_t len = __shfl(glen, grp, 64);
+        int32_t steps = len;
+        for (int off = 32; off > 0; off >>= 1) steps = max(steps, __shfl_xor(steps, off, 64));
+        steps = __builtin_amdgcn_readfirstlane(steps);
+        leaf_steps += steps;
+        float *slot = buf + grp * kSlot;
+        // atom gl + 8 r of the group's leaf k; lanes past the leaf size load atom 0
+        // (named registers, not an array: the loads stay in flight across the step)
+        // LOCAL: the leaf-local copies (-2 q', |q'|^2) and the leaf's
+        // (centre, R^2), loaded with the atoms
+        // (leaf form: the last leaf may hold fewer than A; its missing atoms
+        // are masked out of the hits, tq and pos have room for a leaf more)
+        const float4 *src = (LOCAL ? tq : pos) + (gl < A ? gl : 0);
+        const float4 zero = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        float4 v0 = zero, v1 = zero, v2 = zero, v3 = zero, cn = zero;
+        auto load4 = [&](int32_t e) {
+            const float4 *lp = src + ((e >> 8) - 1) * A;
+            v0 = lp[0];
+            if constexpr (NV > 1) v1 = lp[8];
+            if constexpr (NV > 2) { v2 = lp[16]; v3 = lp[24]; }
+            if constexpr (LOCAL) cn = lc[(e >> 8) - 1];
+        };
+        if (len > 0) load4(gq[grp * kGroupQ]);
+        for (int32_t k = 0; k < steps; ++k) {
+            wave_lds_sync();  // the previous step's reads are done
+            if (k < len && gl < A) {
+                float4 *dst = reinterpret_cast<float4 *>(slot) + gl;
+                dst[0] = v0;
+                if constexpr (NV > 1) dst[8] = v1;
+                if constexpr (NV > 2) { dst[16] = v2; dst[24] = v3; }
+            }
+            wave_lds_sync();
+            const float4 cc = cn;  // the staged leaf's centre and R^2 (LOCAL)
+            const int32_t e = k < len ? gq[grp * kGroupQ + k] : 0;
+            if (k + 1 < len) load4(gq[grp * kGroupQ + k + 1]);
+            uint32_t hits = 0u;
+            const int32_t base = ((e >> 8) - 1) * A;
+            // the list's pair test: |p - q|^2 < rl2, in this order of operations
+            auto exact = [&](const float4 &q) -> bool {
+                const float dx = p.x - q.x, dy = p.y - q.y, dz = p.z - q.z;
+                const float s = dx * dx + dy * dy + dz * dz;
+                return s < rl2;
             };
-            if (len > 0) load4(gq[grp * kGroupQ]);
-            for (int32_t k = 0; k < steps; ++k) {
-                wave_lds_sync();  // the previous step's reads are done
-                if (k < len && gl < A) {
-                    float4 *dst = reinterpret_cast<float4 *>(slot) + gl;
-                    dst[0] = v0;
-                    if constexpr (NV > 1) dst[8] = v1;
-                    if constexpr (NV > 2) { dst[16] = v2; dst[24] = v3; }
+            if ((e >> gl) & 1) {
+                if constexpr (LOCAL) {
+                    // |p - q|^2 - rl2 = |a|^2 - rl2 + (-2 q').a + |q'|^2 with a = p - c:
+                    // three FMAs per atom against the staged copy.  Its distance
+                    // from the exact test's value is below 16 u (|a| + R + r)^2
+                    // (u = 2^-24: the roundings of a, q', |q'|^2, the FMAs and
+                    // of the exact test itself), which E bounds from above
+                    // (3 (x^2 + y^2 + z^2) >= (x + y + z)^2); a wave with any
+                    // test within E of the radius redoes the leaf exactly from
+                    // the positions, so the list is the exact test's.
+                    const float ax = p.x - cc.x, ay = p.y - cc.y, az = p.z - cc.z;
+                    const float cp = __builtin_fmaf(az, az, __builtin_fmaf(ay, ay, __builtin_fmaf(ax, ax, -rl2)));
+                    const float E = 48.0f * 0x1p-24f * (cp + 2.0f * rl2 + cc.w);
+                    uint64_t band = 0;
+#pragma unroll
+                    for (int m = A - 1; m >= 0; --m) {
+                        const float4 q = *reinterpret_cast<const float4 *>(slot + 4 * m);
+                        const float t =
+                            __builtin_fmaf(ax, q.x, __builtin_fmaf(ay, q.y, __builtin_fmaf(az, q.z, q.w))) + cp;
+                        // t's sign bit (a zero t is within E: the exact test decides),
+                        // shifted in below the bits of atoms m + 1 .. A - 1 by one
+                        // funnel shift, so atom m ends at bit m
+                        hits = __builtin_amdgcn_alignbit(hits, __float_as_uint(t), 31);
+                        band |= __builtin_amdgcn_ballot_w64(fabsf(t) < E);
+                    }
+                    if (band != 0) {  // rare: a test within E of the radius
+                        hits = 0u;
+#pragma unroll 1
+                        for (int m = 0; m < A; ++m) hits |= (exact(pos[TREE ? base + m : min(base + m, n - 1)]) ? 1u : 0u) << m;
+                    }
+                } else {
+#pragma unroll
+                    for (int m = 0; m < A; ++m)
+                        hits |= (exact(*reinterpret_cast<const float4 *>(slot + 4 * m)) ? 1u : 0u) << m;
+                }
+                if (!TREE && n - base < A) hits &= (1u << (n - base)) - 1u;
+                const uint32_t self = (uint32_t)(i - base);
+                if (self < (uint32_t)A) hits &= ~(1u << self);
+                if (hits) {
+                    const uint32_t g = (uint32_t)(base >> 5), b = hits << (base & 31);
+                    if (g == pend_g) {
+                        pend_b |= b;
+                    } else {
+                        if (pend_g != ~0u) {
+                            if (nrec < cap) myrec[nrec] = make_uint2(pend_g, pend_b);
+                            ++nrec;
+                        }
+                        pend_g = g;
+                        pend_b = b;
+                    }
+                    rcnt += __popc(hits);
+                }
+            }
+        }
+        glen = 0;
+        nqu = 0;
+        wave_lds_sync();
+    };
+
+    if constexpr (TREE) {
+        int32_t sp = 1, fetched = 0;
+        stk[0] = nL + 1;  // the root is internal (nL >= 2)
+        wave_lds_sync();
+        while (sp > 0 || nqu > 0) {
+            if (nqu > 0 && (sp == 0 || nqu > kGroupQ - 4 * F)) {
+                drain();
+                continue;
+            }
+            // ---- phase 1: expand up to F records of the stack top ----
+            ++rounds;
+            // (each record pushes at most 4 entries: k pops leave room for them)
+            const int32_t room = (kStack2 - kStackDfs - sp) / 3;
+            int32_t k = sp < F ? sp : F;
+            if (k > room) k = room > 1 ? room : 1;
+            fetched += k;
+            // more records than the tree has internal nodes, or a stack that could overflow
+            if (fetched > nL || sp + 3 * k > kStack2) { bad = true; break; }
+            sp -= k;
+            {
+                // lane l loads float4 l & 7 of records (l >> 3) + 8 u, u < F / 8
+                float4 v[F / 8];
+#pragma unroll
+                for (int u = 0; u < F / 8; ++u) {
+                    const int32_t slot = (lane >> 3) + 8 * u;
+                    v[u] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+                    if (slot < k) v[u] = B.wide[8 * (int64_t)(stk[sp + slot] - nL - 1) + (lane & 7)];
                 }
                 wave_lds_sync();
-                const float4 cc = cn;  // the staged leaf's centre and R^2 (LOCAL)
-                const int32_t e = k < len ? gq[grp * kGroupQ + k] : 0;
-                if (k + 1 < len) load4(gq[grp * kGroupQ + k + 1]);
-                uint32_t hits = 0u;
-                const int32_t base = ((e >> 8) - 1) * A;
-                // the list's pair test: |p - q|^2 < rl2, in this order of operations
-                auto exact = [&](const float4 &q) -> bool {
-                    const float dx = p.x - q.x, dy = p.y - q.y, dz = p.z - q.z;
-                    const float s = dx * dx + dy * dy + dz * dz;
-                    return s < rl2;
-                };
-                if ((e >> gl) & 1) {
-                    if constexpr (LOCAL) {
-                        // |p - q|^2 - rl2 = |a|^2 - rl2 + (-2 q').a + |q'|^2 with a = p - c:
-                        // three FMAs per atom against the staged copy.  Its distance
-                        // from the exact test's value is below 16 u (|a| + R + r)^2
-                        // (u = 2^-24: the roundings of a, q', |q'|^2, the FMAs and
-                        // of the exact test itself), which E bounds from above
-                        // (3 (x^2 + y^2 + z^2) >= (x + y + z)^2); a wave with any
-                        // test within E of the radius redoes the leaf exactly from
-                        // the positions, so the list is the exact test's.
-                        const float ax = p.x - cc.x, ay = p.y - cc.y, az = p.z - cc.z;
-                        const float cp = __builtin_fmaf(az, az, __builtin_fmaf(ay, ay, __builtin_fmaf(ax, ax, -rl2)));
-                        const float E = 48.0f * 0x1p-24f * (cp + 2.0f * rl2 + cc.w);
-                        uint64_t band = 0;
 #pragma unroll
-                        for (int m = A - 1; m >= 0; --m) {
-                            const float4 q = *reinterpret_cast<const float4 *>(slot + 4 * m);
-                            const float t =
-                                __builtin_fmaf(ax, q.x, __builtin_fmaf(ay, q.y, __builtin_fmaf(az, q.z, q.w))) + cp;
-                            // t's sign bit (a zero t is within E: the exact test decides),
-                            // shifted in below the bits of atoms m + 1 .. A - 1 by one
-                            // funnel shift, so atom m ends at bit m
-                            hits = __builtin_amdgcn_alignbit(hits, __float_as_uint(t), 31);
-                            band |= __builtin_amdgcn_ballot_w64(fabsf(t) < E);
-                        }
-                        if (band != 0) {  // rare: a test within E of the radius
-                            hits = 0u;
-#pragma unroll 1
-                            for (int m = 0; m < A; ++m) hits |= (exact(pos[base + m]) ? 1u : 0u) << m;
-                        }
-                    } else {
+                for (int u = 0; u < F / 8; ++u) rec[lane + 64 * u] = v[u];
+                wave_lds_sync();
+            }
+            const uint32_t nn = (uint32_t)(2 * nL - 1);  // valid node numbers are 1 .. 2 nL - 1
+            auto entry = [&](float mnx, float mny, float mnz, float mxx, float mxy, float mxz, float idf) {
+                const int32_t c = __builtin_amdgcn_readfirstlane(__float_as_int(idf));
+                if (c == 0) return;
+                if ((uint32_t)(c - 1) >= nn) { bad = true; return; }
+                const float ex = fmaxf(fmaxf(mnx - p.x, p.x - mxx), -hc) + hc;
+                const float ey = fmaxf(fmaxf(mny - p.y, p.y - mxy), -hc) + hc;
+                const float ez = fmaxf(fmaxf(mnz - p.z, p.z - mxz), -hc) + hc;
+                const bool ov = active & (ex * ex + ey * ey + ez * ez < rlb2);
+                const uint64_t mk = __builtin_amdgcn_ballot_w64(ov);
+                if (mk) {
+                    if (c <= nL) enqueue(c, mk);
+                    else stk[sp++] = c;
+                }
+            };
+            for (int32_t r = 0; r < k; ++r) {
+                const float4 mnx = rec[8 * r], mny = rec[8 * r + 1], mnz = rec[8 * r + 2];
+                const float4 mxx = rec[8 * r + 3], mxy = rec[8 * r + 4], mxz = rec[8 * r + 5];
+                const float4 ids = rec[8 * r + 6];
+                // an internal node has two children, so a record has >= 2 entries
+                if (__builtin_amdgcn_readfirstlane(__float_as_int(ids.y)) == 0) { bad = true; break; }
+                entry(mnx.x, mny.x, mnz.x, mxx.x, mxy.x, mxz.x, ids.x);
+                entry(mnx.y, mny.y, mnz.y, mxx.y, mxy.y, mxz.y, ids.y);
+                entry(mnx.z, mny.z, mnz.z, mxx.z, mxy.z, mxz.z, ids.z);
+                entry(mnx.w, mny.w, mnz.w, mxx.w, mxy.w, mxz.w, ids.w);
+                if (bad) break;
+            }
+            if (bad) break;
+            wave_lds_sync();
+        }
+        if (bad && lane == 0) atomicOr(&ctr[2], nd::kStatusTree);
+    } else {
+        // The wave's box and largest slack: the same distance from box to box.
+        // Rounded differences, maxima and sums of squares keep their order, so it
+        // is no larger than any lane's, for a leaf or for a chunk around it.
+        const float inf = __int_as_float(0x7F800000);
+        float wlx = active ? p.x : inf, wly = active ? p.y : inf, wlz = active ? p.z : inf;
+        float whx = active ? p.x : -inf, why = active ? p.y : -inf, whz = active ? p.z : -inf;
+        float wsl = active ? slack : 0.0f;
 #pragma unroll
-                        for (int m = 0; m < A; ++m)
-                            hits |= (exact(*reinterpret_cast<const float4 *>(slot + 4 * m)) ? 1u : 0u) << m;
-                    }
-                    const uint32_t self = (uint32_t)(i - base);
-                    if (self < (uint32_t)A) hits &= ~(1u << self);
-                    if constexpr (REC) {
-                        if (hits) {
-                            const uint32_t g = (uint32_t)(base >> 5), b = hits << (base & 31);
-                            if (g == pend_g) {
-                                pend_b |= b;
-                            } else {
-                                if (pend_g != ~0u) {
-                                    if (nrec < cap) myrec[nrec] = make_uint2(pend_g, pend_b);
-                                    ++nrec;
-                                }
-                                pend_g = g;
-                                pend_b = b;
-                            }
-                            rcnt += __popc(hits);
+        for (int off = 32; off > 0; off >>= 1) {
+            wlx = fminf(wlx, __shfl_xor(wlx, off, 64));
+            wly = fminf(wly, __shfl_xor(wly, off, 64));
+            wlz = fminf(wlz, __shfl_xor(wlz, off, 64));
+            whx = fmaxf(whx, __shfl_xor(whx, off, 64));
+            why = fmaxf(why, __shfl_xor(why, off, 64));
+            whz = fmaxf(whz, __shfl_xor(whz, off, 64));
+            wsl = fmaxf(wsl, __shfl_xor(wsl, off, 64));
+        }
+        const float whc = h - wsl, rlw2 = rlb2 * (1.0f + 0x1p-20f);
+        // whether the wave's box comes near a stored box (min xyz, max x | max y, max z, ..)
+        auto near = [&](const float4 &a, const float4 &b) -> bool {
+            const float ex = fmaxf(fmaxf(a.x - whx, wlx - a.w), -whc) + whc;
+            const float ey = fmaxf(fmaxf(a.y - why, wly - b.x), -whc) + whc;
+            const float ez = fmaxf(fmaxf(a.z - whz, wlz - b.y), -whc) + whc;
+            return !(ex * ex + ey * ey + ez * ez >= rlw2);
+        };
+        // which of the 64 boxes from `first` on (count in all) the wave comes near
+        auto near64 = [&](const float4 *boxes, int32_t first, int32_t count) -> uint64_t {
+            const int32_t k = first + lane;
+            bool ov = false;
+            if (k < count) ov = near(boxes[2 * (int64_t)k], boxes[2 * (int64_t)k + 1]);
+            return __builtin_amdgcn_ballot_w64(ov);
+        };
+        const int32_t nC = (nL + kLeafChunk - 1) / kLeafChunk, nS = (nC + kLeafChunk - 1) / kLeafChunk;
+        int32_t sbase = -kLeafChunk;          // first super of the batch in smask
+        int32_t cbase = 0, lbase = 0;         // first chunk of cmask, first leaf of lmask
+        uint64_t smask = 0, cmask = 0, lmask = 0;  // supers, chunks and leaves still to look at
+        bool more = true;
+        while (more) {
+            // ---- phase 1: queue leaves until a queue may be full or none are left ----
+            while (nqu < kGroupQ) {
+                if (lmask == 0) {
+                    while (cmask == 0) {
+                        while (smask == 0) {
+                            sbase += kLeafChunk;
+                            if (sbase >= nS) break;
+                            smask = B.supers ? near64(B.supers, sbase, nS)
+                                           : (nS - sbase >= 64 ? ~0ull : (1ull << (nS - sbase)) - 1ull);
                         }
-                    } else {
-                        while (hits) {
-                            const int32_t m = __builtin_ctz(hits);
-                            hits &= hits - 1u;
-                            __builtin_amdgcn_raw_buffer_store_b32(base + m, lrs, voff, 0, 0);
-                            voff += 256u;
-                        }
+                        if (smask == 0) break;
+                        cbase = (sbase + __builtin_ctzll(smask)) * kLeafChunk;
+                        smask &= smask - 1ull;
+                        cmask = near64(B.chunks, cbase, nC);
                     }
+                    if (cmask == 0) {
+                        more = false;
+                        break;
+                    }
+                    lbase = (cbase + __builtin_ctzll(cmask)) * kLeafChunk;
+                    cmask &= cmask - 1ull;
+                    lmask = ~0ull;
+                    ++rounds;
+                }
+                // this chunk's leaf boxes, one per lane (again after a drain)
+                float4 a = make_float4(inf, inf, inf, -inf), b = make_float4(-inf, -inf, 0.0f, 0.0f);
+                if (lbase + lane < nL) {
+                    const float4 *q = reinterpret_cast<const float4 *>(B.leaves + lbase + lane);
+                    a = q[0];
+                    b = q[1];
+                }
+                lmask &= __builtin_amdgcn_ballot_w64(lbase + lane < nL && near(a, b));
+                while (lmask != 0 && nqu < kGroupQ) {
+                    const int32_t l = __builtin_ctzll(lmask);
+                    lmask &= lmask - 1ull;
+                    ++tests;
+                    auto box = [&](float v) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l)); };
+                    const float mnx = box(a.x), mny = box(a.y), mnz = box(a.z);
+                    const float mxx = box(a.w), mxy = box(b.x), mxz = box(b.y);
+                    const float ex = fmaxf(fmaxf(mnx - p.x, p.x - mxx), -hc) + hc;
+                    const float ey = fmaxf(fmaxf(mny - p.y, p.y - mxy), -hc) + hc;
+                    const float ez = fmaxf(fmaxf(mnz - p.z, p.z - mxz), -hc) + hc;
+                    const uint64_t mk = __builtin_amdgcn_ballot_w64(active & (ex * ex + ey * ey + ez * ez < rlb2));
+                    if (mk) enqueue(lbase + l + 1, mk);
                 }
             }
-            glen = 0;
-            nqu = 0;
+            if (nqu == 0) break;
             wave_lds_sync();
-            continue;
+            drain();
         }
-        // ---- phase 1: expand up to F records of the stack top ----
-        ++rounds;
-        // (each record pushes at most 4 entries: k pops leave room for them)
-        const int32_t room = (kStack2 - kStackDfs - sp) / 3;
-        int32_t k = sp < F ? sp : F;
-        if (k > room) k = room > 1 ? room : 1;
-        fetched += k;
-        // more records than the tree has internal nodes, or a stack that could overflow
-        if (fetched > nL || sp + 3 * k > kStack2) { bad = true; break; }
-        sp -= k;
-        {
-            // lane l loads float4 l & 7 of records (l >> 3) + 8 u, u < F / 8
-            float4 v[F / 8];
-#pragma unroll
-            for (int u = 0; u < F / 8; ++u) {
-                const int32_t slot = (lane >> 3) + 8 * u;
-                v[u] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-                if (slot < k) v[u] = wide[8 * (int64_t)(stk[sp + slot] - nL - 1) + (lane & 7)];
-            }
-            wave_lds_sync();
-#pragma unroll
-            for (int u = 0; u < F / 8; ++u) rec[lane + 64 * u] = v[u];
-            wave_lds_sync();
-        }
-        const uint32_t nn = (uint32_t)(2 * nL - 1);  // valid node numbers are 1 .. 2 nL - 1
-        auto entry = [&](float mnx, float mny, float mnz, float mxx, float mxy, float mxz, float idf) {
-            const int32_t c = __builtin_amdgcn_readfirstlane(__float_as_int(idf));
-            if (c == 0) return;
-            if ((uint32_t)(c - 1) >= nn) { bad = true; return; }
-            const float ex = fmaxf(fmaxf(mnx - p.x, p.x - mxx), -hc) + hc;
-            const float ey = fmaxf(fmaxf(mny - p.y, p.y - mxy), -hc) + hc;
-            const float ez = fmaxf(fmaxf(mnz - p.z, p.z - mxz), -hc) + hc;
-            const bool ov = active & (ex * ex + ey * ey + ez * ez < rlb2);
-            const uint64_t mk = __builtin_amdgcn_ballot_w64(ov);
-            if (mk) {
-                if (c <= nL) enqueue(c, mk);
-                else stk[sp++] = c;
-            }
-        };
-        for (int32_t r = 0; r < k; ++r) {
-            const float4 mnx = rec[8 * r], mny = rec[8 * r + 1], mnz = rec[8 * r + 2];
-            const float4 mxx = rec[8 * r + 3], mxy = rec[8 * r + 4], mxz = rec[8 * r + 5];
-            const float4 ids = rec[8 * r + 6];
-            // an internal node has two children, so a record has >= 2 entries
-            if (__builtin_amdgcn_readfirstlane(__float_as_int(ids.y)) == 0) { bad = true; break; }
-            entry(mnx.x, mny.x, mnz.x, mxx.x, mxy.x, mxz.x, ids.x);
-            entry(mnx.y, mny.y, mnz.y, mxx.y, mxy.y, mxz.y, ids.y);
-            entry(mnx.z, mny.z, mnz.z, mxx.z, mxy.z, mxz.z, ids.z);
-            entry(mnx.w, mny.w, mnz.w, mxx.w, mxy.w, mxz.w, ids.w);
-            if (bad) break;
-        }
-        if (bad) break;
-        wave_lds_sync();
     }
-    if (bad && lane == 0) atomicOr(&ctr[2], nd::kStatusTree);
-    // the wave's work estimate for the next walk's block placement: a CU's
-    // walk time follows its waves' leaf steps and round trips (~0.12 and
-    // ~0.28 us each when four workgroups share the CU)
-    if (work != nullptr && lane == 0) work[4 * blk + w] = 5 * leaf_steps + 12 * rounds;
-    if (REC && pend_g != ~0u) {
+    // the wave's work estimate for the next walk's block placement.  Tree: a
+    // CU's walk time follows its waves' leaf steps and round trips (~0.12 and
+    // ~0.28 us each when four workgroups share the CU).  Leaf form: some 230
+    // vector instructions a leaf step, 32 a leaf's box test, 100 a chunk.
+    if (work != nullptr && lane == 0)
+        work[4 * blk + w] = TREE ? 5 * leaf_steps + 12 * rounds : 7 * leaf_steps + tests + 3 * rounds;
+    if (pend_g != ~0u) {
         if (nrec < cap) myrec[nrec] = make_uint2(pend_g, pend_b);
         ++nrec;
     }
-    const int32_t cnt = REC ? rcnt : (int32_t)((voff - (uint32_t)lane * 4u) >> 8);
     if (active) {
-        ncount[i] = cnt;
-        if constexpr (REC) nrecs[i] = nrec;
+        ncount[i] = rcnt;
+        nrecs[i] = nrec;
     }
-    int32_t m = cnt;
+    int32_t m = rcnt;
     for (int off = 32; off > 0; off >>= 1) m = max(m, __shfl_down(m, off, 64));
     if (lane == 0 && m > 0) {
         // the counter only grows: skip the (serialising) atomic when it is
@@ -1353,15 +1471,16 @@ walk3_body(const float4 *__restrict__ pos, const float4 *__restrict__ wide, int3
     }
 }
 
-template <int A, bool REC = false, int F = kFront, bool LOCAL = false>
+// The walk alone (dense workloads: the table build's larger record buffer
+// would lower a joint kernel's occupancy).
+template <int A, int F, bool TREE>
 __global__ void __launch_bounds__(nd::kBlock)
-k_nlist3(const float4 *__restrict__ pos, const float4 *__restrict__ wide, int32_t n, int32_t nL,
-         float h, float rl2, int32_t cap, int32_t *__restrict__ nbr, int32_t *__restrict__ ncount,
-         int32_t *__restrict__ ctr, uint2 *__restrict__ recs = nullptr, int32_t *__restrict__ nrecs = nullptr,
-         const float4 *__restrict__ tq = nullptr, const float4 *__restrict__ lc = nullptr) {
-    __shared__ Walk3Lds<A, F> L;
-    walk3_body<A, REC, F, LOCAL>(pos, wide, n, nL, h, rl2, cap, nbr, ncount, ctr, recs, nrecs, L,
-                                 xcd_block(blockIdx.x, gridDim.x), nullptr, tq, lc);
+k_nlist3(const float4 *__restrict__ pos, WalkBoxes B, int32_t n, int32_t nL, float h, float rl2, int32_t cap,
+         int32_t *__restrict__ ncount, int32_t *__restrict__ ctr, uint2 *__restrict__ recs,
+         int32_t *__restrict__ nrecs) {
+    __shared__ Walk3Lds<A, F, TREE> L;
+    walk3_body<A, F, TREE, false>(pos, B, n, nL, h, rl2, cap, ncount, ctr, recs, nrecs, L,
+                                  xcd_block(blockIdx.x, gridDim.x), nullptr);
 }
 
 // ---- neighbourhood tables ----
@@ -1570,7 +1689,7 @@ k_table(const int32_t *__restrict__ nbr, const int32_t *__restrict__ ncount, int
     }
 }
 
-// Tables from the two-phase walk's records (k_nlist3<A, true>): a record per
+// Tables from the two-phase walk's records (walk3_body): a record per
 // (atom, leaf with neighbours), ~9 per atom at density 0.8, instead of a list
 // entry per neighbour (~76), so the walk writes and this kernel reads ~4x
 // fewer bytes.  While the records go into the hash they are copied to LDS
@@ -1812,23 +1931,21 @@ k_table_rec(const uint2 *__restrict__ recs, const int32_t *__restrict__ nrecs,
 // All workgroups of a launch are resident at once (four per CU), so the
 // kernel ends with its busiest CU; the order gives every CU of an XCD a
 // similar total.  Any permutation gives the same lists and tables.
-template <int A, int F>
+template <int A, int F, bool TREE>
 __global__ void __launch_bounds__(nd::kBlock, 4)  // four waves per SIMD: all 4 workgroups per CU resident
-k_walk_table(const float4 *__restrict__ pos, const float4 *__restrict__ wide, int32_t n, int32_t nL, float h,
-             float rl2, int32_t cap, int32_t *__restrict__ nbr, int32_t *__restrict__ ncount,
+k_walk_table(const float4 *__restrict__ pos, WalkBoxes B, int32_t n, int32_t nL, float h, float rl2, int32_t cap, int32_t *__restrict__ nbr, int32_t *__restrict__ ncount,
              int32_t *__restrict__ ctr, uint2 *__restrict__ recs, int32_t *__restrict__ nrecs, int32_t cap2,
              int32_t lcap, int32_t eshift, uint32_t *__restrict__ nbr16, int32_t *__restrict__ tables,
              int32_t *__restrict__ tcount, SimMisc *__restrict__ misc, volatile int32_t *hstale,
              uint32_t *__restrict__ slot_info, const int32_t *__restrict__ order, int32_t *__restrict__ work,
              const float4 *__restrict__ tq, const float4 *__restrict__ lc) {
     union Lds {
-        Walk3Lds<A, F> walk;
+        Walk3Lds<A, F, TREE> walk;
         TableRecLds<kRecLds> table;
     };
     __shared__ Lds L;
     const int32_t blk = __builtin_amdgcn_readfirstlane(order[xcd_block(blockIdx.x, gridDim.x)]);
-    walk3_body<A, true, F, true>(pos, wide, n, nL, h, rl2, cap, nbr, ncount, ctr, recs, nrecs, L.walk, blk, work,
-                                 tq, lc);
+    walk3_body<A, F, TREE, true>(pos, B, n, nL, h, rl2, cap, ncount, ctr, recs, nrecs, L.walk, blk, work, tq, lc);
     __syncthreads();  // every wave's walk is done with the LDS
     table_rec_body<kRecLds>(recs, nrecs, ncount, n, cap, cap2, lcap, eshift, nbr16, tables, tcount, nbr, misc,
                             hstale, slot_info, L.table, blk);
@@ -1932,7 +2049,7 @@ struct nd_sim {
     nd_sim_params p{};
     int32_t n = 0, nL = 0, apl = 0;
     bool wide = false;  // FP64 storage (MIXED, FP64)
-    nd::DevBuf pos[2], vel[2], frc, orig[2], pos32, fix[2], codes, perm, nodes, store, kids, nbr,
+    nd::DevBuf pos[2], vel[2], frc, orig[2], pos32, fix[2], codes, perm, nodes, store, kids, leaf_chunks, nbr,
         ncount, misc, partials, rows, snap_pos, snap_vel, snap_frc, snap_orig, rep, boxes;
     nd::DevBuf wsnap_pos, wsnap_vel, wsnap_orig;  // start of a window in a checked rerun
     nd::DevBuf cpos, cstart;  // cell-list walk: cell-sorted positions, cell starts
@@ -1948,7 +2065,7 @@ struct nd_sim {
     nd::DevBuf recs, nrecs;   // the two-phase walk's (group, mask) records per atom
     int32_t lcap = 0;         // table capacity (records) per workgroup
     int32_t pair_batch = kPairBatch;  // step kernel: neighbours per pipeline batch (FP32)
-    int32_t walk_front = kFront;      // two-phase walk: records per phase-1 round trip
+    int32_t walk_front = kFront;      // two-phase walk's tree form: records per phase-1 round trip
     int32_t atom_lanes = 1;           // step kernel: lanes per atom (1 or 2)
     nd::CellGrid cg{};
     int32_t nrep = 0;  // packed replicas (0: one system)
@@ -2013,7 +2130,7 @@ template <class F>
 void for_each_buf(nd_sim *s, F &&f) {
     nd::DevBuf *bufs[] = {&s->pos[0], &s->pos[1], &s->vel[0], &s->vel[1], &s->frc, &s->orig[0],
                           &s->orig[1], &s->pos32, &s->fix[0], &s->fix[1], &s->codes, &s->perm, &s->nodes,
-                          &s->store, &s->kids, &s->rep, &s->boxes, &s->nbr, &s->ncount, &s->misc,
+                          &s->store, &s->kids, &s->leaf_chunks, &s->rep, &s->boxes, &s->nbr, &s->ncount, &s->misc,
                           &s->partials, &s->rows, &s->snap_pos, &s->snap_vel, &s->snap_frc, &s->snap_orig,
                           &s->sort.keys_alt, &s->sort.vals_alt, &s->sort.hist, &s->sort.flags, &s->cpos,
                           &s->cstart, &s->path, &s->nbr16, &s->tables, &s->tcount, &s->slot_info, &s->recs, &s->nrecs,
@@ -2097,12 +2214,22 @@ int32_t resort_period(const nd_sim *s) {
     return s->p.resort_every > 0 ? s->p.resort_every : s->p.rebuild_every;
 }
 
-// The two-phase walk (records of four-wide nodes, leaf-local copies) runs
-// the simulation's list when asked for and the leaf size and count allow it.
-bool two_phase_walk(const nd_sim *s) {
-    return s->p.list_walk == 0 && s->nL < kMaxLeaves3 &&
+// Leaves of the leaf form of the two-phase walk, and boxes of 64 each.
+int32_t walk_leaves(const nd_sim *s) { return (int32_t)(((int64_t)s->n + kWalkLeaf - 1) / kWalkLeaf); }
+int32_t chunk_count(int32_t boxes) { return (boxes + kLeafChunk - 1) / kLeafChunk; }
+
+// The two-phase walk makes the simulation's list when asked for and the leaves
+// can be counted: its leaf form, which needs no tree and takes any leaf size,
+// or for MIXED, whose FP32 partial sums depend on the order of the lists, its
+// tree form, where the leaf size allows it.
+bool leaf_walk(const nd_sim *s) {
+    return s->p.list_walk == 0 && s->p.precision != ND_PREC_MIXED && walk_leaves(s) < kMaxLeaves3;
+}
+bool tree_walk(const nd_sim *s) {
+    return s->p.list_walk == 0 && s->p.precision == ND_PREC_MIXED && s->nL < kMaxLeaves3 &&
            (s->apl == 4 || s->apl == 8 || s->apl == 16 || s->apl == 32);
 }
+bool two_phase_walk(const nd_sim *s) { return leaf_walk(s) || tree_walk(s); }
 
 // A rebuild at step k re-sorts (new keys, order and topology) when the
 // period says so or when no tree matches the current order.
@@ -2163,7 +2290,10 @@ void launch_rebuild(nd_sim *s, bool full) {
             k_pos32<<<g, nd::kBlock, 0, st>>>(s->pos[s->cur].as<double4>(), n, s->pos32.as<float4>());
         const float *p32 = s->wide ? reinterpret_cast<const float *>(s->pos32.p)
                                    : reinterpret_cast<const float *>(s->pos[s->cur].p);
-        if (two_phase) {
+        if (leaf_walk(s)) {
+            nd::launch_leaf_chunk_boxes(st, p32, 4, n, s->rlist, s->nodes.as<nd_node>(), s->leaf_chunks.as<float4>(),
+                                        s->leaf_q.as<float4>(), s->leaf_c.as<float4>());
+        } else if (two_phase) {
             nd::launch_lbvh_refit_wide4(st, p32, 4, s->nL, s->apl, s->rlist, s->nodes.as<nd_node>(),
                                         s->store.as<int32_t>(), s->kids.as<float4>(), s->leaf_q.as<float4>(),
                                         s->leaf_c.as<float4>());
@@ -2188,8 +2318,21 @@ void launch_rebuild(nd_sim *s, bool full) {
         }
     } else {
         float4 *kids = s->kids.as<float4>();
-        if (two_phase) {
+        WalkBoxes B{};
+        const bool tree = tree_walk(s);
+        const int32_t leaves = tree ? s->nL : walk_leaves(s);
+        if (tree) {
             if (!records_done) nd::launch_lbvh_wide4(st, s->nodes.as<nd_node>(), s->nL, kids);
+            B.wide = kids;
+        } else if (two_phase) {
+            const int32_t nC = chunk_count(leaves);
+            float4 *ch = s->leaf_chunks.as<float4>();  // the chunks' boxes, then the supers'
+            B.leaves = s->nodes.as<nd_node>();
+            B.chunks = ch;
+            if (nC > kFlatChunks) {
+                B.supers = ch + 2 * (int64_t)nC;
+                nd::launch_chunk_boxes(st, reinterpret_cast<const nd_node *>(ch), nC, ch + 2 * (int64_t)nC);
+            }
         } else {
             nd::launch_lbvh_wide(st, s->nodes.as<nd_node>(), s->nL, kids);
         }
@@ -2207,22 +2350,24 @@ void launch_rebuild(nd_sim *s, bool full) {
                 // walk and table build in one kernel
                 const int32_t *ord = s->walk_order.as<int32_t>();
                 int32_t *wk = s->walk_work.as<int32_t>();
-#define ND_WALKTAB(A, F)                                                                                  \
-    k_walk_table<A, F><<<g, nd::kBlock, 0, st>>>(p4, kids, n, s->nL, hl, rl2, s->cap, nb, nc, ctr, rc, nr, c2, \
-                                                 s->lcap, es, n16, tb, tc, misc, s->hstale, si, ord, wk, tql, lcl)
-                if (s->walk_front == 16) {
+#define ND_WALKTAB(A, F, TREE)                                                                                   \
+    k_walk_table<A, F, TREE><<<g, nd::kBlock, 0, st>>>(p4, B, n, leaves, hl, rl2, s->cap, nb, nc, ctr, rc, nr, c2, \
+                                                       s->lcap, es, n16, tb, tc, misc, s->hstale, si, ord, wk, tql, lcl)
+                if (!tree) {
+                    ND_WALKTAB(kWalkLeaf, kFront, false);
+                } else if (s->walk_front == 16) {
                     switch (s->apl) {
-                        case 4: ND_WALKTAB(4, 16); break;
-                        case 8: ND_WALKTAB(8, 16); break;
-                        case 16: ND_WALKTAB(16, 16); break;
-                        default: ND_WALKTAB(32, 16); break;
+                        case 4: ND_WALKTAB(4, 16, true); break;
+                        case 8: ND_WALKTAB(8, 16, true); break;
+                        case 16: ND_WALKTAB(16, 16, true); break;
+                        default: ND_WALKTAB(32, 16, true); break;
                     }
                 } else {
                     switch (s->apl) {
-                        case 4: ND_WALKTAB(4, 8); break;
-                        case 8: ND_WALKTAB(8, 8); break;
-                        case 16: ND_WALKTAB(16, 8); break;
-                        default: ND_WALKTAB(32, 8); break;
+                        case 4: ND_WALKTAB(4, 8, true); break;
+                        case 8: ND_WALKTAB(8, 8, true); break;
+                        case 16: ND_WALKTAB(16, 8, true); break;
+                        default: ND_WALKTAB(32, 8, true); break;
                     }
                 }
 #undef ND_WALKTAB
@@ -2232,20 +2377,23 @@ void launch_rebuild(nd_sim *s, bool full) {
             }
             // dense workloads: the walk, then the table build with the larger
             // record buffer (its LDS would lower the walk's occupancy)
-#define ND_NLIST3(A, F) k_nlist3<A, true, F><<<g, nd::kBlock, 0, st>>>(p4, kids, n, s->nL, hl, rl2, s->cap, nb, nc, ctr, rc, nr)
-            if (s->walk_front == 16) {
+#define ND_NLIST3(A, F, TREE) \
+    k_nlist3<A, F, TREE><<<g, nd::kBlock, 0, st>>>(p4, B, n, leaves, hl, rl2, s->cap, nc, ctr, rc, nr)
+            if (!tree) {
+                ND_NLIST3(kWalkLeaf, kFront, false);
+            } else if (s->walk_front == 16) {
                 switch (s->apl) {
-                    case 4: ND_NLIST3(4, 16); break;
-                    case 8: ND_NLIST3(8, 16); break;
-                    case 16: ND_NLIST3(16, 16); break;
-                    default: ND_NLIST3(32, 16); break;
+                    case 4: ND_NLIST3(4, 16, true); break;
+                    case 8: ND_NLIST3(8, 16, true); break;
+                    case 16: ND_NLIST3(16, 16, true); break;
+                    default: ND_NLIST3(32, 16, true); break;
                 }
             } else {
                 switch (s->apl) {
-                    case 4: ND_NLIST3(4, 8); break;
-                    case 8: ND_NLIST3(8, 8); break;
-                    case 16: ND_NLIST3(16, 8); break;
-                    default: ND_NLIST3(32, 8); break;
+                    case 4: ND_NLIST3(4, 8, true); break;
+                    case 8: ND_NLIST3(8, 8, true); break;
+                    case 16: ND_NLIST3(16, 8, true); break;
+                    default: ND_NLIST3(32, 8, true); break;
                 }
             }
 #undef ND_NLIST3
@@ -2282,20 +2430,23 @@ void launch_sort_and_build(nd_sim *s) {
     // the walk, and take two radix passes instead of three; the tree is built
     // on the same truncated keys.  The masked key keeps its 30 bits.
     const int32_t key_bits = (s->p.morton_mode != ND_MORTON_MASKED && n <= (1 << 20)) ? 20 : 30;
+    const bool leaves_only = leaf_walk(s);  // no tree
+    const int32_t slots = leaves_only ? 0 : s->nL - 1;  // the tree build's, cleared with the keys
     if (s->wide)
         k_sim_keys<double><<<g, nd::kBlock, 0, st>>>(s->pos[s->cur].as<double4>(), n, s->p.morton_mode,
                                                      lo, scale, 30 - key_bits, codes, perm, misc,
-                                                     s->store.as<int32_t>(), s->nL - 1);
+                                                     s->store.as<int32_t>(), slots);
     else
         k_sim_keys<float><<<g, nd::kBlock, 0, st>>>(s->pos[s->cur].as<float4>(), n, s->p.morton_mode,
                                                     lo, scale, 30 - key_bits, codes, perm, misc,
-                                                    s->store.as<int32_t>(), s->nL - 1);
+                                                    s->store.as<int32_t>(), slots);
     // keys are < 2^key_bits, so the sign-flipped key's higher bits are constant
     nd::radix_sort_keys10(st, s->sort, codes, perm, n, key_bits, &codes, &perm);
     const int a = s->cur ^ 1, va = s->vcur ^ 1;
     // leaf boxes in the permutation for power-of-two leaves up to 64 (the
     // cell walk needs no tree, so none there)
-    const bool boxes = s->p.list_walk != 3 && s->apl <= 64 && (s->apl & (s->apl - 1)) == 0;
+    const int32_t per_leaf = leaves_only ? kWalkLeaf : s->apl;
+    const bool boxes = s->p.list_walk != 3 && per_leaf <= 64 && (per_leaf & (per_leaf - 1)) == 0;
     // the two-phase walk's leaf-local copies, written with the leaf boxes
     float4 *lq = two_phase_walk(s) ? s->leaf_q.as<float4>() : nullptr;
     float4 *lcn = two_phase_walk(s) ? s->leaf_c.as<float4>() : nullptr;
@@ -2308,7 +2459,7 @@ void launch_sort_and_build(nd_sim *s) {
         s->wide ? s->pos32.as<float4>() : nullptr, s->wide ? fix_ptr(s, a) : nullptr, s->sp, misc, h, nodes, \
         lq, lcn)
 #define ND_PERMUTE_SEG(PT)                                        \
-    switch (boxes ? s->apl : 0) {                                \
+    switch (boxes ? per_leaf : 0) {                                \
         case 1: ND_PERMUTE(PT, 1); break;                         \
         case 2: ND_PERMUTE(PT, 2); break;                         \
         case 4: ND_PERMUTE(PT, 4); break;                         \
@@ -2329,6 +2480,10 @@ void launch_sort_and_build(nd_sim *s) {
     s->vcur = va;
     if (s->p.list_walk == 3) {  // the cell list needs no tree
         ND_HIP(hipGetLastError());
+        return;
+    }
+    if (leaves_only) {  // the leaves' boxes (the permutation's) and their chunks'
+        nd::launch_chunk_boxes(st, nodes, walk_leaves(s), s->leaf_chunks.as<float4>());
         return;
     }
     const float *p32 = s->wide ? reinterpret_cast<const float *>(s->pos32.p)
@@ -2856,19 +3011,25 @@ int nd_sim_create(nd_ctx *ctx, const nd_sim_params *p, nd_sim **out) {
         s->rlist = (float)(rl + (span + rl) * 9.5367431640625e-07);
         const size_t pb = pos_bytes(s), n = (size_t)s->n;
         for (int b = 0; b < 2; ++b) {
-            s->pos[b].reserve(pb);
+            s->pos[b].reserve(pb + sizeof(float4) * kWalkLeaf);  // the walk reads whole leaves
             s->vel[b].reserve(pb);
             s->orig[b].reserve(sizeof(int32_t) * n);
         }
         s->frc.reserve(pb);
-        if (s->wide) s->pos32.reserve(sizeof(float4) * n);
+        if (s->wide) s->pos32.reserve(sizeof(float4) * (n + kWalkLeaf));
         if (p->precision == ND_PREC_MIXED)
             for (int b = 0; b < 2; ++b) s->fix[b].reserve(sizeof(int4) * n);
         s->codes.reserve(sizeof(int32_t) * n);
         s->perm.reserve(sizeof(int32_t) * n);
-        s->nodes.reserve(sizeof(nd_node) * (size_t)(2 * s->nL - 1));
-        s->store.reserve(sizeof(int32_t) * nd::lbvh_scratch_ints(s->nL));
-        s->kids.reserve(8 * sizeof(float4) * (size_t)(s->nL - 1));  // four-wide records
+        if (leaf_walk(s)) {
+            const int32_t nC = chunk_count(walk_leaves(s));
+            s->nodes.reserve(sizeof(nd_node) * (size_t)walk_leaves(s));  // the leaves' boxes
+            s->leaf_chunks.reserve(2 * sizeof(float4) * ((size_t)nC + (size_t)chunk_count(nC)));
+        } else {
+            s->nodes.reserve(sizeof(nd_node) * (size_t)(2 * s->nL - 1));
+            s->store.reserve(sizeof(int32_t) * nd::lbvh_scratch_ints(s->nL));
+            s->kids.reserve(8 * sizeof(float4) * (size_t)(s->nL - 1));  // four-wide records
+        }
         s->ncount.reserve(sizeof(int32_t) * n);
         s->path.reserve(sizeof(uint16_t) * n);
         s->nrecs.reserve(sizeof(int32_t) * n);
@@ -2900,8 +3061,8 @@ int nd_sim_create(nd_ctx *ctx, const nd_sim_params *p, nd_sim **out) {
             for (int32_t b = 0; b < nb; ++b) iota[b] = b;
             s->walk_order.reserve(sizeof(int32_t) * (size_t)nb);
             s->walk_work.reserve(sizeof(int32_t) * 4 * (size_t)nb);
-            s->leaf_q.reserve(sizeof(float4) * (size_t)s->n);
-            s->leaf_c.reserve(sizeof(float4) * (size_t)(s->nL > 0 ? s->nL : 1));
+            s->leaf_q.reserve(sizeof(float4) * ((size_t)s->n + kWalkLeaf));
+            s->leaf_c.reserve(sizeof(float4) * (size_t)std::max(s->nL, walk_leaves(s)));
             ND_HIP(hipMemcpyAsync(s->walk_order.p, iota.data(), sizeof(int32_t) * (size_t)nb,
                                   hipMemcpyHostToDevice, ctx->stream));
             ND_HIP(hipMemsetAsync(s->walk_work.p, 0, sizeof(int32_t) * 4 * (size_t)nb, ctx->stream));
