@@ -146,9 +146,9 @@ void launch_lbvh_refit_wide4(hipStream_t s, const float *xyz_sorted, int32_t xyz
 // Boxes (2 float4 each: min xyz, max x | max y, max z, 0, 0) of every 64
 // consecutive boxes of the same layout.
 void launch_chunk_boxes(hipStream_t s, const nd_node *boxes, int32_t count, float4 *chunks);
-// Without a tree: boxes (+- r/2) of leaves of 32 atoms (the last may hold
+// Without a tree: boxes (+- r/2) of leaves of 16 or 32 atoms (the last may hold
 // fewer), of every 64 leaves, and the leaf-local copies as above.
-void launch_leaf_chunk_boxes(hipStream_t s, const float *xyz, int32_t stride, int32_t n, float r, nd_node *leaves,
+void launch_leaf_chunk_boxes(hipStream_t s, const float *xyz, int32_t stride, int32_t n, int32_t apl, float r, nd_node *leaves,
                              float4 *chunks, float4 *tq, float4 *lc);
 // slots_cleared: the caller has already zeroed store[0 .. nL-2] (the CAS slots);
 // leaves_done: the caller has already written the leaf boxes (+- r/2).

@@ -565,11 +565,11 @@ void launch_chunk_boxes(hipStream_t s, const nd_node *boxes, int32_t count, floa
     ND_HIP(hipGetLastError());
 }
 
-void launch_leaf_chunk_boxes(hipStream_t s, const float *xyz, int32_t stride, int32_t n, float r, nd_node *leaves,
+void launch_leaf_chunk_boxes(hipStream_t s, const float *xyz, int32_t stride, int32_t n, int32_t apl, float r, nd_node *leaves,
                              float4 *chunks, float4 *tq, float4 *lc) {
-    constexpr int32_t kAtoms = 32 * kChunk;
-    k_leaf_chunk_boxes<32><<<(unsigned)((n + kAtoms - 1) / kAtoms), kBlock, 0, s>>>(xyz, stride, n, r / 2.0f, leaves,
-                                                                                 chunks, tq, lc);
+    const unsigned g = (unsigned)(((int64_t)n + apl * kChunk - 1) / (apl * kChunk));
+    if (apl == 16) k_leaf_chunk_boxes<16><<<g, kBlock, 0, s>>>(xyz, stride, n, r / 2.0f, leaves, chunks, tq, lc);
+    else k_leaf_chunk_boxes<32><<<g, kBlock, 0, s>>>(xyz, stride, n, r / 2.0f, leaves, chunks, tq, lc);
     ND_HIP(hipGetLastError());
 }
 

@@ -1109,7 +1109,9 @@ using nd::wave_lds_sync;
 // kFront: records per phase-1 round trip (8, or 16 where the autotuner picks it)
 constexpr int kFront = 8, kStack2 = 256, kStackDfs = 128, kGroupQ = 128;
 constexpr int32_t kMaxLeaves3 = 1 << 23;
-constexpr int kWalkLeaf = 32;     // atoms per leaf of the leaf form
+constexpr int kWalkLeaf = 32;     // atoms per leaf of the leaf form,
+constexpr int kSplitLeaf = 16;    // and where kSplit waves share each 64 atoms
+constexpr int kSplit = 4;
 constexpr int kLeafChunk = 64;    // leaves per chunk, chunks per super
 constexpr int kFlatChunks = 512;  // more chunks than this have supers
 
@@ -1131,34 +1133,51 @@ __host__ __device__ __forceinline__ int32_t rec_stride(int32_t cap) { return (ca
 // (recs[i * rec_stride(cap) + k], k < nrecs[i]; blocks of 64 B multiples, so a
 // reader fetches two records per 16-byte load); each holds at least one
 // neighbour, so there are never more records than list entries.
+// The largest list length of a wave's lanes into ctr[0] (ctr[1]: over cap).
+__device__ __forceinline__ void count_max(int32_t count, int32_t cap, int32_t *__restrict__ ctr) {
+    int32_t m = count;
+    for (int off = 32; off > 0; off >>= 1) m = max(m, __shfl_down(m, off, 64));
+    if ((threadIdx.x & 63) == 0 && m > 0) {
+        // the counter only grows: skip the (serialising) atomic when it is
+        // already at least m
+        if (m > __hip_atomic_load(&ctr[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(&ctr[0], m);
+        if (m > cap) atomicOr(&ctr[1], 1);
+    }
+}
+
 // LDS of the walk: per wave a staging buffer (8 group slots of A atoms, or
 // F fetched records), a node stack and 8 group queues with dummy slots.
-template <int A, int F, bool TREE> struct Walk3Lds {
+template <int A, int F, bool TREE, int S = 1> struct Walk3Lds {
+    static constexpr int kQ = S > 1 ? kGroupQ / S : kGroupQ;  // entries per group queue
     static constexpr int kSlot = 4 * A + 4;  // floats per group slot (16 B pad: no bank conflicts)
     static constexpr int kRec = TREE ? 32 * F : 0;  // records: 8 float4 each
     static constexpr int kBufF = 8 * kSlot > kRec ? 8 * kSlot : kRec;
-    static constexpr int kW = nd::kBlock / 64;
+    static constexpr int kW = nd::kBlock / 64 * S;
     __align__(16) float buf[kW][kBufF];
     int32_t stk[TREE ? kW : 1][TREE ? kStack2 : 1];
-    int32_t q[kW][8 * kGroupQ + 64];
+    int32_t q[kW][8 * kQ + 64];
 };
 
-template <int A, int F, bool TREE, bool LOCAL>
+// S > 1 (leaf form): S waves share 64 atoms, wave slice w / 4 taking every S-th
+// leaf of a chunk; its records go to recs (each slice has its own) and its
+// counts to ncount / nrecs as threads, not atoms, number them.
+template <int A, int F, bool TREE, bool LOCAL, int S = 1>
 __device__ __forceinline__ void
 walk3_body(const float4 *__restrict__ pos, const WalkBoxes B, int32_t n, int32_t nL, float h, float rl2, int32_t cap,
            int32_t *__restrict__ ncount, int32_t *__restrict__ ctr, uint2 *__restrict__ recs,
-           int32_t *__restrict__ nrecs, Walk3Lds<A, F, TREE> &L, int32_t blk, int32_t *__restrict__ work,
+           int32_t *__restrict__ nrecs, Walk3Lds<A, F, TREE, S> &L, int32_t blk, int32_t *__restrict__ work,
            const float4 *__restrict__ tq = nullptr, const float4 *__restrict__ lc = nullptr) {
     static_assert(A == 4 || A == 8 || A == 16 || A == 32, "leaf size");
     constexpr int NV = (A + 7) / 8;      // atoms a lane stages per leaf (1, 2 or 4)
-    constexpr int kSlot = Walk3Lds<A, F, TREE>::kSlot;
+    constexpr int kSlot = Walk3Lds<A, F, TREE, S>::kSlot, kQ = Walk3Lds<A, F, TREE, S>::kQ;
+    static_assert(S == 1 || (!TREE && (S & (S - 1)) == 0), "waves per 64 atoms");
     const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int grp = lane >> 3, gl = lane & 7;
     float *buf = L.buf[w];
     float4 *rec = reinterpret_cast<float4 *>(buf);
     int32_t *stk = L.stk[TREE ? w : 0], *gq = L.q[w];  // the stack: tree form
 
-    const int32_t i = blk * nd::kBlock + threadIdx.x;
+    const int32_t i = blk * nd::kBlock + (threadIdx.x & (nd::kBlock - 1));
     const bool active = i < n;
     int32_t rcnt = 0, nrec = 0;           // list entries and records so far
     uint32_t pend_g = ~0u, pend_b = 0u;    // the record being built (leaves of one group merge)
@@ -1182,7 +1201,7 @@ walk3_body(const float4 *__restrict__ pos, const WalkBoxes B, int32_t n, int32_t
     auto enqueue = [&](int32_t leaf, uint64_t mk) {
         const uint32_t bits = (uint32_t)(mk >> (8 * lane)) & 0xFFu;
         const bool put = (lane < 8) & (bits != 0u);
-        gq[put ? lane * kGroupQ + glen : 8 * kGroupQ + lane] = (leaf << 8) | (int32_t)bits;
+        gq[put ? lane * kQ + glen : 8 * kQ + lane] = (leaf << 8) | (int32_t)bits;
         glen += put ? 1 : 0;
         ++nqu;
     };
@@ -1213,7 +1232,7 @@ walk3_body(const float4 *__restrict__ pos, const WalkBoxes B, int32_t n, int32_t
             if constexpr (NV > 2) { v2 = lp[16]; v3 = lp[24]; }
             if constexpr (LOCAL) cn = lc[(e >> 8) - 1];
         };
-        if (len > 0) load4(gq[grp * kGroupQ]);
+        if (len > 0) load4(gq[grp * kQ]);
         for (int32_t k = 0; k < steps; ++k) {
             wave_lds_sync();  // the previous step's reads are done
             if (k < len && gl < A) {
@@ -1224,8 +1243,8 @@ walk3_body(const float4 *__restrict__ pos, const WalkBoxes B, int32_t n, int32_t
             }
             wave_lds_sync();
             const float4 cc = cn;  // the staged leaf's centre and R^2 (LOCAL)
-            const int32_t e = k < len ? gq[grp * kGroupQ + k] : 0;
-            if (k + 1 < len) load4(gq[grp * kGroupQ + k + 1]);
+            const int32_t e = k < len ? gq[grp * kQ + k] : 0;
+            if (k + 1 < len) load4(gq[grp * kQ + k + 1]);
             uint32_t hits = 0u;
             const int32_t base = ((e >> 8) - 1) * A;
             // the list's pair test: |p - q|^2 < rl2, in this order of operations
@@ -1298,7 +1317,7 @@ walk3_body(const float4 *__restrict__ pos, const WalkBoxes B, int32_t n, int32_t
         stk[0] = nL + 1;  // the root is internal (nL >= 2)
         wave_lds_sync();
         while (sp > 0 || nqu > 0) {
-            if (nqu > 0 && (sp == 0 || nqu > kGroupQ - 4 * F)) {
+            if (nqu > 0 && (sp == 0 || nqu > kQ - 4 * F)) {
                 drain();
                 continue;
             }
@@ -1395,9 +1414,11 @@ walk3_body(const float4 *__restrict__ pos, const WalkBoxes B, int32_t n, int32_t
         int32_t cbase = 0, lbase = 0;         // first chunk of cmask, first leaf of lmask
         uint64_t smask = 0, cmask = 0, lmask = 0;  // supers, chunks and leaves still to look at
         bool more = true;
+        // the leaves of a chunk that this wave takes
+        const uint64_t mine = S == 1 ? ~0ull : (~0ull / ((1ull << S) - 1ull)) << __builtin_amdgcn_readfirstlane(w / (nd::kBlock / 64));
         while (more) {
             // ---- phase 1: queue leaves until a queue may be full or none are left ----
-            while (nqu < kGroupQ) {
+            while (nqu < kQ) {
                 if (lmask == 0) {
                     while (cmask == 0) {
                         while (smask == 0) {
@@ -1417,7 +1438,7 @@ walk3_body(const float4 *__restrict__ pos, const WalkBoxes B, int32_t n, int32_t
                     }
                     lbase = (cbase + __builtin_ctzll(cmask)) * kLeafChunk;
                     cmask &= cmask - 1ull;
-                    lmask = ~0ull;
+                    lmask = mine;
                     ++rounds;
                 }
                 // this chunk's leaf boxes, one per lane (again after a drain)
@@ -1428,7 +1449,7 @@ walk3_body(const float4 *__restrict__ pos, const WalkBoxes B, int32_t n, int32_t
                     b = q[1];
                 }
                 lmask &= __builtin_amdgcn_ballot_w64(lbase + lane < nL && near(a, b));
-                while (lmask != 0 && nqu < kGroupQ) {
+                while (lmask != 0 && nqu < kQ) {
                     const int32_t l = __builtin_ctzll(lmask);
                     lmask &= lmask - 1ull;
                     ++tests;
@@ -1457,18 +1478,16 @@ walk3_body(const float4 *__restrict__ pos, const WalkBoxes B, int32_t n, int32_t
         if (nrec < cap) myrec[nrec] = make_uint2(pend_g, pend_b);
         ++nrec;
     }
+    if constexpr (S > 1) {
+        ncount[threadIdx.x] = rcnt;
+        nrecs[threadIdx.x] = min(nrec, cap);
+        return;
+    }
     if (active) {
         ncount[i] = rcnt;
         nrecs[i] = nrec;
     }
-    int32_t m = rcnt;
-    for (int off = 32; off > 0; off >>= 1) m = max(m, __shfl_down(m, off, 64));
-    if (lane == 0 && m > 0) {
-        // the counter only grows: skip the (serialising) atomic when it is
-        // already at least m
-        if (m > __hip_atomic_load(&ctr[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(&ctr[0], m);
-        if (m > cap) atomicOr(&ctr[1], 1);
-    }
+    count_max(rcnt, cap, ctr);
 }
 
 // The walk alone (dense workloads: the table build's larger record buffer
@@ -1951,6 +1970,77 @@ k_walk_table(const float4 *__restrict__ pos, WalkBoxes B, int32_t n, int32_t nL,
                             hstale, slot_info, L.table, blk);
 }
 
+// The same with kSplit waves for each 64 atoms, where the workgroups leave most
+// CUs idle (up to 16,384 atoms): a wave's chain of leaf tests bounds the kernel
+// there (4,096 atoms: 49.0 -> 37.4 us; 32,768: 20.2 and 20.4 us a step with a
+// list every ten).  The first four waves join the slices' records, a slice after
+// the other, and build the table; the others have ended (a barrier waits for a
+// workgroup's remaining waves only).
+__global__ void __launch_bounds__(nd::kBlock * kSplit)
+k_walk_table_split(const float4 *__restrict__ pos, WalkBoxes B, int32_t n, int32_t nL, float h, float rl2, int32_t cap,
+                   int32_t *__restrict__ nbr, int32_t *__restrict__ ncount, int32_t *__restrict__ ctr,
+                   uint2 *__restrict__ recs, int32_t *__restrict__ nrecs, int32_t cap2, int32_t lcap, int32_t eshift,
+                   uint32_t *__restrict__ nbr16, int32_t *__restrict__ tables, int32_t *__restrict__ tcount,
+                   SimMisc *__restrict__ misc, volatile int32_t *hstale, uint32_t *__restrict__ slot_info,
+                   const float4 *__restrict__ tq, const float4 *__restrict__ lc, int64_t slice_recs) {
+    union Lds {
+        Walk3Lds<kSplitLeaf, kFront, false, kSplit> walk;
+        TableRecLds<kRecLds> table;
+    };
+    __shared__ Lds L;
+    __shared__ int32_t s_cnt[kSplit * nd::kBlock], s_nr[kSplit * nd::kBlock];
+    const int32_t blk = xcd_block(blockIdx.x, gridDim.x), tid = threadIdx.x;
+    const int32_t slice = __builtin_amdgcn_readfirstlane(tid / nd::kBlock);
+    walk3_body<kSplitLeaf, kFront, false, true, kSplit>(pos, B, n, nL, h, rl2, cap, s_cnt, ctr,
+                                                        recs + slice * slice_recs, s_nr, L.walk, blk, nullptr, tq, lc);
+    __syncthreads();  // every wave's records are written, and it is done with the LDS
+    if (tid >= nd::kBlock) return;
+    const int32_t i = blk * nd::kBlock + tid;
+    int32_t cnt = 0, nr = 0;
+    if (i < n) {
+        cnt = s_cnt[tid];
+        nr = s_nr[tid];
+        uint2 *my = recs + (int64_t)i * rec_stride(cap);
+        int32_t m[kSplit], most = 0;
+#pragma unroll
+        for (int s = 1; s < kSplit; ++s) {
+            cnt += s_cnt[s * nd::kBlock + tid];
+            m[s] = s_nr[s * nd::kBlock + tid];
+            most = max(most, m[s]);
+        }
+        int32_t at[kSplit];  // where slice s goes
+        int32_t end = nr;
+#pragma unroll
+        for (int s = 1; s < kSplit; ++s) {
+            at[s] = end;
+            end += m[s];
+        }
+        for (int32_t k = 0; k < most; k += 4) {
+            uint4 a[kSplit], b[kSplit];  // four records of every slice in flight
+#pragma unroll
+            for (int s = 1; s < kSplit; ++s) {
+                const uint4 *src = reinterpret_cast<const uint4 *>(my + s * slice_recs + k);
+                a[s] = k < m[s] ? src[0] : make_uint4(0u, 0u, 0u, 0u);
+                b[s] = k + 2 < m[s] ? src[1] : make_uint4(0u, 0u, 0u, 0u);
+            }
+#pragma unroll
+            for (int s = 1; s < kSplit; ++s) {
+                const uint2 r[4] = {make_uint2(a[s].x, a[s].y), make_uint2(a[s].z, a[s].w),
+                                    make_uint2(b[s].x, b[s].y), make_uint2(b[s].z, b[s].w)};
+#pragma unroll
+                for (int u = 0; u < 4; ++u)
+                    if (k + u < m[s] && at[s] + k + u < cap) my[at[s] + k + u] = r[u];
+            }
+        }
+        nr = end;
+        ncount[i] = cnt;
+        nrecs[i] = nr;
+    }
+    count_max(cnt, cap, ctr);
+    table_rec_body<kRecLds>(recs, nrecs, ncount, n, cap, cap2, lcap, eshift, nbr16, tables, tcount, nbr, misc,
+                            hstale, slot_info, L.table, blk);
+}
+
 // The walk order alone (when the step after a walk writes no energy row;
 // otherwise k_energy_finalize's blocks 1-8 compute it).
 __global__ void __launch_bounds__(nd::kBlock)
@@ -2061,6 +2151,7 @@ struct nd_sim {
     nd::DevBuf leaf_q;                 // two-phase walk: per atom (-2 q', |q'|^2) about its leaf's centre
     nd::DevBuf leaf_c;                 // two-phase walk: per leaf (centre, largest |q'|^2)
     int32_t cus_per_xcd = 32;          // compute units per XCD (the walk order's slot width)
+    bool walk_split = false;           // the leaf walk's workgroups leave most CUs idle: kSplit waves per 64 atoms
     bool order_pending = false;        // a fused walk ran; its work estimates are not yet ordered
     nd::DevBuf recs, nrecs;   // the two-phase walk's (group, mask) records per atom
     int32_t lcap = 0;         // table capacity (records) per workgroup
@@ -2184,21 +2275,6 @@ void copy_h2d(const nd::DevBuf &dst, const void *src, size_t bytes, hipStream_t 
     ND_HIP(hipMemcpyAsync(static_cast<char *>(dst.p) + off, src, bytes, hipMemcpyHostToDevice, st));
 }
 
-void alloc_lists(nd_sim *s, int32_t cap) {
-    // a wave's block of the list (cap rows of 256 B) is addressed through a
-    // buffer resource with a 31-bit byte range
-    if (cap > nd::kMaxListRows)
-        throw nd::Error(ND_ERR_CAPACITY, "simulation: 2^23 or more neighbours per atom");
-    s->cap = cap;
-    s->sp.cap = cap;
-    // one block of cap rows x 64 slots per 64 atoms (n rounded up to 64)
-    const size_t n64 = ((size_t)s->n + 63) & ~(size_t)63;
-    s->nbr.reserve(sizeof(int32_t) * (size_t)cap * n64);
-    s->nbr16.reserve(sizeof(uint32_t) * (size_t)rows16(cap) * n64);
-    s->recs.reserve(sizeof(uint2) * (size_t)rec_stride(cap) * n64);
-    drop_graphs(s);
-}
-
 hipEvent_t next_event(nd_sim *s) {
     if (s->ev_used == s->ev_pool.size()) {
         hipEvent_t e;
@@ -2215,7 +2291,8 @@ int32_t resort_period(const nd_sim *s) {
 }
 
 // Leaves of the leaf form of the two-phase walk, and boxes of 64 each.
-int32_t walk_leaves(const nd_sim *s) { return (int32_t)(((int64_t)s->n + kWalkLeaf - 1) / kWalkLeaf); }
+int32_t leaf_atoms(const nd_sim *s) { return s->walk_split ? kSplitLeaf : kWalkLeaf; }
+int32_t walk_leaves(const nd_sim *s) { return (int32_t)(((int64_t)s->n + leaf_atoms(s) - 1) / leaf_atoms(s)); }
 int32_t chunk_count(int32_t boxes) { return (boxes + kLeafChunk - 1) / kLeafChunk; }
 
 // The two-phase walk makes the simulation's list when asked for and the leaves
@@ -2230,6 +2307,21 @@ bool tree_walk(const nd_sim *s) {
            (s->apl == 4 || s->apl == 8 || s->apl == 16 || s->apl == 32);
 }
 bool two_phase_walk(const nd_sim *s) { return leaf_walk(s) || tree_walk(s); }
+
+void alloc_lists(nd_sim *s, int32_t cap) {
+    // a wave's block of the list (cap rows of 256 B) is addressed through a
+    // buffer resource with a 31-bit byte range
+    if (cap > nd::kMaxListRows)
+        throw nd::Error(ND_ERR_CAPACITY, "simulation: 2^23 or more neighbours per atom");
+    s->cap = cap;
+    s->sp.cap = cap;
+    // one block of cap rows x 64 slots per 64 atoms (n rounded up to 64)
+    const size_t n64 = ((size_t)s->n + 63) & ~(size_t)63;
+    s->nbr.reserve(sizeof(int32_t) * (size_t)cap * n64);
+    s->nbr16.reserve(sizeof(uint32_t) * (size_t)rows16(cap) * n64);
+    s->recs.reserve(sizeof(uint2) * (size_t)rec_stride(cap) * n64 * (s->walk_split && leaf_walk(s) ? kSplit : 1));
+    drop_graphs(s);
+}
 
 // A rebuild at step k re-sorts (new keys, order and topology) when the
 // period says so or when no tree matches the current order.
@@ -2291,7 +2383,7 @@ void launch_rebuild(nd_sim *s, bool full) {
         const float *p32 = s->wide ? reinterpret_cast<const float *>(s->pos32.p)
                                    : reinterpret_cast<const float *>(s->pos[s->cur].p);
         if (leaf_walk(s)) {
-            nd::launch_leaf_chunk_boxes(st, p32, 4, n, s->rlist, s->nodes.as<nd_node>(), s->leaf_chunks.as<float4>(),
+            nd::launch_leaf_chunk_boxes(st, p32, 4, n, leaf_atoms(s), s->rlist, s->nodes.as<nd_node>(), s->leaf_chunks.as<float4>(),
                                         s->leaf_q.as<float4>(), s->leaf_c.as<float4>());
         } else if (two_phase) {
             nd::launch_lbvh_refit_wide4(st, p32, 4, s->nL, s->apl, s->rlist, s->nodes.as<nd_node>(),
@@ -2353,7 +2445,12 @@ void launch_rebuild(nd_sim *s, bool full) {
 #define ND_WALKTAB(A, F, TREE)                                                                                   \
     k_walk_table<A, F, TREE><<<g, nd::kBlock, 0, st>>>(p4, B, n, leaves, hl, rl2, s->cap, nb, nc, ctr, rc, nr, c2, \
                                                        s->lcap, es, n16, tb, tc, misc, s->hstale, si, ord, wk, tql, lcl)
-                if (!tree) {
+                if (!tree && s->walk_split) {
+                    const int64_t per_slice = (int64_t)rec_stride(s->cap) * ((n + 63) & ~63);
+                    k_walk_table_split<<<g, nd::kBlock * kSplit, 0, st>>>(
+                        p4, B, n, leaves, hl, rl2, s->cap, nb, nc, ctr, rc, nr, c2, s->lcap, es, n16, tb, tc, misc,
+                        s->hstale, si, tql, lcl, per_slice);
+                } else if (!tree) {
                     ND_WALKTAB(kWalkLeaf, kFront, false);
                 } else if (s->walk_front == 16) {
                     switch (s->apl) {
@@ -2372,14 +2469,17 @@ void launch_rebuild(nd_sim *s, bool full) {
                 }
 #undef ND_WALKTAB
                 ND_HIP(hipGetLastError());
-                s->order_pending = true;  // the next force step's tail orders the next walk
+                // the next force step's tail orders the next walk, if CUs have several workgroups
+                s->order_pending = (int32_t)g > 8 * s->cus_per_xcd;
                 return;
             }
             // dense workloads: the walk, then the table build with the larger
             // record buffer (its LDS would lower the walk's occupancy)
 #define ND_NLIST3(A, F, TREE) \
     k_nlist3<A, F, TREE><<<g, nd::kBlock, 0, st>>>(p4, B, n, leaves, hl, rl2, s->cap, nc, ctr, rc, nr)
-            if (!tree) {
+            if (!tree && s->walk_split) {
+                ND_NLIST3(kSplitLeaf, kFront, false);
+            } else if (!tree) {
                 ND_NLIST3(kWalkLeaf, kFront, false);
             } else if (s->walk_front == 16) {
                 switch (s->apl) {
@@ -2445,7 +2545,7 @@ void launch_sort_and_build(nd_sim *s) {
     const int a = s->cur ^ 1, va = s->vcur ^ 1;
     // leaf boxes in the permutation for power-of-two leaves up to 64 (the
     // cell walk needs no tree, so none there)
-    const int32_t per_leaf = leaves_only ? kWalkLeaf : s->apl;
+    const int32_t per_leaf = leaves_only ? leaf_atoms(s) : s->apl;
     const bool boxes = s->p.list_walk != 3 && per_leaf <= 64 && (per_leaf & (per_leaf - 1)) == 0;
     // the two-phase walk's leaf-local copies, written with the leaf boxes
     float4 *lq = two_phase_walk(s) ? s->leaf_q.as<float4>() : nullptr;
@@ -3003,6 +3103,10 @@ int nd_sim_create(nd_ctx *ctx, const nd_sim_params *p, nd_sim **out) {
         s->apl = p->atomsperleaf;
         s->nL = p->n / p->atomsperleaf;
         s->wide = p->precision != ND_PREC_FP32;
+        int cus = 256;
+        ND_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ctx->device));
+        s->cus_per_xcd = cus >= 8 ? cus / 8 : 1;
+        s->walk_split = 4 * (int)nd::grid_for(s->n) <= cus;
         // The list is built from FP32 coordinates; pad its radius by the FP32
         // rounding of coordinates in the box (2^-20 relative) so that it stays
         // a superset of the pairs inside the cutoff in every precision form.
@@ -3067,9 +3171,6 @@ int nd_sim_create(nd_ctx *ctx, const nd_sim_params *p, nd_sim **out) {
                                   hipMemcpyHostToDevice, ctx->stream));
             ND_HIP(hipMemsetAsync(s->walk_work.p, 0, sizeof(int32_t) * 4 * (size_t)nb, ctx->stream));
             ND_HIP(hipStreamSynchronize(ctx->stream));
-            int cus = 256;
-            ND_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ctx->device));
-            s->cus_per_xcd = cus >= 8 ? cus / 8 : 1;
         }
         s->misc.reserve(sizeof(SimMisc));
         s->partials.reserve(sizeof(double) * 4 * (size_t)nd::grid_for(s->n));

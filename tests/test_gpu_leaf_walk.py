@@ -23,9 +23,9 @@ def _run(pkg, n, apl, walk, precision, steps, state):
     return np.array(sim.get_state()[0]), np.array(sim.energies())
 
 
-# two leaves of one atom; one wave less one atom; one more than a leaf, a
-# workgroup and a chunk (2,048 atoms); odd leaf sizes
-@pytest.mark.parametrize("n,apl", [(2, 1), (63, 3), (66, 2), (257, 1), (2049, 3), (4100, 5), (30003, 3)])
+# up to 16,384 atoms four waves share each 64: one wave less one atom, one more
+# than a workgroup and than a chunk (1,024 or 2,048 atoms), odd leaf sizes
+@pytest.mark.parametrize("n,apl", [(2, 1), (63, 3), (66, 2), (257, 1), (2049, 3), (4100, 5), (16383, 3), (16641, 3), (65793, 3)])
 def test_ragged_leaves(pkg, n, apl):
     s = _state(pkg, n, n)
     x0, e0 = _run(pkg, n, apl, 0, "fp64", 13, s)
