@@ -204,6 +204,67 @@ k_radix_scatter(const int32_t *__restrict__ keys_in, const int32_t *__restrict__
     }
 }
 
+// Few keys: one launch that counts, for each key, the keys before it (smaller,
+// or equal and earlier), which is its place.  A radix pass is three launches of
+// 3.3 to 6.6 us whatever the size; here a workgroup keeps all keys in LDS and
+// ranks kRankRun of them (few, so that 4,096 keys fill the CUs: 64 a workgroup
+// took 9.0 us), a lane comparing one of them with every 64th run of keys.
+// 4,096 keys of 20 bits: 26.7 us in two 10-bit passes, 6.4 ranked; a step with a
+// list of 8,192 atoms takes 106 us, of 8,193 in radix passes 114.
+constexpr int kRankMax = 8192, kRankThreads = 1024, kRankRun = 16;
+
+__global__ void __launch_bounds__(kRankThreads)
+k_rank_sort(const int32_t *__restrict__ keys, const int32_t *__restrict__ vals, int32_t n, uint32_t mask,
+            int32_t *__restrict__ keys_out, int32_t *__restrict__ vals_out) {
+    constexpr int kWaves = kRankThreads / 64, kPer = kRankMax / kRankThreads, kSlices = kRankThreads / kRankRun;
+    extern __shared__ __align__(16) uint32_t s_key[];  // n rounded up to kRankRun
+    __shared__ int32_t s_count[kWaves][kRankRun];
+    const int32_t tid = threadIdx.x, w = tid >> 6, own = tid % kRankRun, slice = tid / kRankRun;
+    const int32_t nruns = (n + kRankRun - 1) / kRankRun, mine = blockIdx.x, i = mine * kRankRun + own;
+    int32_t v[kPer], my_key = 0, my_val = 0;
+#pragma unroll
+    for (int u = 0; u < kPer; ++u) {  // every load in flight
+        const int32_t t = u * kRankThreads + tid;
+        v[u] = t < n ? keys[t] : 0;
+    }
+    if (tid < kRankRun && i < n) {
+        my_key = keys[i];
+        my_val = vals[i];
+    }
+#pragma unroll
+    for (int u = 0; u < kPer; ++u) {
+        const int32_t t = u * kRankThreads + tid;
+        // past the end: after all
+        if (t < nruns * kRankRun) s_key[t] = t < n ? ((uint32_t)v[u] ^ 0x80000000u) & mask : 0xFFFFFFFFu;
+    }
+    __syncthreads();
+    const uint32_t key = s_key[i];
+    int32_t before = 0;
+    for (int32_t r = slice; r < nruns; r += kSlices) {
+        const uint4 *run = reinterpret_cast<const uint4 *>(s_key + kRankRun * r);
+        // equal keys: all of an earlier run's come before, of the own run those
+        // of earlier lanes
+        const int32_t ties = r < mine ? kRankRun : (r == mine ? own : 0);
+#pragma unroll
+        for (int k = 0; k < kRankRun / 4; ++k) {
+            const uint4 q = run[k];
+            before += (q.x < key) + (q.y < key) + (q.z < key) + (q.w < key);
+            before += ((q.x == key) & (4 * k < ties)) + ((q.y == key) & (4 * k + 1 < ties)) +
+                      ((q.z == key) & (4 * k + 2 < ties)) + ((q.w == key) & (4 * k + 3 < ties));
+        }
+    }
+#pragma unroll
+    for (int o = kRankRun; o < 64; o <<= 1) before += __shfl_xor(before, o, 64);
+    if ((tid & 63) < kRankRun) s_count[w][own] = before;
+    __syncthreads();
+    if (tid >= kRankRun || i >= n) return;
+    int32_t at = 0;
+#pragma unroll
+    for (int k = 0; k < kWaves; ++k) at += s_count[k][own];
+    keys_out[at] = my_key;
+    vals_out[at] = my_val;
+}
+
 __global__ void __launch_bounds__(nd::kBlock)
 k_keybits(const int32_t *__restrict__ keys, int32_t n, uint32_t *__restrict__ out) {
     uint32_t o = 0u, a = 0xFFFFFFFFu;
@@ -299,6 +360,15 @@ int radix_passes(hipStream_t s, SortBufs &b, int32_t *keys, int32_t *vals, int32
     return passes;
 }
 
+// n <= kRankMax pairs in the order of their keys' bits in mask (sign flipped).
+void rank_sort(hipStream_t s, const int32_t *keys, const int32_t *vals, int32_t n, uint32_t mask, int32_t *keys_out,
+               int32_t *vals_out) {
+    const size_t nruns = ((size_t)n + kRankRun - 1) / kRankRun;
+    k_rank_sort<<<(unsigned)nruns, kRankThreads, sizeof(uint32_t) * kRankRun * nruns, s>>>(keys, vals, n, mask,
+                                                                                       keys_out, vals_out);
+    ND_HIP(hipGetLastError());
+}
+
 }  // namespace
 
 void radix_sort_pairs(hipStream_t s, SortBufs &b, int32_t *keys, int32_t *vals, int32_t n,
@@ -316,6 +386,14 @@ void radix_sort_keys10(hipStream_t s, SortBufs &b, int32_t *keys, int32_t *vals,
     *keys_sorted = keys;
     *vals_sorted = vals;
     if (n <= 1) return;
+    if (n <= kRankMax && key_bits < 32) {
+        b.keys_alt.reserve(sizeof(int32_t) * (size_t)n);
+        b.vals_alt.reserve(sizeof(int32_t) * (size_t)n);
+        *keys_sorted = b.keys_alt.as<int32_t>();
+        *vals_sorted = b.vals_alt.as<int32_t>();
+        rank_sort(s, keys, vals, n, (1u << key_bits) - 1u, *keys_sorted, *vals_sorted);
+        return;
+    }
     const int passes = radix_passes<10>(s, b, keys, vals, n, 0, key_bits);
     if (passes & 1) {
         *keys_sorted = b.keys_alt.as<int32_t>();
@@ -325,10 +403,16 @@ void radix_sort_keys10(hipStream_t s, SortBufs &b, int32_t *keys, int32_t *vals,
 
 // The varying bits lo .. hi take one 10-bit pass where they fit (22 against 2 x
 // 15 us at 262,144 keys: the masked key of the unit cube has 10), else 8-bit
-// passes from lo up, windows without a varying bit left out.
+// passes from lo up, windows without a varying bit left out; few keys are ranked.
 void radix_sort_bits(hipStream_t s, SortBufs &b, uint32_t vary, int32_t n, int32_t **keys, int32_t **vals,
                      int32_t *keys2, int32_t *vals2) {
     if (n <= 1 || vary == 0u) return;
+    if (n <= kRankMax) {
+        rank_sort(s, *keys, *vals, n, 0xFFFFFFFFu, keys2, vals2);
+        std::swap(*keys, keys2);
+        std::swap(*vals, vals2);
+        return;
+    }
     const int lo = __builtin_ctz(vary), span = 32 - __builtin_clz(vary) - lo;
     const bool ten = span > 8 && span <= 10;
     const size_t ntiles = radix_scratch_blocks(n), R = ten ? 1024 : 256;
