@@ -1158,8 +1158,8 @@ template <int A, int F, bool TREE, int S = 1> struct Walk3Lds {
     int32_t q[kW][8 * kQ + 64];
 };
 
-// S > 1 (leaf form): S waves share 64 atoms, wave slice w / 4 taking every S-th
-// leaf of a chunk; its records go to recs (each slice has its own) and its
+// S > 1 (leaf form): S waves share 64 atoms, wave slice w / 4 taking the leaves
+// of every S-th 32-atom group of a chunk; its records go to recs (each slice has its own) and its
 // counts to ncount / nrecs as threads, not atoms, number them.
 template <int A, int F, bool TREE, bool LOCAL, int S = 1>
 __device__ __forceinline__ void
@@ -1414,8 +1414,12 @@ walk3_body(const float4 *__restrict__ pos, const WalkBoxes B, int32_t n, int32_t
         int32_t cbase = 0, lbase = 0;         // first chunk of cmask, first leaf of lmask
         uint64_t smask = 0, cmask = 0, lmask = 0;  // supers, chunks and leaves still to look at
         bool more = true;
-        // the leaves of a chunk that this wave takes
-        const uint64_t mine = S == 1 ? ~0ull : (~0ull / ((1ull << S) - 1ull)) << __builtin_amdgcn_readfirstlane(w / (nd::kBlock / 64));
+        // the leaves of a chunk that this wave takes: all, or every S-th 32-atom
+        // group's (its leaves' hits join in one record)
+        constexpr int kGrp = 32 / A;
+        const uint64_t mine = S == 1 ? ~0ull
+                                     : ((~0ull / ((1ull << (S * kGrp % 64)) - 1ull)) * ((1ull << kGrp) - 1ull))
+                                           << (kGrp * __builtin_amdgcn_readfirstlane(w / (nd::kBlock / 64)));
         while (more) {
             // ---- phase 1: queue leaves until a queue may be full or none are left ----
             while (nqu < kQ) {
@@ -1531,10 +1535,11 @@ __device__ __forceinline__ uint32_t group_hash(int32_t g) {
 // empty), the mask of its atoms in use and (after finish()) the table
 // position of the group's first atom in use.
 struct TableLds {
+    static constexpr int kMaxThreads = nd::kBlock * kSplit;
     int32_t key[kHashSlots];
     uint32_t mask[kHashSlots];
     int32_t base[kHashSlots];
-    int32_t part[nd::kBlock / 64];
+    int32_t part[kMaxThreads / 64];
     int32_t fail;
 
     __device__ void init() {
@@ -1562,8 +1567,9 @@ struct TableLds {
     // After every insert (and a barrier): group bases by an exclusive scan of
     // the masks' population counts; returns the table size, or -1 when the
     // table does not fit (lcap) or the hash overflowed.  Ends with a barrier.
-    __device__ int32_t finish(int32_t lcap) {
-        constexpr int kPer = kHashSlots / nd::kBlock;
+    // NT: threads of the workgroup.
+    template <int NT = nd::kBlock> __device__ int32_t finish(int32_t lcap) {
+        constexpr int kPer = kHashSlots / NT;
         const int32_t tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
         int32_t c[kPer], tot = 0;
 #pragma unroll
@@ -1577,7 +1583,7 @@ struct TableLds {
         __syncthreads();
         int32_t wbase = 0, U = 0;
 #pragma unroll
-        for (int k = 0; k < nd::kBlock / 64; ++k) {
+        for (int k = 0; k < NT / 64; ++k) {
             wbase += k < w ? part[k] : 0;
             U += part[k];
         }
@@ -1592,8 +1598,8 @@ struct TableLds {
     // A wave writes the runs of its lanes' non-empty slots two at a time,
     // a half-wave per run (lane b of the half writes the entry of bit b), so
     // the stores of a run are consecutive rather than one lane's serial loop.
-    __device__ void write(int32_t *tab) const {
-        constexpr int kPer = kHashSlots / nd::kBlock;
+    template <int NT = nd::kBlock> __device__ void write(int32_t *tab) const {
+        constexpr int kPer = kHashSlots / NT;
         const int lane = threadIdx.x & 63, bit = lane & 31;
 #pragma unroll
         for (int k = 0; k < kPer; ++k) {
@@ -1724,7 +1730,7 @@ k_table(const int32_t *__restrict__ nbr, const int32_t *__restrict__ ncount, int
 // CU) unless the first checked build of a simulation saw more than 1/64 of
 // its workgroups spill, as on dense blobs (about 13 records per atom), which
 // then take RL = 5120 (53.3 KB: three per CU).
-constexpr int kRecLds = 3072, kRecLdsBig = 5120;
+constexpr int kRecLds = 3072, kRecLdsBig = 5120, kRecLdsSplit = 4096;
 
 // LDS of a table build from records: the hash and RL records (hash slot, mask)
 template <int RL> struct TableRecLds {
@@ -1971,11 +1977,17 @@ k_walk_table(const float4 *__restrict__ pos, WalkBoxes B, int32_t n, int32_t nL,
 }
 
 // The same with kSplit waves for each 64 atoms, where the workgroups leave most
-// CUs idle (up to 16,384 atoms): a wave's chain of leaf tests bounds the kernel
-// there (4,096 atoms: 49.0 -> 37.4 us; 32,768: 20.2 and 20.4 us a step with a
-// list every ten).  The first four waves join the slices' records, a slice after
-// the other, and build the table; the others have ended (a barrier waits for a
-// workgroup's remaining waves only).
+// CUs idle (up to 16,384 atoms): there a wave's chains of leaf tests and, in the
+// table build, of LDS reads per list entry bound the kernel.  Each slice enters
+// its own records in the hash and expands them into its own part of the lists.
+// 4,096 atoms: 49.0 us with one wave, 37.1 with the walk split, 35.0 with both;
+// 8,192 atoms with a list every step: 106 and 79.6 us a step; 32,768 gain nothing
+// (20.2 and 20.4 us a step with a list every ten).
+struct TableSplitLds {
+    TableRecLds<kRecLdsSplit> table;
+    int32_t roff[nd::kBlock * kSplit], wsum[nd::kBlock * kSplit / 64];
+};
+
 __global__ void __launch_bounds__(nd::kBlock * kSplit)
 k_walk_table_split(const float4 *__restrict__ pos, WalkBoxes B, int32_t n, int32_t nL, float h, float rl2, int32_t cap,
                    int32_t *__restrict__ nbr, int32_t *__restrict__ ncount, int32_t *__restrict__ ctr,
@@ -1983,62 +1995,137 @@ k_walk_table_split(const float4 *__restrict__ pos, WalkBoxes B, int32_t n, int32
                    uint32_t *__restrict__ nbr16, int32_t *__restrict__ tables, int32_t *__restrict__ tcount,
                    SimMisc *__restrict__ misc, volatile int32_t *hstale, uint32_t *__restrict__ slot_info,
                    const float4 *__restrict__ tq, const float4 *__restrict__ lc, int64_t slice_recs) {
+    constexpr int NT = nd::kBlock * kSplit;
     union Lds {
         Walk3Lds<kSplitLeaf, kFront, false, kSplit> walk;
+        TableSplitLds split;
         TableRecLds<kRecLds> table;
     };
     __shared__ Lds L;
-    __shared__ int32_t s_cnt[kSplit * nd::kBlock], s_nr[kSplit * nd::kBlock];
-    const int32_t blk = xcd_block(blockIdx.x, gridDim.x), tid = threadIdx.x;
-    const int32_t slice = __builtin_amdgcn_readfirstlane(tid / nd::kBlock);
+    __shared__ int32_t s_cnt[NT], s_nr[NT];
+    const int32_t blk = xcd_block(blockIdx.x, gridDim.x), tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    const int32_t t = tid & (nd::kBlock - 1), slice = __builtin_amdgcn_readfirstlane(tid / nd::kBlock);
+    const int32_t i = blk * nd::kBlock + t;
     walk3_body<kSplitLeaf, kFront, false, true, kSplit>(pos, B, n, nL, h, rl2, cap, s_cnt, ctr,
                                                         recs + slice * slice_recs, s_nr, L.walk, blk, nullptr, tq, lc);
-    __syncthreads();  // every wave's records are written, and it is done with the LDS
-    if (tid >= nd::kBlock) return;
-    const int32_t i = blk * nd::kBlock + tid;
-    int32_t cnt = 0, nr = 0;
-    if (i < n) {
-        cnt = s_cnt[tid];
-        nr = s_nr[tid];
-        uint2 *my = recs + (int64_t)i * rec_stride(cap);
-        int32_t m[kSplit], most = 0;
+    const int32_t nr = i < n ? s_nr[tid] : 0;  // this thread's own
+    __syncthreads();  // every wave's counts are written, and it is done with the LDS
+    // atom t's neighbours over the slices
+    int32_t cnt = 0;
 #pragma unroll
-        for (int s = 1; s < kSplit; ++s) {
-            cnt += s_cnt[s * nd::kBlock + tid];
-            m[s] = s_nr[s * nd::kBlock + tid];
-            most = max(most, m[s]);
-        }
-        int32_t at[kSplit];  // where slice s goes
-        int32_t end = nr;
-#pragma unroll
-        for (int s = 1; s < kSplit; ++s) {
-            at[s] = end;
-            end += m[s];
-        }
-        for (int32_t k = 0; k < most; k += 4) {
-            uint4 a[kSplit], b[kSplit];  // four records of every slice in flight
-#pragma unroll
-            for (int s = 1; s < kSplit; ++s) {
-                const uint4 *src = reinterpret_cast<const uint4 *>(my + s * slice_recs + k);
-                a[s] = k < m[s] ? src[0] : make_uint4(0u, 0u, 0u, 0u);
-                b[s] = k + 2 < m[s] ? src[1] : make_uint4(0u, 0u, 0u, 0u);
-            }
-#pragma unroll
-            for (int s = 1; s < kSplit; ++s) {
-                const uint2 r[4] = {make_uint2(a[s].x, a[s].y), make_uint2(a[s].z, a[s].w),
-                                    make_uint2(b[s].x, b[s].y), make_uint2(b[s].z, b[s].w)};
-#pragma unroll
-                for (int u = 0; u < 4; ++u)
-                    if (k + u < m[s] && at[s] + k + u < cap) my[at[s] + k + u] = r[u];
-            }
-        }
-        nr = end;
-        ncount[i] = cnt;
-        nrecs[i] = nr;
+    for (int s = 0; s < kSplit; ++s) cnt += i < n ? s_cnt[s * nd::kBlock + t] : 0;
+    if (slice == 0) {
+        if (i < n) ncount[i] = cnt;
+        count_max(cnt, cap, ctr);
     }
-    count_max(cnt, cap, ctr);
-    table_rec_body<kRecLds>(recs, nrecs, ncount, n, cap, cap2, lcap, eshift, nbr16, tables, tcount, nbr, misc,
-                            hstale, slot_info, L.table, blk);
+    cnt = min(cnt, cap);
+
+    TableLds &T = L.split.table.T;
+    uint2 *s_rec = L.split.table.rec;  // (hash slot, mask)
+    T.init();
+    int32_t incl = nr;
+    for (int off = 1; off < 64; off <<= 1) {
+        const int32_t y = __shfl_up(incl, off, 64);
+        if (lane >= off) incl += y;
+    }
+    if (lane == 63) L.split.wsum[w] = incl;
+    __syncthreads();
+    int32_t roff = incl - nr, rtot = 0;
+#pragma unroll
+    for (int k = 0; k < NT / 64; ++k) {
+        roff += k < w ? L.split.wsum[k] : 0;
+        rtot += L.split.wsum[k];
+    }
+    const uint2 *my = recs + slice * slice_recs + (int64_t)i * rec_stride(cap);
+    int32_t U = -1;
+    if (rtot <= kRecLdsSplit) {  // uniform over the workgroup
+        for (int32_t k0 = 0; k0 < nr; k0 += 4) {
+            const uint4 *src = reinterpret_cast<const uint4 *>(my + k0);
+            const uint4 a = src[0], b = k0 + 2 < nr ? src[1] : make_uint4(0u, 0u, 0u, 0u);
+            const uint2 r[4] = {make_uint2(a.x, a.y), make_uint2(a.z, a.w), make_uint2(b.x, b.y),
+                                make_uint2(b.z, b.w)};
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+                if (k0 + u < nr)
+                    s_rec[roff + k0 + u] = make_uint2((uint32_t)T.insert((int32_t)r[u].x, r[u].y), r[u].y);
+        }
+        L.split.roff[tid] = roff;
+        __syncthreads();
+        U = T.finish<NT>(lcap);  // ends with a barrier
+    }
+    if (U < 0) {
+        // too many records or no table (uniform): the first four waves join the
+        // slices' records, a slice after the other, and build as one wave per 64
+        // atoms does (a barrier waits for the waves that have not ended)
+        __syncthreads();
+        if (slice != 0) return;
+        if (i < n) {
+            uint2 *all = recs + (int64_t)i * rec_stride(cap);
+            int32_t at = nr;
+            for (int s = 1; s < kSplit; ++s) {
+                const int32_t m = s_nr[s * nd::kBlock + t];
+                for (int32_t k = 0; k < m; ++k, ++at)
+                    if (at < cap) all[at] = all[s * slice_recs + k];
+            }
+            nrecs[i] = at;
+        }
+        table_rec_body<kRecLds>(recs, nrecs, ncount, n, cap, cap2, lcap, eshift, nbr16, tables, tcount, nbr, misc,
+                                hstale, slot_info, L.table, blk);
+        return;
+    }
+    stale_to_host(misc, hstale);
+    if (tid == 0) tcount[blk] = U;
+    T.write<NT>(tables + (int64_t)blk * lcap);
+    // lists by decreasing length (as table_rec_body): every slice sorts the same
+    // 256 keys, and writes the same words across waves
+    uint32_t key = ((uint32_t)(0xFFFF - min(cnt, 0xFFFF)) << 8) | (uint32_t)t;
+    uint32_t *sk = reinterpret_cast<uint32_t *>(T.key);
+    __syncthreads();  // the table write's reads of the hash keys are done
+#pragma unroll
+    for (int k = 2; k <= nd::kBlock; k <<= 1) {
+#pragma unroll
+        for (int j = k >> 1; j > 0; j >>= 1) {
+            uint32_t other;
+            if (j >= 64) {
+                __syncthreads();
+                sk[t] = key;
+                __syncthreads();
+                other = sk[t ^ j];
+            } else {
+                other = (uint32_t)__shfl_xor((int)key, j, 64);
+            }
+            const bool up = (t & k) == 0, lower = (t & j) == 0;
+            key = (lower == up) ? min(key, other) : max(key, other);
+        }
+    }
+    const int32_t a = (int32_t)(key & 0xFFu);
+    int32_t len = 0, e = 0;  // column t's list, and this slice's first entry of it
+#pragma unroll
+    for (int s = 0; s < kSplit; ++s) {
+        const int32_t c = blk * nd::kBlock + a < n ? s_cnt[s * nd::kBlock + a] : 0;
+        e += s < slice ? c : 0;
+        len += c;
+    }
+    len = min(len, cap);
+    if (slice == 0) slot_info[i] = ((uint32_t)len << 8) | (uint32_t)a;
+    if (((i >> 6) << 6) >= n) return;  // waves past the last atom own no list block
+    int32_t wmax = len;
+    for (int off = 32; off > 0; off >>= 1) wmax = max(wmax, __shfl_xor(wmax, off, 64));
+    const int32_t rows = 2 * (max((wmax + 1) >> 1, 1) + 2);  // entries of a column, sentinels among them
+    uint16_t *out = reinterpret_cast<uint16_t *>(nbr16 + ((int64_t)(i >> 6) * cap2) * 64 + lane);
+    auto put = [&](int32_t at, uint32_t v) { out[(at >> 1) * 128 + (at & 1)] = (uint16_t)(v << eshift); };
+    const int32_t m = blk * nd::kBlock + a < n ? s_nr[slice * nd::kBlock + a] : 0;
+    const int32_t r0 = L.split.roff[slice * nd::kBlock + a];
+    for (int32_t k = 0; k < m; ++k) {
+        const uint2 r = s_rec[r0 + k];
+        const int32_t cb = T.base[r.x];
+        const uint32_t gm = T.mask[r.x];
+        for (uint32_t bits = r.y; bits; bits &= bits - 1u, ++e) {
+            const int32_t b = __builtin_ctz(bits);
+            if (e < cap) put(e, (uint32_t)(cb + __popc(gm & ((1u << b) - 1u))));
+        }
+    }
+    for (int32_t k = len + slice; k < rows; k += kSplit) put(k, (uint32_t)U);
 }
 
 // The walk order alone (when the step after a walk writes no energy row;

@@ -44,3 +44,23 @@ def test_more_chunks_than_are_looked_at_one_by_one(pkg):
     # FP32 positions of a box of side 110 (half an ulp 4e-6, one rounding a step)
     assert np.abs(x0 - x3).max() < 2e-4
     assert np.allclose(e0[:, 2:4], e3[:, 2:4], rtol=1e-6)
+
+
+def test_more_records_than_the_shared_table_build_holds(pkg):
+    """Density 4: 370 neighbours an atom in more records than LDS takes, so the
+    waves' records are joined in memory (then the kernels for dense systems)."""
+    n = 4100
+    L = (n / 4.0) ** (1.0 / 3.0)
+    x, q = pkg.synth.lattice_positions(n, L, 3), pkg.synth.balanced_charges(n, 3)
+    out = []
+    for walk in (0, 3):
+        sim = pkg.Simulation(n, pkg.SimSpec(duration=0, stepwidth=1e-5, rc=2.5, rc_coul=2.5, skin=0.3, rebuild_every=4,
+                                            lo=0.0, hi=L, precision="fp64", energy_every=1, atomsperleaf=5,
+                                            resort_every=8, list_walk=walk))
+        sim.set_state(x, np.zeros((n, 3)), q)
+        sim.run(13)
+        out.append((np.array(sim.get_state()[2]), np.array(sim.energies())))
+    (f0, e0), (f3, e3) = out
+    assert np.array_equal(e0[:, 4], e3[:, 4])
+    # 13 steps of FP64 rounding in sums of 370 pair forces
+    assert np.abs(f0 - f3).max() < 1e-10 * np.abs(f3).max()
