@@ -1114,10 +1114,14 @@ constexpr int kSplitLeaf = 16;    // and where kSplit waves share each 64 atoms
 constexpr int kSplit = 4;
 constexpr int kLeafChunk = 64;    // leaves per chunk, chunks per super
 constexpr int kFlatChunks = 512;  // more chunks than this have supers
+// Up to this many chunks no box of theirs is made or tested: most are near any
+// wave, and a launch a list is saved (4,096 atoms with a list every step: 65.7 -> 62.4
+// us a step).
+constexpr int kPlainChunks = 4;
 
 // What phase 1 reads: the leaves' boxes (padded by h on each side) and the boxes
-// of 64 leaves and of 64 chunks (supers null where the chunks are few), or the
-// tree's four-wide records.
+// of 64 leaves and of 64 chunks (null where they are not needed), or the tree's
+// four-wide records.
 struct WalkBoxes {
     const nd_node *leaves;
     const float4 *chunks, *supers, *wide;
@@ -1409,6 +1413,7 @@ walk3_body(const float4 *__restrict__ pos, const WalkBoxes B, int32_t n, int32_t
             if (k < count) ov = near(boxes[2 * (int64_t)k], boxes[2 * (int64_t)k + 1]);
             return __builtin_amdgcn_ballot_w64(ov);
         };
+        auto all64 = [](int32_t count) -> uint64_t { return count >= 64 ? ~0ull : (1ull << count) - 1ull; };
         const int32_t nC = (nL + kLeafChunk - 1) / kLeafChunk, nS = (nC + kLeafChunk - 1) / kLeafChunk;
         int32_t sbase = -kLeafChunk;          // first super of the batch in smask
         int32_t cbase = 0, lbase = 0;         // first chunk of cmask, first leaf of lmask
@@ -1428,13 +1433,12 @@ walk3_body(const float4 *__restrict__ pos, const WalkBoxes B, int32_t n, int32_t
                         while (smask == 0) {
                             sbase += kLeafChunk;
                             if (sbase >= nS) break;
-                            smask = B.supers ? near64(B.supers, sbase, nS)
-                                           : (nS - sbase >= 64 ? ~0ull : (1ull << (nS - sbase)) - 1ull);
+                            smask = B.supers ? near64(B.supers, sbase, nS) : all64(nS - sbase);
                         }
                         if (smask == 0) break;
                         cbase = (sbase + __builtin_ctzll(smask)) * kLeafChunk;
                         smask &= smask - 1ull;
-                        cmask = near64(B.chunks, cbase, nC);
+                        cmask = B.chunks ? near64(B.chunks, cbase, nC) : all64(nC - cbase);
                     }
                     if (cmask == 0) {
                         more = false;
@@ -2507,7 +2511,7 @@ void launch_rebuild(nd_sim *s, bool full) {
             const int32_t nC = chunk_count(leaves);
             float4 *ch = s->leaf_chunks.as<float4>();  // the chunks' boxes, then the supers'
             B.leaves = s->nodes.as<nd_node>();
-            B.chunks = ch;
+            B.chunks = nC > kPlainChunks ? ch : nullptr;
             if (nC > kFlatChunks) {
                 B.supers = ch + 2 * (int64_t)nC;
                 nd::launch_chunk_boxes(st, reinterpret_cast<const nd_node *>(ch), nC, ch + 2 * (int64_t)nC);
@@ -2670,7 +2674,8 @@ void launch_sort_and_build(nd_sim *s) {
         return;
     }
     if (leaves_only) {  // the leaves' boxes (the permutation's) and their chunks'
-        nd::launch_chunk_boxes(st, nodes, walk_leaves(s), s->leaf_chunks.as<float4>());
+        if (chunk_count(walk_leaves(s)) > kPlainChunks)
+            nd::launch_chunk_boxes(st, nodes, walk_leaves(s), s->leaf_chunks.as<float4>());
         return;
     }
     const float *p32 = s->wide ? reinterpret_cast<const float *>(s->pos32.p)
