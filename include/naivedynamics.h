@@ -272,8 +272,9 @@ typedef struct {
                              rebuild_every; 0 = every rebuild).  Rebuilds in between
                              keep the atom order and tree topology and refit the
                              boxes to the current positions. */
-    int32_t list_walk;    /* list walk: 0 = two-phase child-box walk (node frontier, then
-                             queued leaves), 1 = rope walk, 2 = one-node child-box walk,
+    int32_t list_walk;    /* list walk: 0 = two-phase walk (leaves found through the boxes
+                             of 64 leaves, or of a tree for MIXED; then their
+                             atoms), 1 = rope walk, 2 = one-node child-box walk,
                              3 = uniform cell list over [lo, hi]^3 (no LBVH; the
                              comparison point; needs hi > lo) */
     int32_t pair_batch;   /* step kernel: neighbours per software-pipeline batch, 2, 4 or

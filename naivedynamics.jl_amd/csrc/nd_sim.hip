@@ -1499,15 +1499,17 @@ walk3_body(const float4 *__restrict__ pos, const WalkBoxes B, int32_t n, int32_t
 }
 
 // The walk alone (dense workloads: the table build's larger record buffer
-// would lower a joint kernel's occupancy).
+// would lower a joint kernel's occupancy).  The leaf form tests the leaf-local
+// copies at four waves per SIMD (96 replicas: 162 -> 150 us); the tree form's
+// five measured no faster with them.
 template <int A, int F, bool TREE>
-__global__ void __launch_bounds__(nd::kBlock)
+__global__ void __launch_bounds__(nd::kBlock, TREE ? 1 : 4)
 k_nlist3(const float4 *__restrict__ pos, WalkBoxes B, int32_t n, int32_t nL, float h, float rl2, int32_t cap,
          int32_t *__restrict__ ncount, int32_t *__restrict__ ctr, uint2 *__restrict__ recs,
-         int32_t *__restrict__ nrecs) {
+         int32_t *__restrict__ nrecs, const float4 *__restrict__ tq, const float4 *__restrict__ lc) {
     __shared__ Walk3Lds<A, F, TREE> L;
-    walk3_body<A, F, TREE, false>(pos, B, n, nL, h, rl2, cap, ncount, ctr, recs, nrecs, L,
-                                  xcd_block(blockIdx.x, gridDim.x), nullptr);
+    walk3_body<A, F, TREE, !TREE>(pos, B, n, nL, h, rl2, cap, ncount, ctr, recs, nrecs, L,
+                                  xcd_block(blockIdx.x, gridDim.x), nullptr, tq, lc);
 }
 
 // ---- neighbourhood tables ----
@@ -2567,7 +2569,7 @@ void launch_rebuild(nd_sim *s, bool full) {
             // dense workloads: the walk, then the table build with the larger
             // record buffer (its LDS would lower the walk's occupancy)
 #define ND_NLIST3(A, F, TREE) \
-    k_nlist3<A, F, TREE><<<g, nd::kBlock, 0, st>>>(p4, B, n, leaves, hl, rl2, s->cap, nc, ctr, rc, nr)
+    k_nlist3<A, F, TREE><<<g, nd::kBlock, 0, st>>>(p4, B, n, leaves, hl, rl2, s->cap, nc, ctr, rc, nr, tql, lcl)
             if (!tree && s->walk_split) {
                 ND_NLIST3(kSplitLeaf, kFront, false);
             } else if (!tree) {

@@ -48,7 +48,7 @@ class SimSpec:
     resort_every: int = 0
     list_walk: int = 0
     pair_batch: int = 0   # step kernel pipeline batch (0 = 4; FP32: 2, 4 or 8)
-    walk_front: int = 0   # two-phase walk records per round trip (0 = 8; or 16)
+    walk_front: int = 0   # two-phase walk over a tree (MIXED): records per round trip (0 = 8; or 16)
     atom_lanes: int = 0   # step kernel lanes per atom (0 = 1; or 2)
 
 
