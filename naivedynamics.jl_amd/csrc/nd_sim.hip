@@ -1506,10 +1506,12 @@ template <int A, int F, bool TREE>
 __global__ void __launch_bounds__(nd::kBlock, TREE ? 1 : 4)
 k_nlist3(const float4 *__restrict__ pos, WalkBoxes B, int32_t n, int32_t nL, float h, float rl2, int32_t cap,
          int32_t *__restrict__ ncount, int32_t *__restrict__ ctr, uint2 *__restrict__ recs,
-         int32_t *__restrict__ nrecs, const float4 *__restrict__ tq, const float4 *__restrict__ lc) {
+         int32_t *__restrict__ nrecs, const float4 *__restrict__ tq, const float4 *__restrict__ lc,
+         const int32_t *__restrict__ order, int32_t *__restrict__ work) {
     __shared__ Walk3Lds<A, F, TREE> L;
-    walk3_body<A, F, TREE, !TREE>(pos, B, n, nL, h, rl2, cap, ncount, ctr, recs, nrecs, L,
-                                  xcd_block(blockIdx.x, gridDim.x), nullptr, tq, lc);
+    int32_t blk = xcd_block(blockIdx.x, gridDim.x);
+    if (order != nullptr) blk = __builtin_amdgcn_readfirstlane(order[blk]);
+    walk3_body<A, F, TREE, !TREE>(pos, B, n, nL, h, rl2, cap, ncount, ctr, recs, nrecs, L, blk, work, tq, lc);
 }
 
 // ---- neighbourhood tables ----
@@ -2568,8 +2570,13 @@ void launch_rebuild(nd_sim *s, bool full) {
             }
             // dense workloads: the walk, then the table build with the larger
             // record buffer (its LDS would lower the walk's occupancy)
+            // placed by the work order where all workgroups are resident at once (96
+            // replicas, whose edges make heavy blocks: walk 150 -> 138 us)
+            const bool placed = !tree && (int32_t)g > 8 * s->cus_per_xcd && (int32_t)g <= 4 * 8 * s->cus_per_xcd;
+            const int32_t *ord = placed ? s->walk_order.as<int32_t>() : nullptr;
+            int32_t *wk = placed ? s->walk_work.as<int32_t>() : nullptr;
 #define ND_NLIST3(A, F, TREE) \
-    k_nlist3<A, F, TREE><<<g, nd::kBlock, 0, st>>>(p4, B, n, leaves, hl, rl2, s->cap, nc, ctr, rc, nr, tql, lcl)
+    k_nlist3<A, F, TREE><<<g, nd::kBlock, 0, st>>>(p4, B, n, leaves, hl, rl2, s->cap, nc, ctr, rc, nr, tql, lcl, ord, wk)
             if (!tree && s->walk_split) {
                 ND_NLIST3(kSplitLeaf, kFront, false);
             } else if (!tree) {
@@ -2591,6 +2598,7 @@ void launch_rebuild(nd_sim *s, bool full) {
             }
 #undef ND_NLIST3
             ND_HIP(hipGetLastError());
+            s->order_pending = placed;
             k_table_rec<kRecLdsBig><<<g, nd::kBlock, 0, st>>>(rc, nr, nc, n, s->cap, c2, s->lcap, es, n16, tb, tc,
                                                               nb, misc, s->hstale, si);
             ND_HIP(hipGetLastError());
