@@ -1172,6 +1172,7 @@ walk3_body(const float4 *__restrict__ pos, const WalkBoxes B, int32_t n, int32_t
            int32_t *__restrict__ nrecs, Walk3Lds<A, F, TREE, S> &L, int32_t blk, int32_t *__restrict__ work,
            const float4 *__restrict__ tq = nullptr, const float4 *__restrict__ lc = nullptr) {
     static_assert(A == 4 || A == 8 || A == 16 || A == 32, "leaf size");
+    static_assert(TREE || LOCAL, "a ragged last leaf is read from tq");
     constexpr int NV = (A + 7) / 8;      // atoms a lane stages per leaf (1, 2 or 4)
     constexpr int kSlot = Walk3Lds<A, F, TREE, S>::kSlot, kQ = Walk3Lds<A, F, TREE, S>::kQ;
     static_assert(S == 1 || (!TREE && (S & (S - 1)) == 0), "waves per 64 atoms");
@@ -1225,7 +1226,7 @@ walk3_body(const float4 *__restrict__ pos, const WalkBoxes B, int32_t n, int32_t
         // LOCAL: the leaf-local copies (-2 q', |q'|^2) and the leaf's
         // (centre, R^2), loaded with the atoms
         // (leaf form: the last leaf may hold fewer than A; its missing atoms
-        // are masked out of the hits, tq and pos have room for a leaf more)
+        // are masked out of the hits, and tq has room for them)
         const float4 *src = (LOCAL ? tq : pos) + (gl < A ? gl : 0);
         const float4 zero = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
         float4 v0 = zero, v1 = zero, v2 = zero, v3 = zero, cn = zero;
@@ -3217,12 +3218,12 @@ int nd_sim_create(nd_ctx *ctx, const nd_sim_params *p, nd_sim **out) {
         s->rlist = (float)(rl + (span + rl) * 9.5367431640625e-07);
         const size_t pb = pos_bytes(s), n = (size_t)s->n;
         for (int b = 0; b < 2; ++b) {
-            s->pos[b].reserve(pb + sizeof(float4) * kWalkLeaf);  // the walk reads whole leaves
+            s->pos[b].reserve(pb);
             s->vel[b].reserve(pb);
             s->orig[b].reserve(sizeof(int32_t) * n);
         }
         s->frc.reserve(pb);
-        if (s->wide) s->pos32.reserve(sizeof(float4) * (n + kWalkLeaf));
+        if (s->wide) s->pos32.reserve(sizeof(float4) * n);
         if (p->precision == ND_PREC_MIXED)
             for (int b = 0; b < 2; ++b) s->fix[b].reserve(sizeof(int4) * n);
         s->codes.reserve(sizeof(int32_t) * n);
@@ -3267,7 +3268,7 @@ int nd_sim_create(nd_ctx *ctx, const nd_sim_params *p, nd_sim **out) {
             for (int32_t b = 0; b < nb; ++b) iota[b] = b;
             s->walk_order.reserve(sizeof(int32_t) * (size_t)nb);
             s->walk_work.reserve(sizeof(int32_t) * 4 * (size_t)nb);
-            s->leaf_q.reserve(sizeof(float4) * ((size_t)s->n + kWalkLeaf));
+            s->leaf_q.reserve(sizeof(float4) * ((size_t)s->n + kWalkLeaf));  // the leaf form reads whole leaves
             s->leaf_c.reserve(sizeof(float4) * (size_t)std::max(s->nL, walk_leaves(s)));
             ND_HIP(hipMemcpyAsync(s->walk_order.p, iota.data(), sizeof(int32_t) * (size_t)nb,
                                   hipMemcpyHostToDevice, ctx->stream));
