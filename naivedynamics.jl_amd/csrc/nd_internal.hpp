@@ -258,7 +258,7 @@ struct PairSearch {
     float thr;              // accepted: s < thr
     float certain;          // s below this implies the walk's box test
 };
-// Smallest float whose correctly rounded square root is >= r (r normal, positive).
+// Smallest float whose correctly rounded square root is >= r (0 where r is not positive).
 float root_threshold(float r);
 // Counts per slot (half shell: per cell-sorted place) and, by atomic maximum,
 // the largest (maxcnt may be null).

@@ -884,6 +884,7 @@ __global__ void k_count_result(const int64_t *__restrict__ total, const int32_t 
 namespace nd {
 
 float root_threshold(float r) {
+    if (!(r > 0.0f)) return 0.0f;  // no root is below r
     // sqrt is monotonic: sqrt(s) < r for exactly the floats below this one
     float t = r * r;
     while (t > 0.0f && std::sqrt(t) >= r) t = std::nextafter(t, 0.0f);
