@@ -28,7 +28,8 @@
 // r there), and farther pairs' distances grow faster than their error while
 // |a| < 1e5 r.  A test inside +-E of a limit is redone by the exact one (some
 // 1e-5 of the tests), so the lists are the exact test's.  Where |a| or r leave
-// the range of this bound, E is infinite and every test is the exact one.
+// the range of this bound, E is not a number, neither limit decides and every
+// test is the exact one (|b|^2 may overflow there for a pair within the radius).
 //
 // Order.  The lists have to come in the order of a single-threaded reference
 // run, which is by place in the key order ("slot") of the later atom, not by
@@ -207,7 +208,7 @@ k_cell_search(PairArgs A) {
         const float a2 = __builtin_fmaf(az, az, __builtin_fmaf(ay, ay, ax * ax));
         const float reach = 2.0f * sqrtf(a2) + A.r;
         const bool bound = A.r >= 1e-15f && A.r <= 1e12f && reach < 1e5f * A.r;
-        const float E = bound ? 1.2e-6f * (reach * reach + A.r * A.r) : INFINITY;
+        const float E = bound ? 1.2e-6f * (reach * reach + A.r * A.r) : NAN;
         const float lo = (A.certain - a2) - E, hi = (A.thr - a2) + E;
         int32_t row_at = 0;  // row of the next batch's first candidate, or one before it
         for (int32_t s0 = 0; s0 < total; s0 += 64 * kBatches) {
