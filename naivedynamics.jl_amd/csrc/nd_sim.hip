@@ -1270,7 +1270,11 @@ walk3_body(const float4 *__restrict__ pos, const WalkBoxes B, int32_t n, int32_t
                     // the positions, so the list is the exact test's.
                     const float ax = p.x - cc.x, ay = p.y - cc.y, az = p.z - cc.z;
                     const float cp = __builtin_fmaf(az, az, __builtin_fmaf(ay, ay, __builtin_fmaf(ax, ax, -rl2)));
-                    const float E = 48.0f * 0x1p-24f * (cp + 2.0f * rl2 + cc.w);
+                    // Not finite (an atom thrown 1e19 out, in this leaf or this
+                    // lane): t may be infinite or not a number for a pair
+                    // inside the radius, so E is no number and all is redone.
+                    const float E0 = 48.0f * 0x1p-24f * (cp + 2.0f * rl2 + cc.w);
+                    const float E = E0 < 1e38f ? E0 : NAN;
                     uint64_t band = 0;
 #pragma unroll
                     for (int m = A - 1; m >= 0; --m) {
@@ -1281,7 +1285,7 @@ walk3_body(const float4 *__restrict__ pos, const WalkBoxes B, int32_t n, int32_t
                         // shifted in below the bits of atoms m + 1 .. A - 1 by one
                         // funnel shift, so atom m ends at bit m
                         hits = __builtin_amdgcn_alignbit(hits, __float_as_uint(t), 31);
-                        band |= __builtin_amdgcn_ballot_w64(fabsf(t) < E);
+                        band |= __builtin_amdgcn_ballot_w64(!(fabsf(t) >= E));
                     }
                     if (band != 0) {  // rare: a test within E of the radius
                         hits = 0u;
