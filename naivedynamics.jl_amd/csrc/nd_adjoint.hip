@@ -48,6 +48,7 @@
 // differentiation form of the simulate! hot path (Simulator.jl:154-256).
 #include <algorithm>
 #include <cmath>
+#include <cstring>
 #include <vector>
 
 #include "nd_internal.hpp"
@@ -193,6 +194,14 @@ k_adj_to_f32(const R *__restrict__ x, int32_t n, float4 *__restrict__ out) {
     if (i < n) out[i] = make_float4((float)x[i].x, (float)x[i].y, (float)x[i].z, 0.0f);
 }
 
+// What the list builds of a pass tell the host: the largest row, status bits,
+// and the largest row of the first build that had no room for one (if another
+// came after it).  A pass runs on with rows cut short and is repeated with longer
+// ones, so the builds after that one list another trajectory.
+struct ListFlags {
+    int32_t most, status, first, unused;
+};
+
 // Atom i goes to its place in the cells: the cell-sorted FP32 copy with its
 // number in the state's order, and (xo != null) the state into that order.
 template <class R>
@@ -200,9 +209,11 @@ __global__ void __launch_bounds__(nd::kBlock)
 k_adj_place(const float4 *__restrict__ x32, const int2 *__restrict__ cell_of, const int32_t *__restrict__ cells,
             int32_t n, float4 *__restrict__ cpos, int32_t *__restrict__ ckey, const R *__restrict__ x,
             const R *__restrict__ v, const int32_t *__restrict__ orig, const double *__restrict__ q,
-            R *__restrict__ xo, R *__restrict__ vo, int32_t *__restrict__ origo, double *__restrict__ qs) {
+            R *__restrict__ xo, R *__restrict__ vo, int32_t *__restrict__ origo, double *__restrict__ qs,
+            int32_t cap, ListFlags *__restrict__ flags) {
     const int32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
+    if (i == 0 && flags->most > cap && flags->first == 0) flags->first = flags->most;
     const int2 c = cell_of[i];
     const int32_t u = cells[c.x] + c.y;
     const float4 p = x32[i];
@@ -226,7 +237,7 @@ constexpr int kListAtoms = 8;
 __global__ void __launch_bounds__(nd::kBlock)
 k_adj_rows(const float4 *__restrict__ cpos, const int32_t *__restrict__ ckey, const int32_t *__restrict__ cells,
            const nd::CellGrid *__restrict__ grid, int32_t n, float rl2, int32_t cap, int32_t *__restrict__ lists,
-           int32_t *__restrict__ cnt, int32_t *__restrict__ most) {
+           int32_t *__restrict__ cnt, ListFlags *__restrict__ flags) {
     const int lane = threadIdx.x & 63;
     const int32_t t0 = __builtin_amdgcn_readfirstlane((int32_t)((blockIdx.x * blockDim.x + threadIdx.x) >> 6) * kListAtoms);
     if (t0 >= n) return;
@@ -311,7 +322,8 @@ k_adj_rows(const float4 *__restrict__ cpos, const int32_t *__restrict__ ckey, co
     if (lane < nt) cnt[pid] = found;
     int32_t mx = found;
     for (int o = 32; o > 0; o >>= 1) mx = max(mx, __shfl_xor(mx, o, 64));
-    if (lane == 0 && mx > __hip_atomic_load(most, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(most, mx);
+    if (lane == 0 && mx > __hip_atomic_load(&flags->most, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+        atomicMax(&flags->most, mx);
 }
 
 __device__ __forceinline__ double fix_val(unsigned long long v) { return (double)(long long)v * kInvFix; }
@@ -695,8 +707,8 @@ Rows rows_of(nd_adj *s, int32_t w) {
 
 int32_t *order_of(nd_adj *s, int32_t w) { return s->orig.as<int32_t>() + (size_t)s->order[w] * s->p.n; }
 
-// flags: [0] largest row, [1] status bits of the list builds since the last clear
-int32_t *flags_of(nd_adj *s) { return s->hist.as<int32_t>(); }
+// the list builds' flags, then the histogram
+ListFlags *flags_of(nd_adj *s) { return s->hist.as<ListFlags>(); }
 double *hist_of(nd_adj *s) { return s->hist.as<double>() + 2; }
 
 // Rows (and, move, the new order) of window w at the positions in s->x32.
@@ -707,10 +719,10 @@ void build_rows(nd_adj *s, int32_t w, const V *x, const V *v, const int32_t *ori
     const int32_t max_cells = std::max(27, n / 2);
     const float4 *x32 = s->x32.as<float4>();
     const nd::CellGrid *cg = nd::launch_cell_bins(st, s->bins.p, x32, n, s->rlist, max_cells, s->cell_of.as<int2>(),
-                                                  s->cells.as<int32_t>(), flags_of(s) + 1);
+                                                  s->cells.as<int32_t>(), &flags_of(s)->status);
     k_adj_place<V><<<nd::grid_for(n), nd::kBlock, 0, st>>>(
         x32, s->cell_of.as<int2>(), s->cells.as<int32_t>(), n, s->cpos.as<float4>(), s->ckey.as<int32_t>(), x, v, orig,
-        s->q.as<double>(), xo, vo, origo, s->qs.as<double>());
+        s->q.as<double>(), xo, vo, origo, s->qs.as<double>(), s->cap, flags_of(s));
     const Rows R = rows_of(s, w);
     k_adj_rows<<<nd::grid_for(((int64_t)n + kListAtoms - 1) / kListAtoms * 64), nd::kBlock, 0, st>>>(
         s->cpos.as<float4>(), s->ckey.as<int32_t>(), s->cells.as<int32_t>(), cg, n, s->rlist * s->rlist, s->cap,
@@ -774,12 +786,25 @@ void advance(nd_adj *s, int32_t k0, int32_t k1, bool forward, bool finish_first,
     }
 }
 
-// Reads the flags; throws what the list builds found.  Returns the largest row.
-int32_t check_flags(const int32_t *h) {
-    if (h[1] & nd::kStatusDomain) throw nd::Error(ND_ERR_DOMAIN, "adjoint: non-finite coordinate");
-    // (the list build took one grid row per list row)
-    if (h[0] > 65535) throw nd::Error(ND_ERR_CAPACITY, "adjoint: more than 65,535 neighbours per atom");
-    return h[0];
+// Longer rows are refused: at this length one list of a million atoms takes 262 GB.
+constexpr int32_t kMaxRow = 65535;
+
+// Whether the builds so far had room, which is made if not (the pass has to be
+// repeated); throws what else they found.  The largest row of a pass that ran on
+// without room says how much denser the system is about to get, but no more:
+// without their repulsion atoms gather (32,768 atoms moving inwards, rows of at
+// most 275: rows of 1,800 counted), so four times the last row known to be right
+// is the most that is made for.
+bool had_room(nd_adj *s, const ListFlags &f) {
+    if (f.most <= s->cap) {
+        if (f.status & nd::kStatusDomain) throw nd::Error(ND_ERR_DOMAIN, "adjoint: non-finite coordinate");
+        return true;
+    }
+    const int32_t right = f.first > 0 ? f.first : f.most;
+    if (right > kMaxRow) throw nd::Error(ND_ERR_CAPACITY, "adjoint: more than 65,535 neighbours per atom");
+    s->cap = std::min(std::min(f.most + f.most / 4, 4 * right) + 8, s->p.n);
+    reserve_rows(s);
+    return false;
 }
 
 template <class T>
@@ -789,26 +814,25 @@ void forward_impl(nd_adj *s) {
     const int32_t K = s->p.checkpoint_every, T_ = s->p.nsteps, n = s->p.n, nb = s->p.nbins;
     const size_t vb = sizeof(V) * (size_t)n, ib = sizeof(int32_t) * (size_t)n;
     std::vector<double> h(2 + nb);
-    const int32_t *hf = reinterpret_cast<const int32_t *>(h.data());
-    for (int attempt = 0;; ++attempt) {
-        if (attempt == 8) throw nd::Error(ND_ERR_CAPACITY, "adjoint: neighbour rows kept overflowing");
-        auto grow = [&](int32_t most) {
-            s->cap = most + most / 4 + 8;
-            reserve_rows(s);
-        };
-        nd::launch_fill_i32(st, flags_of(s), 4, 0);
+    static_assert(sizeof(ListFlags) == 2 * sizeof(double), "flags before the histogram");
+    auto flags = [&] {
+        ListFlags f;
+        std::memcpy(&f, h.data(), sizeof f);
+        return f;
+    };
+    // every further attempt has longer rows and gets past the build that ended
+    // the one before
+    for (;;) {
+        nd::launch_fill_i32(st, reinterpret_cast<int32_t *>(flags_of(s)), 4, 0);
         s->vcur = 0;
         k_adj_init<T><<<nd::grid_for(n), nd::kBlock, 0, st>>>(
             s->x0.as<double>(), s->v0.as<double>(), s->q.as<double>(), n, s->tmp.as<V>(), s->vel[0].as<V>(),
             s->x32.as<float4>(), order_of(s, s->nwin - 2));
         build_list<T>(s, 0, s->order[s->nwin - 2], seg_at<T>(s, 0));
         // room for the first list is made before the steps run on it
-        ND_HIP(hipMemcpyAsync(h.data(), s->hist.p, 8, hipMemcpyDeviceToHost, st));
+        ND_HIP(hipMemcpyAsync(h.data(), s->hist.p, sizeof(ListFlags), hipMemcpyDeviceToHost, st));
         ND_HIP(hipStreamSynchronize(st));
-        if (const int32_t most = check_flags(hf); most > s->cap) {
-            grow(most);
-            continue;
-        }
+        if (!had_room(s, flags())) continue;
         for (int32_t c = 0; c * K < T_; ++c) {
             const int32_t k0 = c * K, k1 = std::min((c + 1) * K, T_);
             V *vck = nullptr;
@@ -829,9 +853,7 @@ void forward_impl(nd_adj *s) {
         ND_HIP(hipGetLastError());
         ND_HIP(hipMemcpyAsync(h.data(), s->hist.p, sizeof(double) * h.size(), hipMemcpyDeviceToHost, st));
         ND_HIP(hipStreamSynchronize(st));
-        const int32_t most = check_flags(hf);
-        if (most <= s->cap) break;
-        grow(most);  // a later list overflowed: its forces were short
+        if (had_room(s, flags())) break;
     }
     s->rdf.resize(nb);
     s->loss = 0.0;
