@@ -27,7 +27,8 @@
 // Atoms are kept in the order of the last list build, which is the order of
 // the cells (side >= list radius) it searches: a neighbour gather then reads
 // aligned records (position, and in FP64 the charge) that lie near each other,
-// and the build needs no tree.  kRowLanes lanes share an atom's row of the list:
+// and the build needs no tree.  Systems whose clusters lie far apart take cells
+// that do not depend on the extent (BinGrid's lines).  kRowLanes lanes share an atom's row of the list:
 // at N = 32,768 one lane per atom leaves two waves per CU, and a row is a chain
 // of dependent loads.  One launch makes a step: the pair sums of x_k, the half
 // kick that ends step k - 1 and the half kick and drift of step k; in the
@@ -197,10 +198,19 @@ k_adj_to_f32(const R *__restrict__ x, int32_t n, float4 *__restrict__ out) {
 // What the list builds of a pass tell the host: the largest row, status bits,
 // and the largest row of the first build that had no room for one (if another
 // came after it).  A pass runs on with rows cut short and is repeated with longer
-// ones, so the builds after that one list another trajectory.
+// ones, so the builds after that one list another trajectory.  lines: the last
+// list is, or has to be, built over lines of cells (BinGrid).
 struct ListFlags {
-    int32_t most, status, first, unused;
+    int32_t most, status, first, lines;
 };
+
+// Tests an atom, above which a box's cells count as crowded and lines are taken.
+// Forward passes of 20 steps (three lists) over two droplets at growing distance
+// or with an atom far out, by tests: 32,768 atoms 832 / 892 / 1,094 / 1,875 /
+// 4,312 / 16,384: 649 / 669 / 683 / 790 / 1,172 / 1,902 us with the box's cells,
+// 687 / 668 / 692 / 690 / 688 / 700 with lines; 8,192 atoms 824 / 1,328: 519 / 602
+// and 565 / 533.  262,144 atoms, 75,173 tests: 24.5 ms and 2.2.  (A liquid: 480-560.)
+constexpr double kCrowded = 1200.0;
 
 // Atom i goes to its place in the cells: the cell-sorted FP32 copy with its
 // number in the state's order, and (xo != null) the state into that order.
@@ -210,10 +220,13 @@ k_adj_place(const float4 *__restrict__ x32, const int2 *__restrict__ cell_of, co
             int32_t n, float4 *__restrict__ cpos, int32_t *__restrict__ ckey, const R *__restrict__ x,
             const R *__restrict__ v, const int32_t *__restrict__ orig, const double *__restrict__ q,
             R *__restrict__ xo, R *__restrict__ vo, int32_t *__restrict__ origo, double *__restrict__ qs,
-            int32_t cap, ListFlags *__restrict__ flags) {
+            int32_t cap, const nd::BinGrid *__restrict__ grid, ListFlags *__restrict__ flags) {
     const int32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
-    if (i == 0 && flags->most > cap && flags->first == 0) flags->first = flags->most;
+    if (i == 0) {
+        if (flags->most > cap && flags->first == 0) flags->first = flags->most;
+        flags->lines = grid->lines > 0 || (double)grid->tests > kCrowded * n;
+    }
     const int2 c = cell_of[i];
     const int32_t u = cells[c.x] + c.y;
     const float4 p = x32[i];
@@ -231,19 +244,27 @@ k_adj_place(const float4 *__restrict__ x32, const int2 *__restrict__ cell_of, co
 // each in both rows.  A wave takes kListAtoms consecutive atoms in groups of
 // one cell row (k cells of about two dozen atoms): a batch of 64 candidates
 // from the nine rows of cells around the group is tested against its atoms one
-// after another, and a ballot places the hits.
+// after another, and a ballot places the hits.  LINES: the cells are those of
+// lines on a circle; a run of a line is two runs of the table where it passes
+// the circle's end, and a candidate counts only in the run of its own line.
 constexpr int kListAtoms = 8;
+constexpr int kLineCells = 4;  // cells a group may lie in
 
+template <bool LINES>
 __global__ void __launch_bounds__(nd::kBlock)
 k_adj_rows(const float4 *__restrict__ cpos, const int32_t *__restrict__ ckey, const int32_t *__restrict__ cells,
-           const nd::CellGrid *__restrict__ grid, int32_t n, float rl2, int32_t cap, int32_t *__restrict__ lists,
+           const nd::BinGrid *__restrict__ grid, int32_t n, float rl2, int32_t cap, int32_t *__restrict__ lists,
            int32_t *__restrict__ cnt, ListFlags *__restrict__ flags) {
     const int lane = threadIdx.x & 63;
     const int32_t t0 = __builtin_amdgcn_readfirstlane((int32_t)((blockIdx.x * blockDim.x + threadIdx.x) >> 6) * kListAtoms);
-    if (t0 >= n) return;
+    const int32_t lines = grid->lines;
+    // (cells found crowded: no rows, the host asks for lines)
+    if (t0 >= n || LINES != (flags->lines != 0)) return;
+    constexpr int RUNS = LINES ? 18 : 9;
     const int32_t nt = min(kListAtoms, n - t0);
-    const int32_t g0 = grid->g[0], g1 = grid->g[1], g2 = grid->g[2];
-    const int32_t k = max(1, (int32_t)(24.0f * (float)grid->ncell / (float)n));
+    const int32_t g0 = grid->cg.g[0], g1 = grid->cg.g[1], g2 = grid->cg.g[2];
+    const int32_t k = LINES ? kLineCells : max(1, (int32_t)(24.0f * (float)grid->cg.ncell / (float)n));
+    const double inv = grid->inv;
     float px = 0.0f, py = 0.0f, pz = 0.0f;
     int32_t pk = -1, pid = 0, found = 0;
     if (lane < nt) {
@@ -254,18 +275,41 @@ k_adj_rows(const float4 *__restrict__ cpos, const int32_t *__restrict__ ckey, co
         pid = __float_as_int(p.w);
         pk = ckey[t0 + lane];
     }
-    const int32_t prow = pk / g0;
+    const int32_t prow = LINES ? 0 : pk / g0;
+    const double py_ = LINES ? nd::line_coord(inv, py) : 0.0, pz_ = LINES ? nd::line_coord(inv, pz) : 0.0;
     auto lf = [](float v, int l) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l)); };
     int32_t q0 = 0;
     while (q0 < nt) {
         const int32_t k0 = __builtin_amdgcn_readlane(pk, q0), row = __builtin_amdgcn_readlane(prow, q0);
-        const uint64_t in = __builtin_amdgcn_ballot_w64(lane >= q0 && lane < nt && prow == row && pk < k0 + k);
-        const int32_t q1 = q0 + __builtin_popcountll(in);
-        const int32_t c0 = k0 - row * g0, c1 = __builtin_amdgcn_readlane(pk, q1 - 1) - row * g0;
+        const double y0 = LINES ? __shfl(py_, q0, 64) : 0.0, z0 = LINES ? __shfl(pz_, q0, 64) : 0.0;
+        // q0 and the atoms after it up to the first of another row or beyond k cells
+        const bool same = LINES ? lane == q0 || (py_ == y0 && pz_ == z0) : prow == row;
+        const uint64_t in = __builtin_amdgcn_ballot_w64(lane >= q0 && lane < nt && same && pk < k0 + k);
+        const int32_t q1 = q0 + (LINES ? __builtin_ctzll(~(in >> q0)) : __builtin_popcountll(in));
+        const int32_t k1 = __builtin_amdgcn_readlane(pk, q1 - 1);
+        const int32_t c0 = k0 - row * g0, c1 = k1 - row * g0;
         const int32_t cy = row % g1, cz = row / g1;
-        // lane j < 9: the run of cell row j around the group
+        // lane j: the run of cell row j around the group (lines: 9 + j its rest
+        // beyond the end of the table), and the row's cell
         int32_t from = 0, to = 0;
-        if (lane < 9) {
+        double ry = 0.0, rz = 0.0;
+        if (LINES && lane < RUNS) {
+            const int32_t dy = lane % 9 % 3 - 1, dz = lane % 9 / 3 - 1, span = k1 - k0 + 3;
+            ry = y0 + dy;
+            rz = z0 + dz;
+            // (cells so far out that one more is the same number have no others beside them)
+            if ((dy == 0 || ry != y0) && (dz == 0 || rz != z0)) {
+                int32_t at = (k0 - 1 + nd::line_start(ry, rz, lines) - nd::line_start(y0, z0, lines)) % lines;
+                if (at < 0) at += lines;
+                if (lane < 9) {
+                    from = cells[at];
+                    to = cells[min(at + span, lines)];
+                } else if (at + span > lines) {
+                    to = cells[at + span - lines];
+                }
+            }
+        }
+        if (!LINES && lane < RUNS) {
             const int32_t y = cy + lane % 3 - 1, z = cz + lane / 3 - 1;
             if (y >= 0 && y < g1 && z >= 0 && z < g2) {
                 const int32_t b = (z * g1 + y) * g0;
@@ -277,33 +321,41 @@ k_adj_rows(const float4 *__restrict__ cpos, const int32_t *__restrict__ ckey, co
         // start less those
         int32_t pre = to - from;
 #pragma unroll
-        for (int o = 1; o < 16; o <<= 1) {
+        for (int o = 1; o < RUNS; o <<= 1) {
             const int32_t v = __shfl_up(pre, o, 64);
             if (lane >= o) pre += v;
         }
-        const int32_t total = __builtin_amdgcn_readlane(pre, 8);
+        const int32_t total = __builtin_amdgcn_readlane(pre, RUNS - 1);
         pre -= to - from;
         const int32_t rise = from - pre;
         int32_t at_run = 0;
-        auto fetch = [&](int32_t s0, int32_t &u) {
+        // run: of each lane's candidate
+        auto fetch = [&](int32_t s0, int32_t &u, int32_t &run) {
             const int32_t ci = s0 + lane;
             u = ci + __builtin_amdgcn_readlane(rise, at_run);
-            while (at_run < 8) {
+            run = at_run;
+            while (at_run < RUNS - 1) {
                 const int32_t p = __builtin_amdgcn_readlane(pre, at_run + 1);
                 if (p > s0 + 63) break;
                 ++at_run;
                 u = ci >= p ? ci + __builtin_amdgcn_readlane(rise, at_run) : u;
+                run = ci >= p ? at_run : run;
             }
             if (ci >= total) u = -1;
             return cpos[u < 0 ? t0 : u];
         };
-        int32_t un;
-        float4 c = fetch(0, un);
+        int32_t un, rn;
+        float4 c = fetch(0, un, rn);
         for (int32_t s0 = 0; s0 < total; s0 += 64) {
             // the next batch is on its way while this one is tested
-            const int32_t u = un;
+            int32_t u = un;
+            const int32_t run = rn;
             const float4 d = c;
-            if (s0 + 64 < total) c = fetch(s0 + 64, un);
+            if (s0 + 64 < total) c = fetch(s0 + 64, un, rn);
+            if (LINES) {  // atoms of other lines in the same table cells
+                const double wy = __shfl(ry, run, 64), wz = __shfl(rz, run, 64);
+                if (nd::line_coord(inv, d.y) != wy || nd::line_coord(inv, d.z) != wz) u = -1;
+            }
             for (int32_t q = q0; q < q1; ++q) {
                 const float dx = d.x - lf(px, q), dy = d.y - lf(py, q), dz = d.z - lf(pz, q);
                 const bool hit = (dx * dx + dy * dy + dz * dz < rl2) & (u >= 0) & (u != t0 + q);
@@ -678,6 +730,7 @@ struct nd_adj {
     std::vector<int32_t> order;    // index of each window's order in orig
     int32_t spare = 0;             // index of the unused order
     nd::DevBuf bins, cell_of, cells, cpos, ckey;  // list build
+    nd::BinMode bin_mode = nd::kBinBox;           // the cells of the pass, chosen at its first list
     nd::DevBuf lam, lam_caller, dq, dpar, out, hist, part, wb;
     int32_t cap = 0;  // row capacity
     bool have_forward = false;
@@ -713,19 +766,22 @@ double *hist_of(nd_adj *s) { return s->hist.as<double>() + 2; }
 
 // Rows (and, move, the new order) of window w at the positions in s->x32.
 template <class V>
-void build_rows(nd_adj *s, int32_t w, const V *x, const V *v, const int32_t *orig, V *xo, V *vo, int32_t *origo) {
+void build_rows(nd_adj *s, int32_t w, nd::BinMode mode, const V *x, const V *v, const int32_t *orig, V *xo, V *vo,
+                int32_t *origo) {
     hipStream_t st = s->ctx->stream;
     const int32_t n = s->p.n;
     const int32_t max_cells = std::max(27, n / 2);
     const float4 *x32 = s->x32.as<float4>();
-    const nd::CellGrid *cg = nd::launch_cell_bins(st, s->bins.p, x32, n, s->rlist, max_cells, s->cell_of.as<int2>(),
-                                                  s->cells.as<int32_t>(), &flags_of(s)->status);
+    const nd::BinGrid *grid = nd::launch_cell_bins(st, s->bins.p, x32, n, s->rlist, max_cells, mode,
+                                                   kCrowded, s->cell_of.as<int2>(), s->cells.as<int32_t>(),
+                                                   &flags_of(s)->status);
     k_adj_place<V><<<nd::grid_for(n), nd::kBlock, 0, st>>>(
         x32, s->cell_of.as<int2>(), s->cells.as<int32_t>(), n, s->cpos.as<float4>(), s->ckey.as<int32_t>(), x, v, orig,
-        s->q.as<double>(), xo, vo, origo, s->qs.as<double>(), s->cap, flags_of(s));
+        s->q.as<double>(), xo, vo, origo, s->qs.as<double>(), s->cap, grid, flags_of(s));
     const Rows R = rows_of(s, w);
-    k_adj_rows<<<nd::grid_for(((int64_t)n + kListAtoms - 1) / kListAtoms * 64), nd::kBlock, 0, st>>>(
-        s->cpos.as<float4>(), s->ckey.as<int32_t>(), s->cells.as<int32_t>(), cg, n, s->rlist * s->rlist, s->cap,
+    const auto rows = mode == nd::kBinLines ? k_adj_rows<true> : k_adj_rows<false>;
+    rows<<<nd::grid_for(((int64_t)n + kListAtoms - 1) / kListAtoms * 64), nd::kBlock, 0, st>>>(
+        s->cpos.as<float4>(), s->ckey.as<int32_t>(), s->cells.as<int32_t>(), grid, n, s->rlist * s->rlist, s->cap,
         const_cast<int32_t *>(R.lists), const_cast<int32_t *>(R.cnt), flags_of(s));
     ND_HIP(hipGetLastError());
     s->holds[slot_of(s, w)] = w;
@@ -734,12 +790,12 @@ void build_rows(nd_adj *s, int32_t w, const V *x, const V *v, const int32_t *ori
 // The list of window w for the positions in s->tmp (order from): moves the
 // state into its order, the positions to xo.
 template <class T>
-void build_list(nd_adj *s, int32_t w, int32_t from, typename V4<T>::R *xo) {
+void build_list(nd_adj *s, int32_t w, int32_t from, typename V4<T>::R *xo, nd::BinMode mode) {
     using V = typename V4<T>::R;
     int32_t *orig = s->orig.as<int32_t>();
     const size_t n = (size_t)s->p.n;
     const int32_t src = from, dst = s->spare;
-    build_rows<V>(s, w, s->tmp.as<V>(), s->vel[s->vcur].as<V>(), orig + (size_t)src * n, xo,
+    build_rows<V>(s, w, mode, s->tmp.as<V>(), s->vel[s->vcur].as<V>(), orig + (size_t)src * n, xo,
                   s->vel[s->vcur ^ 1].as<V>(), orig + (size_t)dst * n);
     s->vcur ^= 1;
     // the order window w had before is free now
@@ -781,8 +837,8 @@ void advance(nd_adj *s, int32_t k0, int32_t k1, bool forward, bool finish_first,
         V *xo = build ? s->tmp.as<V>() : seg_at<T>(s, k + 1 - k0);
         launch_step<T>(s, w, seg_at<T>(s, k - k0), k > k0 || finish_first, k == k0 ? vck : nullptr, xo, build);
         if (!build) continue;
-        if (k + 1 == T_) build_list<T>(s, s->nwin - 2, s->order[w], s->xT.as<V>());
-        else build_list<T>(s, end ? 0 : w + 1, s->order[w], seg_at<T>(s, end ? 0 : k + 1 - k0));
+        if (k + 1 == T_) build_list<T>(s, s->nwin - 2, s->order[w], s->xT.as<V>(), s->bin_mode);
+        else build_list<T>(s, end ? 0 : w + 1, s->order[w], seg_at<T>(s, end ? 0 : k + 1 - k0), s->bin_mode);
     }
 }
 
@@ -820,18 +876,23 @@ void forward_impl(nd_adj *s) {
         std::memcpy(&f, h.data(), sizeof f);
         return f;
     };
-    // every further attempt has longer rows and gets past the build that ended
-    // the one before
+    // the first list says which cells the pass takes; every attempt after that has
+    // longer rows and gets past the build that ended the one before
+    s->bin_mode = nd::kBinCount;
     for (;;) {
         nd::launch_fill_i32(st, reinterpret_cast<int32_t *>(flags_of(s)), 4, 0);
         s->vcur = 0;
         k_adj_init<T><<<nd::grid_for(n), nd::kBlock, 0, st>>>(
             s->x0.as<double>(), s->v0.as<double>(), s->q.as<double>(), n, s->tmp.as<V>(), s->vel[0].as<V>(),
             s->x32.as<float4>(), order_of(s, s->nwin - 2));
-        build_list<T>(s, 0, s->order[s->nwin - 2], seg_at<T>(s, 0));
+        build_list<T>(s, 0, s->order[s->nwin - 2], seg_at<T>(s, 0), s->bin_mode);
         // room for the first list is made before the steps run on it
         ND_HIP(hipMemcpyAsync(h.data(), s->hist.p, sizeof(ListFlags), hipMemcpyDeviceToHost, st));
         ND_HIP(hipStreamSynchronize(st));
+        if (s->bin_mode == nd::kBinCount) {
+            s->bin_mode = flags().lines ? nd::kBinLines : nd::kBinBox;
+            if (s->bin_mode == nd::kBinLines) continue;
+        }
         if (!had_room(s, flags())) continue;
         for (int32_t c = 0; c * K < T_; ++c) {
             const int32_t k0 = c * K, k1 = std::min((c + 1) * K, T_);
@@ -898,7 +959,7 @@ void backward_impl(nd_adj *s) {
             ND_HIP(hipMemcpyAsync(order_of(s, fin), s->ck_orig.as<int32_t>() + (size_t)c * n, ib,
                                   hipMemcpyDeviceToDevice, st));
             k_adj_to_f32<V><<<g, nd::kBlock, 0, st>>>(s->tmp.as<V>(), n, s->x32.as<float4>());
-            build_list<T>(s, 0, s->order[fin], seg_at<T>(s, 0));
+            build_list<T>(s, 0, s->order[fin], seg_at<T>(s, 0), s->bin_mode);
             advance<T>(s, k0, k1, false, false, nullptr);
         }
         int32_t win = -1;
@@ -911,7 +972,7 @@ void backward_impl(nd_adj *s) {
                 if (s->holds[slot_of(s, w)] != w) {
                     // rows not kept: listed again for the window's first positions, in its order
                     k_adj_to_f32<V><<<g, nd::kBlock, 0, st>>>(seg_at<T>(s, w * W), n, s->x32.as<float4>());
-                    build_rows<V>(s, w, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr);
+                    build_rows<V>(s, w, s->bin_mode, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr);
                 }
                 win = w;
             }

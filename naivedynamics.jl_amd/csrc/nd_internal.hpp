@@ -231,14 +231,28 @@ enum : int32_t { kPairsLeaf = 0, kPairsPointOwn = 1, kPairsPointRoot = 2, kPairs
 // is <= cap).  Synchronous.
 int64_t tree_list(nd_ctx *ctx, const float *d_xyz, int32_t kind, int32_t n, int32_t apl, float r, int32_t pred,
                   int32_t morton, nd_pair *d_out, int64_t cap);
-// Atoms into cells of side >= r (at most max_cells), kernels only: cell and
+// The cells of launch_cell_bins: those of a box (lines 0) or, where clusters lie
+// so far apart that a box's cells would be large and crowded, cells of side just
+// over r in all space.  There a line of cells (one y and z) starts at its own
+// pseudo-random place on a circle of `lines` table cells, so atoms r apart are
+// in table cells that follow from each other's, whatever the extent; a table cell
+// can hold atoms of several lines, which a reader tells apart by their y and z.
+struct BinGrid {
+    CellGrid cg;
+    double inv;                // 1 / side of the lines' cells
+    int32_t lines;             // table cells (0: the box's cells)
+    unsigned long long tests;  // kBinCount, where smaller cells would do: pairs of atoms in cells beside each other
+};
+enum BinMode : int32_t { kBinBox = 0, kBinLines = 1, kBinCount = 2 };
+// Atoms into cells of side >= r (at most max_cells >= 27), kernels only: cell and
 // place of each in cell_of, first place of each cell in cells (max_cells + 1
-// ints; cells[ncell] = n), kStatusDomain into *status for a non-finite
-// coordinate.  work: cell_bins_bytes() of device memory.  Returns the grid's
-// device address.
+// ints; cells[cell count] = n), kStatusDomain into *status for a non-finite
+// coordinate.  kBinCount is kBinBox with the tests counted where
+// there may be more than `few` an atom.
+// work: cell_bins_bytes() of device memory.  Returns the grid's device address.
 size_t cell_bins_bytes();
-const CellGrid *launch_cell_bins(hipStream_t st, void *work, const float4 *x, int32_t n, float r, int32_t max_cells,
-                                 int2 *cell_of, int32_t *cells, int32_t *status);
+const BinGrid *launch_cell_bins(hipStream_t st, void *work, const float4 *x, int32_t n, float r, int32_t max_cells,
+                                BinMode mode, double few, int2 *cell_of, int32_t *cells, int32_t *status);
 // Bounding box of the atoms with finite coordinates; false if there are none.
 // Synchronous.
 bool atoms_box(nd_ctx *ctx, const float *d_xyz, int32_t n, double lo[3], double hi[3]);
@@ -268,6 +282,26 @@ void launch_pair_count(hipStream_t st, const PairSearch &S, int64_t *counts, int
 bool pair_emit_fits(int32_t kind, int32_t apl, int32_t maxcnt);
 // Pairs at the exclusive offsets of the counts.
 void launch_pair_emit(hipStream_t st, const PairSearch &S, const int64_t *offsets, int32_t maxcnt, nd_pair *out);
+
+// A line's cell of a coordinate (whole, -0 as 0).
+__device__ __forceinline__ double line_coord(double inv, float x) { return floor((double)x * inv) + 0.0; }
+// Place of the line at (y, z) on a circle of m table cells: the words multiplied
+// and folded, so that the upper half depends on all their bits.
+__device__ __forceinline__ int32_t line_start(double y, double z, int32_t m) {
+    const uint64_t k = 0x9E3779B97F4A7C15ull;  // 2^64 / the golden ratio, odd
+    uint64_t u = (uint64_t)__double_as_longlong(y) * k + (uint64_t)__double_as_longlong(z);
+    u = (u ^ (u >> 32)) * k;
+    u = (u ^ (u >> 32)) * k;
+    return (int32_t)(((u >> 32) * (uint64_t)m) >> 32);
+}
+// Table cell of cell x of a line: exact for any finite x; the first of the line
+// where x is not finite.
+__device__ __forceinline__ int32_t line_cell(double x, double y, double z, int32_t m) {
+    const double q = fmod(x, (double)m);
+    int32_t at = line_start(y, z, m);
+    if (q == q) at += (int32_t)q + (q < 0.0 ? m : 0);
+    return at >= m ? at - m : at;
+}
 
 __device__ __forceinline__ int32_t cell_coord(const CellGrid &cg, float x, int d) {
     const double t = ((double)x - cg.lo[d]) * cg.inv[d];

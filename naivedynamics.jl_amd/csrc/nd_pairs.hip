@@ -451,7 +451,8 @@ k_merge_leaf(const int64_t *__restrict__ offsets, const int32_t *__restrict__ id
 // Keys' bits that vary, cells' crowding and the grid, for the host's one
 // decision before the sort.
 struct Prep {
-    nd::CellGrid cg;
+    nd::BinGrid grid;
+    int32_t stretched;  // cells larger than they need to be, or atoms outside the grid
     float certain;
     int32_t status;
     uint32_t key_or, key_and;
@@ -587,7 +588,8 @@ k_box_result(const BoxPart *__restrict__ part, int32_t nparts, int32_t *__restri
 // The grid spans four standard deviations around the mean where that is less
 // than the bounding box: coordinates outside go to the edge cells, which keeps
 // atoms within a cell's side in neighbouring cells, and a few outliers do not
-// stretch the cells of all others.
+// stretch the cells of all others (far clusters do: the lists over a tree walk it
+// then, the adjoint's take lines).
 __global__ void __launch_bounds__(nd::kBlock)
 k_prep_grid(const BoxPart *__restrict__ part, int32_t nparts, int32_t n, float r, float thr, int32_t max_cells,
             float *__restrict__ box, Prep *__restrict__ prep) {
@@ -622,6 +624,7 @@ k_prep_grid(const BoxPart *__restrict__ part, int32_t nparts, int32_t n, float r
     int64_t g[3];
     double lo[3], ext[3];
     float most = 0.0f;
+    bool stretched = false;
     const double side = (double)r * (1.0 + 1e-4);
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
@@ -643,9 +646,11 @@ k_prep_grid(const BoxPart *__restrict__ part, int32_t nparts, int32_t n, float r
         ext[d] = a <= b ? fmin((double)h, mean + dev) - lo[d] : 0.0;
         const double q = ext[d] > 0.0 ? floor(ext[d] / side) : 1.0;
         g[d] = q >= 1.0 ? (q > 1024.0 ? 1024 : (int64_t)q) : 1;
+        stretched |= q > 1024.0 || (a <= b && ((double)l < lo[d] || lo[d] + ext[d] < (double)h));
         if (a <= b) most = fmaxf(most, fmaxf(fabsf(l), fabsf(h)));
     }
     while (g[0] * g[1] * g[2] > max_cells) {
+        stretched = true;
         const double f = cbrt((double)max_cells / (double)(g[0] * g[1] * g[2]));
 #pragma unroll
         for (int d = 0; d < 3; ++d) {
@@ -660,7 +665,11 @@ k_prep_grid(const BoxPart *__restrict__ part, int32_t nparts, int32_t n, float r
         cg.inv[d] = ext[d] > 0.0 ? (double)g[d] / ext[d] : 0.0;
     }
     cg.ncell = (int32_t)(g[0] * g[1] * g[2]);
-    prep->cg = cg;
+    prep->grid.cg = cg;
+    prep->grid.lines = 0;
+    prep->grid.tests = 0ull;
+    prep->grid.inv = 1.0 / side;
+    prep->stretched = stretched;
     const double in = (double)r * (1.0 - 0x1p-20) - 0x1p-22 * ((double)most + (double)r);
     prep->certain = in > 0.0 ? fminf((float)(in * in * (1.0 - 0x1p-20)), thr) : -1.0f;
 }
@@ -689,16 +698,29 @@ __device__ __forceinline__ int32_t cell_index(const nd::CellGrid &cg, float x, f
     return (nd::cell_coord(cg, z, 2) * cg.g[1] + nd::cell_coord(cg, y, 1)) * cg.g[0] + nd::cell_coord(cg, x, 0);
 }
 
+// Lines without a look at the atoms' box.
+__global__ void k_line_grid(float r, int32_t lines, Prep *__restrict__ prep) {
+    prep->grid.lines = lines;
+    prep->grid.tests = 0ull;
+    prep->grid.inv = 1.0 / ((double)r * (1.0 + 1e-4));
+}
+
 // Cell and place of every atom.
 __global__ void __launch_bounds__(nd::kBlock)
 k_bin_atoms(const float4 *__restrict__ x, int32_t n, const Prep *__restrict__ prep, int32_t *__restrict__ cells,
             int2 *__restrict__ cell_of, int32_t *__restrict__ status) {
-    const int32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    const int32_t i = blockIdx.x * blockDim.x + threadIdx.x, lines = prep->grid.lines;
     if (i >= n) return;
     const float4 p = x[i];
     if (!(__builtin_isfinite(p.x) && __builtin_isfinite(p.y) && __builtin_isfinite(p.z)))
         atomicOr(status, nd::kStatusDomain);
-    const int32_t c = cell_index(prep->cg, p.x, p.y, p.z);
+    int32_t c;
+    if (lines) {
+        const double inv = prep->grid.inv;
+        c = nd::line_cell(nd::line_coord(inv, p.x), nd::line_coord(inv, p.y), nd::line_coord(inv, p.z), lines);
+    } else {
+        c = cell_index(prep->grid.cg, p.x, p.y, p.z);
+    }
     cell_of[i] = make_int2(c, count_in_cell(cells, c));
 }
 
@@ -724,7 +746,7 @@ k_prep_keys(const float *__restrict__ xyz, int32_t n, const float *__restrict__ 
         codes[i] = code;
         perm[i] = i;
         if (!ok) atomicOr(status, nd::kStatusDomain);
-        const int32_t c = cell_index(prep->cg, x, y, z);
+        const int32_t c = cell_index(prep->grid.cg, x, y, z);
         const int32_t place = count_in_cell(cells, c);
         cell_of[i] = make_int2(c, place);
         const uint32_t k = (uint32_t)code ^ 0x80000000u;
@@ -738,13 +760,33 @@ k_prep_keys(const float *__restrict__ xyz, int32_t n, const float *__restrict__ 
     }
 }
 
-// Sum and sum of squares of each tile of cell counts.
+__device__ __forceinline__ int32_t table_cells(const nd::BinGrid &g) { return g.lines ? g.lines : g.cg.ncell; }
+
+// Atoms in the cells around cell c of a box, itself included.
+__device__ __forceinline__ int32_t atoms_around(const int32_t *__restrict__ cells, const nd::CellGrid &cg, int32_t c) {
+    const int32_t g0 = cg.g[0], g1 = cg.g[1], g2 = cg.g[2];
+    const int32_t x = c % g0, y = c / g0 % g1, z = c / g0 / g1;
+    int32_t sum = 0;
+#pragma unroll
+    for (int k = 0; k < 27; ++k) {  // every load in flight
+        const int32_t u = x + k % 3 - 1, v = y + k / 3 % 3 - 1, w = z + k / 9 - 1;
+        const bool in = (uint32_t)u < (uint32_t)g0 && (uint32_t)v < (uint32_t)g1 && (uint32_t)w < (uint32_t)g2;
+        const int32_t there = cells[in ? (w * g1 + v) * g0 + u : c];
+        sum += in ? there : 0;
+    }
+    return sum;
+}
+
+// Sum and sum of squares of each tile of cell counts.  COUNT: where the cells are
+// larger than they need to be, also the pairs of atoms in the same or
+// neighbouring cells, all tiles' together.
+template <bool COUNT>
 __global__ void __launch_bounds__(nd::kBlock)
 k_cell_tiles(const int32_t *__restrict__ cells, const Prep *__restrict__ prep, int32_t *__restrict__ tsum,
-             uint64_t *__restrict__ tsq) {
+             uint64_t *__restrict__ tsq, double few, unsigned long long *__restrict__ tests) {
     __shared__ int32_t s1[kWaves];
     __shared__ uint64_t s2[kWaves];
-    const int32_t ncell = prep->cg.ncell, base = blockIdx.x * kTileCells;
+    const int32_t ncell = table_cells(prep->grid), base = blockIdx.x * kTileCells;
     if (base >= ncell) return;
     int32_t a = 0;
     uint64_t b = 0;
@@ -770,6 +812,20 @@ k_cell_tiles(const int32_t *__restrict__ cells, const Prep *__restrict__ prep, i
         tsum[blockIdx.x] = a;
         tsq[blockIdx.x] = b;
     }
+    if constexpr (COUNT) {
+        // 27 sum c^2 bounds the pairs: tiles below `few` an atom are left out (the
+        // look around costs 20 us, a gas has nothing to gain from it)
+        __shared__ int32_t look;
+        if (threadIdx.x == 0) look = prep->stretched && 27.0 * (double)b > few * (double)a;
+        __syncthreads();
+        if (look == 0) return;
+        unsigned long long t = 0ull;
+        for (int32_t k = threadIdx.x; k < kTileCells && base + k < ncell; k += nd::kBlock)
+            if (const int32_t c = cells[base + k]; c > 0)
+                t += (unsigned long long)c * (unsigned long long)atoms_around(cells, prep->grid.cg, base + k);
+        for (int o = 32; o > 0; o >>= 1) t += __shfl_xor(t, o, 64);
+        if ((threadIdx.x & 63) == 0 && t > 0ull) atomicAdd(tests, t);
+    }
 }
 
 // First place of each cell (in place over the counts: cells[ncell] = n); the
@@ -779,7 +835,7 @@ k_cell_starts(int32_t *__restrict__ cells, int32_t n, const Prep *__restrict__ p
               const uint64_t *__restrict__ tsq, const uint32_t *__restrict__ kb, int32_t nkb,
               const int32_t *__restrict__ status, Prep *__restrict__ host) {
     __shared__ int32_t part[nd::kBlock];
-    const int32_t ncell = prep->cg.ncell, base = blockIdx.x * kTileCells, t = threadIdx.x;
+    const int32_t ncell = table_cells(prep->grid), base = blockIdx.x * kTileCells, t = threadIdx.x;
     if (base >= ncell) return;
     // atoms before this tile
     int32_t before = 0;
@@ -1005,19 +1061,21 @@ struct BinWork {
 
 size_t cell_bins_bytes() { return sizeof(BinWork); }
 
-const CellGrid *launch_cell_bins(hipStream_t st, void *work, const float4 *x, int32_t n, float r, int32_t max_cells,
-                                 int2 *cell_of, int32_t *cells, int32_t *status) {
+const BinGrid *launch_cell_bins(hipStream_t st, void *work, const float4 *x, int32_t n, float r, int32_t max_cells,
+                                BinMode mode, double few, int2 *cell_of, int32_t *cells, int32_t *status) {
     BinWork *w = static_cast<BinWork *>(work);
     if (max_cells > kMaxCells) max_cells = kMaxCells;
     const int32_t tiles = (max_cells + kTileCells - 1) / kTileCells;
     const unsigned g = grid_for(n), nb = std::min<unsigned>(g, kBoxBlocks);
     k_prep_boxes<true><<<nb, kBlock, 0, st>>>(Xyz4{x}, n, w->part, cells, max_cells + 1, &w->word, &w->word);
-    k_prep_grid<<<1, kBlock, 0, st>>>(w->part, (int32_t)nb, n, r, 0.0f, max_cells, nullptr, &w->prep);
+    if (mode == kBinLines) k_line_grid<<<1, 1, 0, st>>>(r, max_cells, &w->prep);
+    else k_prep_grid<<<1, kBlock, 0, st>>>(w->part, (int32_t)nb, n, r, 0.0f, max_cells, nullptr, &w->prep);
     k_bin_atoms<<<g, kBlock, 0, st>>>(x, n, &w->prep, cells, cell_of, status);
-    k_cell_tiles<<<tiles, kBlock, 0, st>>>(cells, &w->prep, w->tsum, w->tsq);
+    const auto count = mode == kBinCount ? k_cell_tiles<true> : k_cell_tiles<false>;
+    count<<<tiles, kBlock, 0, st>>>(cells, &w->prep, w->tsum, w->tsq, few, &w->prep.grid.tests);
     k_cell_starts<<<tiles, kBlock, 0, st>>>(cells, n, &w->prep, w->tsum, w->tsq, nullptr, 0, nullptr, nullptr);
     ND_HIP(hipGetLastError());
-    return &w->prep.cg;
+    return &w->prep.grid;
 }
 
 bool atoms_box(nd_ctx *ctx, const float *d_xyz, int32_t n, double lo[3], double hi[3]) {
@@ -1106,7 +1164,7 @@ int64_t tree_list(nd_ctx *ctx, const float *d_xyz, int32_t kind, int32_t n, int3
         k_prep_keys<true><<<g, kBlock, 0, st>>>(d_xyz, n, box, prep, codes, perm, cells, cell_of, kb, status);
     else
         k_prep_keys<false><<<g, kBlock, 0, st>>>(d_xyz, n, box, prep, codes, perm, cells, cell_of, kb, status);
-    k_cell_tiles<<<tiles, kBlock, 0, st>>>(cells, prep, tsum, tsq);
+    k_cell_tiles<false><<<tiles, kBlock, 0, st>>>(cells, prep, tsum, tsq, 0.0, nullptr);
     k_cell_starts<<<tiles, kBlock, 0, st>>>(cells, n, prep, tsum, tsq, kb, (int32_t)g, status, hp);
     ND_HIP(hipGetLastError());
     ND_HIP(hipStreamSynchronize(st));
@@ -1157,7 +1215,7 @@ int64_t tree_list(nd_ctx *ctx, const float *d_xyz, int32_t kind, int32_t n, int3
     S.kind = kind;
     S.n = n;
     S.apl = apl;
-    S.cg = p.cg;
+    S.cg = p.grid.cg;
     S.cpos = ctx->cell_pos.as<float4>();
     S.ckey = ctx->cell_keys.as<int32_t>();
     S.cstart = cells;
