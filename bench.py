@@ -214,7 +214,7 @@ def precision_form(pkg, steps=500):
 
 def batched_form(pkg, steps=200):
     """512 replicas of log-uniform size in [256, 16384] (density 0.8, LJ), packed
-    into one launch sequence per step, leaf size and walk autotuned; against one
+    into one launch sequence per step, list walk and tile shapes autotuned; against one
     simulation (one launch sequence) per replica."""
     B = pkg.batched
     sizes = B.replica_sizes(512, seed=11)

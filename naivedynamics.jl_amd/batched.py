@@ -3,15 +3,15 @@ sequence per step.
 
 The replicas are packed in space, each in its own wall box, with gaps wider
 than the neighbour-list radius between boxes.  The packed set is one
-simulation: one key sort, one LBVH, one list walk and one fused force +
-integrate kernel per step serve every replica, and a rebuild window is one
-captured hipGraph.  No listed pair joins two replicas (their atoms stay in
+simulation: one key sort, one list walk and one fused force + integrate
+kernel per step serve every replica, and a rebuild window is one captured
+hipGraph.  No listed pair joins two replicas (their atoms stay in
 their boxes and the boxes are further apart than the list radius), and each
 atom reflects off its own replica's box (nd_sim_set_replicas), so every
 replica follows the dynamics it would follow alone.  Uneven sizes cost
 nothing extra: the work is balanced per atom, not per replica.
 
-Padding atoms (fewer than one leaf) complete the last LBVH leaf; they sit
+Padding atoms (fewer than one leaf) complete the last leaf; they sit
 far apart on a line past the packed region, carry no charge and no velocity,
 and never interact.
 
@@ -149,19 +149,22 @@ class BatchedSimulation:
 
 
 def autotune(reps, spec, candidates=None, windows=3, ctx=None, log=None, tiles=True):
-    """Pick the packed run's traversal and force tile shapes by timing
+    """Pick the packed run's list walk and tile shapes by timing
     `windows` rebuild windows of each candidate after one warm-up window (every
-    window graph captured before timing).  Stage 1: LBVH leaf size (the
-    traversal and force tile: 8, 16 or 32 atoms) with the two-phase (0) or rope
-    (1) walk, and the cell list (3, no tree).  Stage 2 (`tiles`), from the
-    stage-1 winner, one dimension at a time: the two-phase walk's tree records
-    per round trip (`walk_front` 8 or 16) and the step kernel's neighbours per
-    pipeline batch (`pair_batch` 2, 4 or 8, FP32 only) and its lanes per atom
-    (`atom_lanes` 1 or 2).  Returns (best spec, [(leaf, walk, walk_front,
+    window graph captured before timing).  Stage 1: the two-phase walk (0), the
+    rope walk (1) with 8, 16 or 32 atoms per LBVH leaf, and the cell list (3, no
+    tree).  The two-phase walk has leaves of its own and no tree; only the mixed
+    form's walks the LBVH, with each leaf size.  Stage 2 (`tiles`), from the
+    stage-1 winner, one dimension at a time: the mixed form's two-phase walk's
+    tree records per round trip (`walk_front` 8 or 16) and the step kernel's
+    neighbours per pipeline batch (`pair_batch` 2, 4 or 8, FP32 only) and its
+    lanes per atom (`atom_lanes` 1 or 2).  Returns (best spec, [(leaf, walk, walk_front,
     pair_batch, atom_lanes, ms_per_step)]); 0 in the shape fields means the
     default (8 records, 4 neighbours, 1 lane)."""
+    over_tree = spec.precision in ("mixed", _lib.PREC_MIXED)  # the two-phase walk's form
     if candidates is None:
-        candidates = [(a, w) for a in (8, 16, 32) for w in (0, 1)] + [(16, 3)]
+        # without a tree the leaf size only pads the packed atoms: the least
+        candidates = [(a, 0) for a in ((8, 16, 32) if over_tree else (8,))] + [(a, 1) for a in (8, 16, 32)] + [(16, 3)]
     table = []
 
     def measure(s2):
@@ -189,7 +192,7 @@ def autotune(reps, spec, candidates=None, windows=3, ctx=None, log=None, tiles=T
             best, best_ms = s2, ms
     if tiles:
         dims = []
-        if best.list_walk == 0:
+        if best.list_walk == 0 and over_tree:
             dims.append(("walk_front", (8, 16)))
         if best.precision == "fp32":
             dims.append(("pair_batch", (2, 4, 8)))
