@@ -50,7 +50,7 @@ __device__ __forceinline__ bool to_units(double f, int32_t *status, unsigned lon
 // lands at ~19 per ns whatever its locality), and a pair list names the same
 // atoms again and again: a list in the order of a search repeats each i over
 // its neighbours and each j over the queries near it, so 18,800 consecutive
-// pairs (1/256 of the list of 131,072 liquid atoms) name about 2,000 atoms.
+// pairs (1/256 of the list of 131,072 liquid atoms) name about 1,100 atoms.
 // Six atomics per pair in memory took 1,098 us there, this takes 84.  An atom
 // that finds no slot in kProbes places is added in memory, so a list in any
 // order gives the same sums.
@@ -185,7 +185,12 @@ void run_pair_force(nd_ctx *ctx, float *d_force, const nd_pair *d_pairs, int64_t
     const int64_t n3 = 3 * (int64_t)n;
     // one workgroup per CU (its table takes most of the CU's LDS), each with
     // one run of the list: the longer the run, the fewer sums leave LDS; a
-    // short list keeps a pair per thread
+    // short list keeps a pair per thread.  A call over the list of 131,072 /
+    // 262,144 / 524,288 / 1,048,576 liquid atoms takes 100 / 166 / 416 / 2,964 us
+    // (atomics on memory 1,151 / 2,088 / 4,517 / 9,034): up to 524,288 a run's
+    // atoms (some 3,600) mostly fit the table, at 1,048,576 (6,000) those left over pay
+    // for their probes and go to memory.  The pairs of 131,072 atoms in random
+    // order, which do so almost always, take 873 (932).
     const int64_t per = std::max<int64_t>((npairs + 255) / 256, kForceThreads);
     const int64_t nblk = (npairs + per - 1) / per;
     ctx->force_acc.reserve(sizeof(unsigned long long) * (size_t)(n3 > 0 ? n3 : 1));

@@ -9,8 +9,8 @@
 // a leaf of four atoms that straddles an octree jump overlaps thousands of
 // leaves (1.7-1.9 ms per pass for 262,144 points at liquid density).
 //
-// One wave takes 16 to 64 consecutive cell-sorted atoms, in groups that lie in
-// up to k cells of one row along x (k so that k cells hold about a dozen
+// One wave takes 16 or 32 consecutive cell-sorted atoms, in groups that lie in
+// up to k cells of one row along x (k so that k cells hold about two dozen
 // atoms).  A group's candidates are the rows of cells around it, each row one
 // contiguous run of the cell-sorted atoms; they are loaded once into registers
 // (kBatches x 64 lanes), then tested against the group's atoms one after
@@ -963,7 +963,10 @@ PairArgs pair_args(const PairSearch &S) {
     A.cg = S.cg;
     const double mean = (double)S.n / S.cg.ncell;
     // longer runs share more of a group's set-up, shorter ones leave enough
-    // waves (8,000 atoms at radius 2.8: cell list 153 us with 16, 186 with 32)
+    // waves.  Lists at radius 2.8 with 16 and 32: 32,768 atoms 279 and 325 us,
+    // 131,072 408 and 415, 196,608 519 and 548, 262,144 620 and 627 (point
+    // queries 510 and 513, cell lists 237 to 255 and 249), 524,288 1,007 and 997,
+    // 1,048,576 1,865 and 1,824
     A.per_wave = S.n >= 262144 ? 32 : 16;
     // where squared distances underflow, atoms more than a cell apart could
     // pass the test: groups of one cell look at its 27 neighbours only

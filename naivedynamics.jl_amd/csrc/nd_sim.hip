@@ -1115,8 +1115,10 @@ constexpr int kSplit = 4;
 constexpr int kLeafChunk = 64;    // leaves per chunk, chunks per super
 constexpr int kFlatChunks = 512;  // more chunks than this have supers
 // Up to this many chunks no box of theirs is made or tested: most are near any
-// wave, and a launch a list is saved (4,096 atoms with a list every step: 65.7 -> 62.4
-// us a step).
+// wave, and a launch a list is saved (500 / 2,000 / 4,096 atoms with a list every
+// step: 49.8 / 70.0 / 63.0 us a step with the boxes, 46.1 / 66.2 / 59.7 without).
+// The gain does not end there: with 5 to 16 chunks it is the same 3 to 4 us
+// (6,144 / 12,288 / 16,384 atoms 78.0 / 95.6 / 101.3 and 74.2 / 91.5 / 99.5).
 constexpr int kPlainChunks = 4;
 
 // What phase 1 reads: the leaves' boxes (padded by h on each side) and the boxes
@@ -1137,6 +1139,7 @@ __host__ __device__ __forceinline__ int32_t rec_stride(int32_t cap) { return (ca
 // (recs[i * rec_stride(cap) + k], k < nrecs[i]; blocks of 64 B multiples, so a
 // reader fetches two records per 16-byte load); each holds at least one
 // neighbour, so there are never more records than list entries.
+
 // The largest list length of a wave's lanes into ctr[0] (ctr[1]: over cap).
 __device__ __forceinline__ void count_max(int32_t count, int32_t cap, int32_t *__restrict__ ctr) {
     int32_t m = count;
@@ -2069,7 +2072,9 @@ k_walk_table_split(const float4 *__restrict__ pos, WalkBoxes B, int32_t n, int32
     if (U < 0) {
         // too many records or no table (uniform): the first four waves join the
         // slices' records, a slice after the other, and build as one wave per 64
-        // atoms does (a barrier waits for the waves that have not ended)
+        // atoms does.  The others end here: the barriers of the build wait for the
+        // waves that have not ended, which is how this hardware's barrier counts (it
+        // is no promise of the language).
         __syncthreads();
         if (slice != 0) return;
         if (i < n) {
