@@ -3159,7 +3159,10 @@ void set_step_params(nd_sim *s) {
     // FP32 (an inexact unit would scale every difference by the same
     // relative error and bias the pressure coherently).
     const double span = p.hi > p.lo ? p.hi - p.lo : 1.0;
-    const double half = p.walls ? 0.5 * span * 1.001 + 1e-6 : 2.0 * span;
+    // Differences of listed atoms have to fit an int32 as well: the list radius
+    // and a skin of motion, in boxes less than twice that wide.
+    const double reach = rcmax + 2.0 * p.skin;
+    const double half = std::max(p.walls ? 0.5 * span * 1.001 + 1e-6 : 2.0 * span, reach);
     q.fx_c = 0.5 * (p.lo + p.hi);
     q.fx_s = std::ldexp(1.0, (int)std::floor(std::log2(0.999 * 2147483648.0 / half)));
     q.fx_inv = (float)(1.0 / q.fx_s);
